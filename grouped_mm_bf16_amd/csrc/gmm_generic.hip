@@ -217,6 +217,7 @@ int launch(const GmmParams& p, hipStream_t stream) {
 }  // namespace
 
 int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream) {
+  if (gmm_staged_eligible(p)) return gmm_launch_staged(p, in_dtype, out_dtype, num_cus, stream);
   p.align = 1;
   p.xcd_remap = 0;
   // at least one full 128 x 128 tile and a contraction worth pipelining: the matrix-core kernel

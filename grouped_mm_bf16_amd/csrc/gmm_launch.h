@@ -7,6 +7,11 @@
 // Each returns 0 on success, 1 if the launch failed, -1 if the dtype pair is unsupported.
 int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream);
 
+// Register-staged MFMA kernel for operands of any alignment (gmm_staged.hip): each operand contiguous along one of
+// its dimensions.  Returns like gmm_launch_generic.
+bool gmm_staged_eligible(const GmmParams& p);
+int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream);
+
 // Operand layout facts the host derived from strides.
 struct GmmLayout {
   bool a_kc;  // A contiguous along K (row-major); otherwise contiguous along M

@@ -1,0 +1,450 @@
+// Register-staged MFMA grouped GEMM for operands of any alignment: bf16, fp16 and fp32, each operand contiguous
+// along K or along M / N, any leading dimension, any base address, with or without a row gather.
+//
+// What it replaces and why.  Operands that the assembly tile cannot take (an extent or a leading dimension that is
+// not a multiple of 8 elements, fp32) went element by element: one 2- or 4-byte load, one bounds check and one 64-bit
+// address per element, fp32 products whatever the type.  gfx950 loads 16 bytes from any address that is a multiple of
+// the element size (measured: 29 us against 27 us aligned), so nothing has to go element by element but an operand's
+// last chunk.  Before and after, us: bf16 8191 x 2047 x 2047 in 8 groups 2291 -> 153 (450 TFLOP/s), 6151 x 1031 x 519
+// in 24 groups 472 -> 36, its weight gradient 437 -> 45; fp32 8192 x 1024 x 4096 920 -> 592 (116 TFLOP/s of 157),
+// 1024 x 1024 x 8192 columns in 8 groups 330 -> 166.
+//
+//   * A K tile is 128 bytes of K per row (64 bf16 / fp16, 32 fp32): every thread carries its 16-byte chunks of the
+//     next K tile in registers while the MFMAs of the present one run out of LDS (two buffers, one barrier per K
+//     tile); two or four workgroups share a CU, so one computes while another stores, fetches or starts up.  fp32
+//     fetches two K tiles ahead (5 % on large problems); for 16-bit operands a second one in flight gained nothing:
+//     small problems are bound by start-up, which more code makes longer, large ones by the LDS.
+//   * Operand contiguous along K: LDS [row][128 bytes], 16-byte chunk index XOR (row >> 1) & 7, a fragment (16 rows,
+//     8 or 4 consecutive k per lane) is one ds_read_b128.  Operand contiguous along M / N: LDS [k][rows] as it comes
+//     from memory; 16-bit fragments are two transposing ds_read_b64_tr_b16 (k rows 4 .. 7 and 8 .. 11 of 16 swap
+//     places so that the 32 lanes served together hit all 64 banks once), fp32 fragments are four ds_read_b32.
+//   * v_mfma_f32_16x16x32_{bf16,f16} / v_mfma_f32_16x16x4_f32, fp32 accumulators, one rounding.  Operands swapped, so
+//     that a lane owns 4 consecutive columns; a wave stages 16 rows at a time in LDS and stores 16 bytes per lane in
+//     whole rows.
+//   * Loads never leave the operand: rows and columns past the extent are clamped (their products are not stored); K
+//     tiles that are cut by the end of the group's range, or whose chunks touch the operand's last bytes, are fetched
+//     with a check per chunk, without branches, in a loop of their own.
+//   * What bounds it: 16-bit, 4 x 4 blocks per wave: LDS reads and writes take 1.5 times the cycles of the MFMAs; fp32:
+//     the MFMA pipe (64 to 75 % busy), the rest is the last, partly filled round.
+#include "gmm_device.h"
+#include "gmm_launch.h"
+
+namespace {
+
+constexpr int NT = 256;            // threads: 2 x 2 waves
+constexpr int ROW_BYTES = 128;     // bytes of K per row and K tile
+
+// Workgroups per CU: what the LDS images (64 to 72 KB, 33 to 35 KB) and the registers allow.
+constexpr int tile_wgs(int edge) { return edge == 128 ? 2 : 4; }
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
+
+// 16 bytes from an address that is a multiple of the element size only (one global_load_dwordx4).
+template <typename T>
+__device__ __forceinline__ uint4 load16(const T* p) {
+  uint4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+// Elements [0, n) of the chunk at p, zeros behind them, without a branch and without reading at or past `end`: a chunk
+// that would cross it is fetched from `last` (the operand's last 16 bytes) and shifted down.  p may lie anywhere if
+// n <= 0.
+template <typename T>
+__device__ __forceinline__ uint4 load_part(const T* p, const T* last, int n) {
+  constexpr int EPC = 16 / int(sizeof(T));
+  const bool cross = p > last || n <= 0;
+  uint4 v = load16(cross ? last : p);
+  const int shift = cross ? int(p - last) : 0;           // elements; only looked at when n > 0
+  if (__ballot(n > 0 && shift > 0)) {
+    // rare (the operand's very last chunk): a loop over single elements
+#pragma unroll 1
+    for (int s = EPC - 1; s > 0; --s) {
+      const bool go = s <= shift;
+      uint4 w;
+      if constexpr (sizeof(T) == 2)
+        w = make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                       __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16);
+      else
+        w = make_uint4(v.y, v.z, v.w, 0u);
+      v.x = go ? w.x : v.x; v.y = go ? w.y : v.y; v.z = go ? w.z : v.z; v.w = go ? w.w : v.w;
+    }
+  }
+  uint32_t* w = &v.x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (sizeof(T) == 2)
+      w[i] = n > 2 * i + 1 ? w[i] : n > 2 * i ? (w[i] & 0xffffu) : 0u;
+    else
+      w[i] = n > i ? w[i] : 0u;
+  }
+  return v;
+}
+
+// LDS image of one operand's K tile of ROWS rows (or columns).
+template <typename T, bool TR, int ROWS>
+struct Image {
+  static constexpr int ESZ = int(sizeof(T));
+  static constexpr int BK = ROW_BYTES / ESZ;
+  static constexpr int PITCH = TR ? ROWS * ESZ + (ESZ == 2 ? 32 : 16) : ROW_BYTES;   // bytes between LDS rows
+  static constexpr int BYTES = TR ? BK * PITCH : ROWS * ROW_BYTES;
+  // transposed 16-bit image: k rows 4..7 and 8..11 of every 16 trade places
+  static __device__ __forceinline__ int slot(int k) { return ESZ == 2 ? (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1) : k; }
+};
+
+// Global -> registers -> LDS of one operand: NCH 16-byte chunks per thread and K tile.
+template <typename T, bool TR, int ROWS>
+struct Stage {
+  using Im = Image<T, TR, ROWS>;
+  static constexpr int EPC = 16 / Im::ESZ;             // elements of a chunk
+  static constexpr int CPR = TR ? ROWS / EPC : 8;      // chunks per LDS row
+  static constexpr int NCH = ROWS * 8 / NT;
+  const T* ptr[NCH];                                   // the thread's chunks of K tile 0
+  const T* last;                                       // the operand's last 16 bytes
+  int64_t step;                                        // elements from one K tile to the next
+  int zero_rows;                                       // bit i: chunk i belongs to a gathered row that does not exist
+  int any_zero;                                        // some lane of the wave has one
+  int n_fast;                                          // K tiles that need no check
+
+  // base: element (row 0, k 0) of the group's operand; the tile's rows start at row0; `ext` rows exist.
+  __device__ __forceinline__ void init(const T* base, int64_t ld, int row0, int ext, int k_lo, int k_hi, int k_ext,
+                                       const GmmParams* gather, int gather_end) {
+    const int tid = threadIdx.x;
+    zero_rows = 0;
+    const int whole = (k_hi - k_lo) / Im::BK;          // K tiles that lie inside the range
+    if constexpr (!TR) {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) {
+        const int q = i * NT + tid, row = q >> 3, c = q & 7;
+        int src = gmm_min(row0 + row, ext - 1);
+        if (gather) {
+          src = row0 + row < gather_end ? gmm_gather_row(*gather, row0 + row) : -1;
+          if (src < 0) { zero_rows |= 1 << i; src = 0; }
+        }
+        ptr[i] = base + int64_t(src) * ld + k_lo + c * EPC;
+      }
+      any_zero = gather ? __ballot(zero_rows != 0) != 0 : 0;
+      last = base + int64_t((gather ? gather->a_rows : ext) - 1) * ld + k_ext - EPC;
+      step = Im::BK;
+      n_fast = whole;
+    } else {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) {
+        const int q = i * NT + tid, k = q / CPR, c = q % CPR;
+        const int col = row0 + c * EPC;
+        ptr[i] = base + int64_t(k_lo + k) * ld + (col < ext ? col : row0);
+      }
+      last = base + int64_t(k_ext - 1) * ld + ext - EPC;
+      step = int64_t(Im::BK) * ld;
+      // the last chunk of a row may reach past the extent, into the next k row: fine as long as there is one
+      const int over = row0 + gmm_min(ROWS, (ext - row0 + EPC - 1) / EPC * EPC) - ext;
+      const int slack = over > 0 ? int((over + ld - 1) / ld) : 0;
+      const int safe = gmm_min(k_hi, k_ext - slack) - k_lo;
+      n_fast = safe > 0 ? safe / Im::BK : 0;
+    }
+  }
+
+  __device__ __forceinline__ void load_fast(uint4 (&r)[NCH], int t) const {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) r[i] = load16(ptr[i] + int64_t(t) * step);
+  }
+
+  // the same for a K tile that needs checks; k_left = k elements of the range from K tile t on
+  __device__ __forceinline__ void load_checked(uint4 (&r)[NCH], int t, int k_left) const {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int q = i * NT + tid;
+      const int n = TR ? (q / CPR < k_left ? EPC : 0) : k_left - (q & 7) * EPC;
+      r[i] = load_part<T>(ptr[i] + int64_t(t) * step, last, n);
+    }
+  }
+
+  __device__ __forceinline__ void store(uint4 (&r)[NCH], char* image) const {
+    const int tid = threadIdx.x;
+    if (!TR && __builtin_amdgcn_readfirstlane(any_zero)) {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) r[i] = (zero_rows & (1 << i)) ? make_uint4(0, 0, 0, 0) : r[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int q = i * NT + tid;
+      int at;
+      if constexpr (!TR) {
+        const int row = q >> 3, c = q & 7;
+        at = row * ROW_BYTES + ((c ^ ((row >> 1) & 7)) << 4);
+      } else {
+        at = Im::slot(q / CPR) * Im::PITCH + (q % CPR) * 16;
+      }
+      *reinterpret_cast<uint4*>(image + at) = r[i];
+    }
+  }
+};
+
+// Fragment of 16 rows starting at `row0` and k half `half` of a K tile: lane l holds row l % 16, the k elements of
+// 16-byte chunk 4 * half + l / 16.
+template <typename T, bool TR, int ROWS>
+__device__ __forceinline__ uint4 read_fragment(const char* image, int row0, int half, int lane) {
+  using Im = Image<T, TR, ROWS>;
+  const int q = lane >> 4, ii = lane & 15;
+  if constexpr (!TR) {
+    const int row = row0 + ii;
+    return *reinterpret_cast<const uint4*>(image + row * ROW_BYTES + (((4 * half + q) ^ ((row >> 1) & 7)) << 4));
+  } else if constexpr (Im::ESZ == 2) {
+    // k = 32 half + 8 q + 0..3 and + 4..7; each group of 16 lanes reads 4 k rows x 16 columns, transposed
+    const int s0 = 32 * half + 16 * (q >> 1) + 4 * (q & 1) + (ii >> 2);
+    const char* p = image + s0 * Im::PITCH + (row0 + 4 * (ii & 3)) * 2;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p + 8 * Im::PITCH));
+    uint4 v;
+    __builtin_memcpy(&v.x, &lo, 8);
+    __builtin_memcpy(&v.z, &hi, 8);
+    return v;
+  } else {
+    const char* p = image + (16 * half + 4 * q) * Im::PITCH + (row0 + ii) * 4;
+    uint4 v;
+    v.x = *reinterpret_cast<const uint32_t*>(p);
+    v.y = *reinterpret_cast<const uint32_t*>(p + Im::PITCH);
+    v.z = *reinterpret_cast<const uint32_t*>(p + 2 * Im::PITCH);
+    v.w = *reinterpret_cast<const uint32_t*>(p + 3 * Im::PITCH);
+    return v;
+  }
+}
+
+// acc += first operand's fragments x second operand's; operands swapped, so that a lane owns 4 consecutive columns.
+template <typename T, int TM, int TN>
+__device__ __forceinline__ void multiply(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x4 (&acc)[TM][TN]) {
+  if constexpr (sizeof(T) == 4) {
+    // element e of every lane's chunk is one k of four: no two MFMAs in a row add to the same accumulator
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const uint32_t x = e == 0 ? a[i].x : e == 1 ? a[i].y : e == 2 ? a[i].z : a[i].w;
+          const uint32_t y = e == 0 ? b[j].x : e == 1 ? b[j].y : e == 2 ? b[j].z : b[j].w;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(y), __uint_as_float(x), acc[i][j], 0, 0, 0);
+        }
+  } else {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if constexpr (__is_same(T, gmm_f16)) {
+          f16x8 x, y;
+          __builtin_memcpy(&x, &a[i], 16);
+          __builtin_memcpy(&y, &b[j], 16);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(y, x, acc[i][j], 0, 0, 0);
+        } else {
+          bf16x8 x, y;
+          __builtin_memcpy(&x, &a[i], 16);
+          __builtin_memcpy(&y, &b[j], 16);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y, x, acc[i][j], 0, 0, 0);
+        }
+      }
+  }
+}
+
+template <typename T, typename OutT, bool A_TR, bool B_TR, int EDGE>
+__global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const GmmParams p) {
+  constexpr int BM = EDGE, BN = EDGE;
+  constexpr int AHEAD = sizeof(T) == 4 ? 2 : 1;   // K tiles fetched ahead (see the top of the file)
+  using ImA = Image<T, A_TR, BM>;
+  using ImB = Image<T, B_TR, BN>;
+  constexpr int BK = ImA::BK;
+  constexpr int WTM = BM / 2, WTN = BN / 2, TM = WTM / 16, TN = WTN / 16;
+  // epilogue: a wave stages 16 rows of its columns, padded by 16 bytes against bank conflicts
+  constexpr int OSZ = int(sizeof(OutT)), OEC = 16 / OSZ;
+  constexpr int EPITCH = WTN * OSZ + 16, ECPR = WTN * OSZ / 16;
+  constexpr int PIPE = 2 * (ImA::BYTES + ImB::BYTES), EPI = 4 * 16 * EPITCH;
+  __shared__ __attribute__((aligned(16))) char lds[PIPE > EPI ? PIPE : EPI];
+  __shared__ int32_t cum[GMM_MAX_GROUPS + 1];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave & 1) * WTM, wn = (wave >> 1) * WTN;
+  const int total = gmm_build_tile_table<NT>(p, BM, BN, cum);
+  const int64_t lda = A_TR ? p.a_sk : p.a_sm, ldb = B_TR ? p.b_sk : p.b_sn;
+
+  for (int t = blockIdx.x; t < total; t += gridDim.x) {
+    const GmmTile tile = gmm_locate_tile(p, cum, gmm_xcd_remap(t, total, gridDim.x), BM, BN);
+    const T* a = static_cast<const T*>(p.a) + int64_t(tile.g) * p.a_sg;
+    const T* b = static_cast<const T*>(p.b) + int64_t(tile.g) * p.b_sg;
+    OutT* c = static_cast<OutT*>(p.c) + int64_t(tile.g) * p.c_sg;
+
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const int klen = tile.k_hi - tile.k_lo;
+    if (klen > 0) {
+      Stage<T, A_TR, BM> sa;
+      Stage<T, B_TR, BN> sb;
+      sa.init(a, lda, tile.m0, p.M, tile.k_lo, tile.k_hi, p.K, p.gather ? &p : nullptr, tile.m_hi);
+      sb.init(b, ldb, tile.n0, p.N, tile.k_lo, tile.k_hi, p.K, nullptr, 0);
+      const int n_fast = gmm_min(sa.n_fast, sb.n_fast), nk = (klen + BK - 1) / BK;
+      // K tile t + 1 .. t + AHEAD are on their way in registers while K tile t is multiplied
+      uint4 ra[AHEAD][sa.NCH], rb[AHEAD][sb.NCH];
+      auto load = [&](int t, int set) {
+        sa.load_checked(ra[set], t, klen - t * BK);
+        sb.load_checked(rb[set], t, klen - t * BK);
+      };
+      auto store = [&](int t, int set) {
+        sa.store(ra[set], lds + (t & 1) * ImA::BYTES);
+        sb.store(rb[set], lds + 2 * ImA::BYTES + (t & 1) * ImB::BYTES);
+      };
+#pragma unroll
+      for (int d = 0; d < AHEAD; ++d)
+        if (d < nk) load(d, d);
+      store(0, 0);
+      __syncthreads();
+      auto compute = [&](int t) {
+        const char* la = lds + (t & 1) * ImA::BYTES;
+        const char* lb = lds + 2 * ImA::BYTES + (t & 1) * ImB::BYTES;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          uint4 fa[TM], fb[TN];
+#pragma unroll
+          for (int i = 0; i < TM; ++i) fa[i] = read_fragment<T, A_TR, BM>(la, wm + 16 * i, half, lane);
+#pragma unroll
+          for (int j = 0; j < TN; ++j) fb[j] = read_fragment<T, B_TR, BN>(lb, wn + 16 * j, half, lane);
+          multiply<T, TM, TN>(fa, fb, acc);
+        }
+      };
+      // interior: the K tiles fetched here need no check.  A loop of its own: with the checked fetch in the same loop
+      // the compiler waits for every load in flight where the two meet.
+      int k0 = 0;
+      for (; k0 + 2 * AHEAD <= n_fast; k0 += AHEAD) {
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d) {
+          sa.load_fast(ra[d], k0 + d + AHEAD);
+          sb.load_fast(rb[d], k0 + d + AHEAD);
+          compute(k0 + d);
+          store(k0 + d + 1, (d + 1) % AHEAD);
+          __syncthreads();
+        }
+      }
+      for (; k0 < nk; k0 += AHEAD) {
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d) {
+          const int kt = k0 + d;
+          if (kt >= nk) break;
+          if (kt + AHEAD < nk) load(kt + AHEAD, d);
+          compute(kt);
+          if (kt + 1 < nk) store(kt + 1, (d + 1) % AHEAD);
+          __syncthreads();
+        }
+      }
+    }
+
+    // Block (i, j), register r: row 16 i + lane % 16, column 16 j + 4 (lane / 16) + r of the wave's part.
+    char* const stage = lds + wave * (16 * EPITCH);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        OutT o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = gmm_from_float<OutT>(acc[i][j][r]);
+        __builtin_memcpy(stage + (lane & 15) * EPITCH + (16 * j + 4 * (lane >> 4)) * OSZ, o, 4 * OSZ);
+      }
+      asm volatile("" ::: "memory");   // the wave's LDS accesses complete in order; the compiler must keep it
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int x = lane; x < 16 * ECPR; x += 64) {
+        const int row = tile.m0 + wm + 16 * i + x / ECPR, col = tile.n0 + wn + (x % ECPR) * OEC;
+        if (row < tile.m_lo || row >= tile.m_hi) continue;
+        const char* src = stage + (x / ECPR) * EPITCH + (x % ECPR) * 16;
+        OutT* dst = c + int64_t(row) * p.c_sm + int64_t(col) * p.c_sn;
+        if (p.c_sn == 1 && col >= tile.n_lo && col + OEC <= tile.n_hi) {
+          __builtin_memcpy(dst, src, 16);
+        } else {
+#pragma unroll 1
+          for (int e = 0; e < OEC; ++e)
+            if (col + e >= tile.n_lo && col + e < tile.n_hi) __builtin_memcpy(dst + e * p.c_sn, src + e * OSZ, OSZ);
+        }
+      }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();   // the next tile's images overwrite the staging area
+  }
+}
+
+template <typename T, typename OutT, int EDGE>
+int launch_layout(GmmParams p, bool a_tr, bool b_tr, int num_cus, hipStream_t stream) {
+  const int64_t bound = (gmm_tile_bound(p.jag, p.G, p.M, p.N, EDGE, EDGE) + 7) / 8 * 8, most = int64_t(tile_wgs(EDGE)) * num_cus;
+  p.num_wg = int(bound < most ? (bound < 8 ? 8 : bound) : most);
+  const dim3 grid(p.num_wg), block(NT);
+  if (a_tr && b_tr)
+    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, true, true, EDGE>), grid, block, 0, stream, p);
+  else if (a_tr)
+    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, true, false, EDGE>), grid, block, 0, stream, p);
+  else if (b_tr)
+    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, false, true, EDGE>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, false, false, EDGE>), grid, block, 0, stream, p);
+  return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+// Tiles of a launch with square tiles of `edge`, the group boundaries taken to cut half a tile each on average.
+int64_t expected_tiles(const GmmParams& p, int edge) {
+  const int64_t tm = (p.M + edge - 1) / edge, tn = (p.N + edge - 1) / edge;
+  if (p.jag == GMM_JAG_M) return (p.M / edge + (p.G + 1) / 2) * tn;
+  if (p.jag == GMM_JAG_N) return tm * (p.N / edge + (p.G + 1) / 2);
+  return p.G * tm * tn;
+}
+
+// fp32: 64 x 64 tiles (four workgroups per CU) or 128 x 128 (two)?  A launch takes whole rounds of its grid, and a
+// round of large tiles takes 1.84 times a round of small ones (2048 x 2048 x 2048, four products: 2 rounds of 258 us
+// against 4 of 140 us), so the cheaper count wins.  Measured, us, small / large: 1024 rows, K 1024, 8192 columns in
+// 8 groups 166 / 216; 4096 x 2048 x 2048 in 8 groups 316 / 394; 1024 x 1024 x 1024 in 8 groups 45 / 77; 8192 x 1024
+// x 4096 in 8 groups 599 / 592; four products of 2048^3 562 / 517.
+// 16-bit operands always take 128 x 128: twice the MFMA rate makes the small tile's LDS reads the bound (8191 x 2047
+// x 2047 in 8 groups: 218 us against 153; 24 groups of 6151 x 1031 x 519: 32 against 36).
+bool small_tiles(const GmmParams& p, int in_dtype, int num_cus) {
+  if (in_dtype != GMM_DT_F32) return false;
+  const int64_t small_round = int64_t(tile_wgs(64)) * num_cus, large_round = int64_t(tile_wgs(128)) * num_cus;
+  const int64_t small = (expected_tiles(p, 64) + small_round - 1) / small_round;
+  const int64_t large = (expected_tiles(p, 128) + large_round - 1) / large_round;
+  return 100 * small < 184 * large;
+}
+
+}  // namespace
+
+bool gmm_staged_eligible(const GmmParams& p) {
+  // each operand contiguous along one of its dimensions; gathered rows only along K; element offsets are 64-bit, so
+  // no extent is too large
+  const bool a_kc = p.a_sk == 1, b_kc = p.b_sk == 1;
+  if (!a_kc && (p.a_sm != 1 || p.gather)) return false;
+  if (!b_kc && p.b_sn != 1) return false;
+  const int64_t lda = a_kc ? p.a_sm : p.a_sk, ldb = b_kc ? p.b_sn : p.b_sk;
+  // a chunk of 16 bytes has to fit into every operand
+  const int64_t rows = p.gather ? p.a_rows : p.M;
+  const int64_t a_len = a_kc ? (rows - 1) * lda + p.K : (p.K - 1) * lda + p.M;
+  const int64_t b_len = b_kc ? (p.N - 1) * ldb + p.K : (p.K - 1) * ldb + p.N;
+  return lda >= 1 && ldb >= 1 && p.K >= 1 && rows >= 1 && a_len >= 8 && b_len >= 8;
+}
+
+int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream) {
+  p.align = 1;
+  const bool a_tr = p.a_sk != 1, b_tr = p.b_sk != 1;
+  if (in_dtype == GMM_DT_F32 && out_dtype == GMM_DT_F32)
+    return small_tiles(p, in_dtype, num_cus) ? launch_layout<float, float, 64>(p, a_tr, b_tr, num_cus, stream)
+                                             : launch_layout<float, float, 128>(p, a_tr, b_tr, num_cus, stream);
+#define GMM_STAGED_CASE(IN_CODE, OUT_CODE, IN_T, OUT_T) \
+  if (in_dtype == IN_CODE && out_dtype == OUT_CODE) return launch_layout<IN_T, OUT_T, 128>(p, a_tr, b_tr, num_cus, stream);
+  GMM_STAGED_CASE(GMM_DT_BF16, GMM_DT_BF16, gmm_bf16, gmm_bf16)
+  GMM_STAGED_CASE(GMM_DT_BF16, GMM_DT_F32, gmm_bf16, float)
+  GMM_STAGED_CASE(GMM_DT_F16, GMM_DT_F16, gmm_f16, gmm_f16)
+  GMM_STAGED_CASE(GMM_DT_F16, GMM_DT_F32, gmm_f16, float)
+#undef GMM_STAGED_CASE
+  return -1;
+}
