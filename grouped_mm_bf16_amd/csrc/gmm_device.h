@@ -46,29 +46,81 @@ __device__ __forceinline__ int gmm_build_tile_table(const GmmParams& p, int bm, 
   return cum[p.G];
 }
 
-// Linear tile id -> tile, using the table above.
-__device__ __forceinline__ GmmTile gmm_locate_tile(const GmmParams& p, const int32_t* cum, int t, int bm, int bn) {
-  int g, local, lo = 0, hi = 0, tm, tn;
+// Linear tile id -> group, index inside the group and the group's range, using the table above; uniform.
+__device__ __forceinline__ void gmm_find_tile(const GmmParams& p, const int32_t* cum, int t, int bm, int bn, int& g,
+                                              int& local, int& lo, int& hi) {
+  lo = hi = 0;
   if (p.jag == GMM_JAG_NONE) {
-    tm = gmm_cdiv(p.M, bm);
-    tn = gmm_cdiv(p.N, bn);
-    g = t / (tm * tn);
-    local = t - g * (tm * tn);
+    const int per = gmm_cdiv(p.M, bm) * gmm_cdiv(p.N, bn);
+    g = t / per;
+    local = t - g * per;
   } else {
-    const int extent = p.jag == GMM_JAG_M ? p.M : (p.jag == GMM_JAG_N ? p.N : p.K);
     g = gmm_find_group(cum, p.G, t);
     local = t - cum[g];
-    gmm_group_range(p.offs, g, extent, lo, hi);
-    g = __builtin_amdgcn_readfirstlane(g);
-    local = __builtin_amdgcn_readfirstlane(local);
-    lo = __builtin_amdgcn_readfirstlane(lo);
-    hi = __builtin_amdgcn_readfirstlane(hi);
-    gmm_group_grid(p.jag, lo, hi, p.M, p.N, bm, bn, p.align, tm, tn);
+    gmm_group_range(p.offs, g, p.jag == GMM_JAG_M ? p.M : (p.jag == GMM_JAG_N ? p.N : p.K), lo, hi);
   }
-  int mt, nt;
+  g = __builtin_amdgcn_readfirstlane(g);
+  local = __builtin_amdgcn_readfirstlane(local);
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  hi = __builtin_amdgcn_readfirstlane(hi);
+}
+
+// Tile `local` of group g.
+__device__ __forceinline__ GmmTile gmm_tile_of_group(const GmmParams& p, int g, int local, int lo, int hi, int bm, int bn) {
+  int tm, tn, mt, nt;
+  gmm_group_grid(p.jag, lo, hi, p.M, p.N, bm, bn, p.align, tm, tn);
   gmm_decode_in_group(local, tm, tn, mt, nt);
   return gmm_make_tile(p, g, lo, hi, mt, nt, bm, bn);
 }
+
+// Linear tile id -> tile, using the table above.
+__device__ __forceinline__ GmmTile gmm_locate_tile(const GmmParams& p, const int32_t* cum, int t, int bm, int bn) {
+  int g, local, lo, hi;
+  gmm_find_tile(p, cum, t, bm, bn, g, local, lo, hi);
+  return gmm_tile_of_group(p, g, local, lo, hi, bm, bn);
+}
+
+// ---- the same table for up to 64 groups in registers ------------------------------------------------ //
+// Lane g of every wave holds group g; a tile's group is the number of groups that end at or before it.  No LDS, no
+// barrier, no search: 1 us from the kernel's start to the first tile where the table in LDS takes 3.3 us (it is a
+// chain of loads, barriers and dependent LDS reads, and every workgroup of a small launch waits for it).
+__device__ __forceinline__ int gmm_wave_inclusive_scan(int v) {
+  // prefix sums inside each row of 16 lanes, then lane 15 of a row into the next row, lane 31 into rows 2 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
+struct GmmWaveGroups {
+  int lo, hi, count, incl;   // of the lane's group: its range, its tiles, tiles up to and including it
+
+  // Returns the total number of tiles.
+  __device__ __forceinline__ int build(const GmmParams& p, int bm, int bn) {
+    const int lane = threadIdx.x & 63;
+    const int extent = p.jag == GMM_JAG_M ? p.M : (p.jag == GMM_JAG_N ? p.N : p.K);
+    lo = hi = count = 0;
+    if (lane < p.G) {
+      int tm, tn;
+      gmm_group_range(p.offs, lane, extent, lo, hi);
+      gmm_group_grid(p.jag, lo, hi, p.M, p.N, bm, bn, p.align, tm, tn);
+      count = tm * tn;
+    }
+    incl = gmm_wave_inclusive_scan(count);
+    return __builtin_amdgcn_readlane(incl, 63);
+  }
+
+  // Group of tile t, the tile's index inside it, the group's range: uniform over the wave.
+  __device__ __forceinline__ void find(int t, int& g, int& local, int& glo, int& ghi) const {
+    g = __popcll(__ballot(incl <= t));
+    local = t - __builtin_amdgcn_readlane(incl, g) + __builtin_amdgcn_readlane(count, g);
+    glo = __builtin_amdgcn_readlane(lo, g);
+    ghi = __builtin_amdgcn_readlane(hi, g);
+  }
+};
 
 // ---- two-height tile list (gmm_sched.h): tables cum[0] (tall) and cum[1] (short), each G + 1 entries ---- //
 template <int NT>
@@ -180,6 +232,24 @@ __device__ __forceinline__ uint16_t gmm_bf16_bits(float f) {
   if ((u & 0x7fffffffu) > 0x7f800000u) return uint16_t((u >> 16) | 0x0040u);
   u += 0x7fffu + ((u >> 16) & 1u);
   return uint16_t(u >> 16);
+}
+
+// Four at a time: v_cvt_pk_bf16_f32 / v_cvt_pk_f16_f32 where there is one.
+template <typename OutT>
+__device__ __forceinline__ void gmm_store4(void* dst, const float* f) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+  const f4 v = {f[0], f[1], f[2], f[3]};
+  if constexpr (__is_same(OutT, float)) {
+    __builtin_memcpy(dst, &v, 16);
+  } else if constexpr (__is_same(OutT, gmm_f16)) {
+    const h4 h = __builtin_convertvector(v, h4);
+    __builtin_memcpy(dst, &h, 8);
+  } else {
+    const b4 b = __builtin_convertvector(v, b4);
+    __builtin_memcpy(dst, &b, 8);
+  }
 }
 
 template <typename T> __device__ __forceinline__ T gmm_from_float(float f);

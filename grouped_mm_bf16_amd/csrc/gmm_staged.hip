@@ -268,11 +268,17 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave & 1) * WTM, wn = (wave >> 1) * WTN;
-  const int total = gmm_build_tile_table<NT>(p, BM, BN, cum);
   const int64_t lda = A_TR ? p.a_sk : p.a_sm, ldb = B_TR ? p.b_sk : p.b_sn;
+  const bool in_registers = p.jag != GMM_JAG_NONE && p.G <= 64;
+  GmmWaveGroups groups{0, 0, 0, 0};
+  const int total = __builtin_amdgcn_readfirstlane(in_registers ? groups.build(p, BM, BN) : gmm_build_tile_table<NT>(p, BM, BN, cum));
 
   for (int t = blockIdx.x; t < total; t += gridDim.x) {
-    const GmmTile tile = gmm_locate_tile(p, cum, gmm_xcd_remap(t, total, gridDim.x), BM, BN);
+    const int id = gmm_xcd_remap(t, total, gridDim.x);
+    int g, local, lo, hi;
+    if (in_registers) groups.find(id, g, local, lo, hi);
+    else gmm_find_tile(p, cum, id, BM, BN, g, local, lo, hi);
+    const GmmTile tile = gmm_tile_of_group(p, g, local, lo, hi, BM, BN);
     const T* a = static_cast<const T*>(p.a) + int64_t(tile.g) * p.a_sg;
     const T* b = static_cast<const T*>(p.b) + int64_t(tile.g) * p.b_sg;
     OutT* c = static_cast<OutT*>(p.c) + int64_t(tile.g) * p.c_sg;
@@ -350,17 +356,15 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        OutT o[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = gmm_from_float<OutT>(acc[i][j][r]);
-        __builtin_memcpy(stage + (lane & 15) * EPITCH + (16 * j + 4 * (lane >> 4)) * OSZ, o, 4 * OSZ);
+        const float f[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+        gmm_store4<OutT>(stage + (lane & 15) * EPITCH + (16 * j + 4 * (lane >> 4)) * OSZ, f);
       }
       asm volatile("" ::: "memory");   // the wave's LDS accesses complete in order; the compiler must keep it
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int x = lane; x < 16 * ECPR; x += 64) {
         const int row = tile.m0 + wm + 16 * i + x / ECPR, col = tile.n0 + wn + (x % ECPR) * OEC;
-        if (row < tile.m_lo || row >= tile.m_hi) continue;
+        if (row < tile.m_lo || row >= tile.m_hi || col >= tile.n_hi || col + OEC <= tile.n_lo) continue;
         const char* src = stage + (x / ECPR) * EPITCH + (x % ECPR) * 16;
         OutT* dst = c + int64_t(row) * p.c_sm + int64_t(col) * p.c_sn;
         if (p.c_sn == 1 && col >= tile.n_lo && col + OEC <= tile.n_hi) {
