@@ -1,6 +1,7 @@
 // C ABI of libgrouped_mm_hip.so (declared in include/grouped_mm_hip.h): argument
 // checks, choice of kernel family, launch.  No allocation, no synchronisation,
 // no exceptions across the boundary.
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
@@ -354,14 +355,28 @@ static int64_t host_tile_list23(const int32_t* offs_host, int32_t G, int32_t jag
   p.offs = offs_host;
   p.G = G; p.jag = jagged; p.M = M; p.N = N; p.K = K; p.align = align; p.tall = tall; p.shrt = shrt;
   const int extent = jagged == GMM_JAG_M ? M : (jagged == GMM_JAG_N ? N : K);
+  // the queue of a jagged contraction runs the longest groups first (the order in which tiles are handed out)
+  std::vector<int32_t> order(size_t(G), 0);
+  for (int g = 0; g < G; ++g) order[g] = g;
+  if (gmm_use_k_queue(p, tile_n, num_workgroups)) {
+    std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
+      int xl, xh, yl, yh;
+      gmm_group_range(offs_host, x, extent, xl, xh);
+      gmm_group_range(offs_host, y, extent, yl, yh);
+      return xh - xl > yh - yl;
+    });
+    group_major = 1;   // every group's tall tiles, then its remainder tiles
+    xcd_remap = 0;     // the tickets of an XCD are neighbours already
+  }
   std::vector<int32_t> ct(size_t(G) + 1, 0), cs(size_t(G) + 1, 0);
-  for (int g = 0; g < G; ++g) {
+  for (int i = 0; i < G; ++i) {
+    const int g = order[i];
     int lo = 0, hi = 0, n_tall, n_short, rem_rows;
     if (jagged != GMM_JAG_NONE) gmm_group_range(offs_host, g, extent, lo, hi);
     gmm_split_rows(gmm_group_rows(jagged, lo, hi, M, align), tall, shrt, n_tall, n_short, rem_rows);
     const int tn = gmm_group_tile_cols(jagged, lo, hi, N, align, tile_n);
-    ct[g + 1] = ct[g] + n_tall * tn + (group_major ? n_short * tn : 0);
-    cs[g + 1] = cs[g] + (group_major ? 0 : n_short * tn);
+    ct[i + 1] = ct[i] + n_tall * tn + (group_major ? n_short * tn : 0);
+    cs[i + 1] = cs[i] + (group_major ? 0 : n_short * tn);
   }
   const int total_tall = ct[G], total_tiles = ct[G] + cs[G];
   // the split of the last round, as gmm_asm_kernel decides it
@@ -386,8 +401,8 @@ static int64_t host_tile_list23(const int32_t* offs_host, int32_t G, int32_t jag
     int cls = tt < total_tall ? 0 : 1;
     const int tc = cls ? tt - total_tall : tt;
     const std::vector<int32_t>& cum = cls ? cs : ct;
-    const int g = gmm_find_group(cum.data(), G, tc);
-    int lo = 0, hi = 0, local = tc - cum[g];
+    const int i = gmm_find_group(cum.data(), G, tc), g = order[i];
+    int lo = 0, hi = 0, local = tc - cum[i];
     if (jagged != GMM_JAG_NONE) gmm_group_range(offs_host, g, extent, lo, hi);
     if (group_major) {
       // one table: a group's tall tiles, then its remainder tiles

@@ -212,6 +212,98 @@ __device__ __forceinline__ GmmTile gmm_locate_tile2(const GmmParams& p, const in
   return gmm_make_tile2(p, g, lo, hi, cls, local, bn);
 }
 
+// ---- tile queue of a jagged contraction -------------------------------------------------------------- //
+// Every group has the same grid of tiles, but its contraction is as long as the group, so dealing tiles round by round
+// leaves whole chips waiting for the workgroups that drew the long groups: 32768 rows in 128 skewed groups, 2048 x 768
+// each, keep the average workgroup busy for 141 us of 234 in a model of the kernel's tile times (258 us measured).  Here the groups are
+// sorted by length, longest first, and a workgroup draws its next tile when it is free (143 us in the model, 211 measured; sorted
+// but dealt round by round 199, drawn in group order 199).
+// The sorted list is cut into spans of one tile per workgroup and every span into one block per XCD, so that the tiles
+// an XCD runs together are neighbours; each XCD has a counter of its own, in the head of the workspace, and a workgroup
+// whose XCD has nothing left draws from the others.  The first tile needs no draw, the following ticket is drawn
+// before a tile runs and looked at after it.  Without a workspace the list is dealt round by round.
+// One thread of the workgroup uses the queue; it ends when all eight counters have run out.
+struct GmmKQueue {
+  int per, total, chunk;   // tiles per group, of the launch, of an XCD's block in a span
+  int turn;                // counters that have run out, counted from the workgroup's own
+  int next;                // tile to run, -1: none left
+  int ticket;              // drawn ticket (index in the counter's part of the list)
+
+  // order[i] = group of rank i, bound[g] .. bound[g + 1] = range of group g.  All threads; ends with a barrier.
+  template <int NT>
+  __device__ __forceinline__ void build(const GmmParams& p, int bn, int32_t* order, int32_t* bound) {
+    const int tid = threadIdx.x;
+    for (int g = tid; g < p.G; g += NT) bound[g + 1] = gmm_min(gmm_max(p.offs[g], 0), p.K);
+    if (tid == 0) bound[0] = 0;
+    __syncthreads();
+    for (int g = tid; g < p.G; g += NT) {
+      const int mine = gmm_max(bound[g + 1] - bound[g], 0);
+      int rank = 0, before = 0;
+#pragma unroll 8
+      for (int h = 0; h < p.G; ++h) {
+        const int end = bound[h + 1], len = gmm_max(end - before, 0);
+        rank += (len > mine || (len == mine && h < g)) ? 1 : 0;
+        before = end;
+      }
+      order[rank] = g;
+    }
+    __syncthreads();
+    int n_tall, n_short, rem_rows;
+    gmm_split_rows(p.M, p.tall, p.shrt, n_tall, n_short, rem_rows);
+    per = (n_tall + n_short) * gmm_cdiv(p.N, bn);
+    total = p.G * per;
+    chunk = int(gridDim.x) >> 3;
+    turn = 0;
+    ticket = int(blockIdx.x) >> 3;
+    next = tile_of(int(blockIdx.x) & 7, ticket);
+  }
+
+  // Tile number `i` of an XCD's part of the list, or -1 past its end.
+  __device__ __forceinline__ int tile_of(int xcd, int i) const {
+    const int span = i / chunk;
+    const int t = (span * 8 + xcd) * chunk + (i - span * chunk);
+    return t < total ? t : -1;
+  }
+
+  __device__ __forceinline__ void draw(const GmmParams& p) {
+    if (!p.ws) { ticket += chunk; return; }
+    if (turn < 8)
+      ticket = chunk + int(__hip_atomic_fetch_add(static_cast<unsigned*>(p.ws) + ((blockIdx.x + turn) & 7) * GMM_WS_QUEUE_PITCH, 1u,
+                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  }
+
+  // The drawn ticket becomes the next tile; a counter that has run out is left for the next one.
+  __device__ __forceinline__ void advance(const GmmParams& p) {
+    next = tile_of(int(blockIdx.x + turn) & 7, ticket);
+    if (!p.ws) return;
+    while (next < 0 && ++turn < 8) {
+      draw(p);
+      next = tile_of(int(blockIdx.x + turn) & 7, ticket);
+    }
+  }
+
+  __device__ __forceinline__ GmmTile locate(const GmmParams& p, const int32_t* order, const int32_t* bound, int bn) const {
+    const int rank = next / per, g = order[rank];
+    int n_tall, n_short, rem_rows, local = next - rank * per;
+    gmm_split_rows(p.M, p.tall, p.shrt, n_tall, n_short, rem_rows);
+    const int tall_tiles = n_tall * gmm_cdiv(p.N, bn);
+    const int cls = local < tall_tiles ? 0 : 1;
+    const int lo = bound[g];
+    return gmm_make_tile2(p, g, lo, gmm_max(bound[g + 1], lo), cls, cls ? local - tall_tiles : local, bn);
+  }
+
+  // The last workgroup to leave puts the counters back to zero for the next launch: all others have drawn their last
+  // tickets.
+  __device__ __forceinline__ void leave(const GmmParams& p) const {
+    if (!p.ws) return;
+    unsigned* const header = static_cast<unsigned*>(p.ws);
+    if (__hip_atomic_fetch_add(&header[GMM_WS_EXITED], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
+    for (int x = 0; x < 8; ++x)
+      __hip_atomic_store(&header[x * GMM_WS_QUEUE_PITCH], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&header[GMM_WS_EXITED], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+};
+
 // Source row of product row m under a row gather; -1 if the index is outside the source matrix.
 __device__ __forceinline__ int gmm_gather_row(const GmmParams& p, int m) {
   const int s = p.gather[m];

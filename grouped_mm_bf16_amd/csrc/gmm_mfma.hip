@@ -459,8 +459,13 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   constexpr int ESZ = OUT_F32 ? 4 : 2;
   constexpr int CDIV = ACT ? 2 : 1;
 
-  int total_tall;
-  const int total_tiles = gmm_build_tile_table2<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, total_tall);
+  // Jagged contraction: the groups' tiles take different times, so the longest come first and a workgroup that is
+  // done takes the next one (GmmKQueue).
+  const bool queue = gmm_use_k_queue(p, GMM_TILE_N, int(gridDim.x));
+  int total_tall = 0, total_tiles = 0;
+  GmmKQueue q;
+  if (queue) q.build<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short);
+  else total_tiles = gmm_build_tile_table2<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, total_tall);
   // The tiles of the last, partly filled round may be cut along K into `nparts` parts each (gmm_tail_split).
   // Tiles before split_base are dealt round-robin (workgroup w takes w, w + grid, ...); the parts are taken
   // from a ticket counter in the workspace by whichever workgroup is free: part q is K part q / tail of tile
@@ -474,23 +479,30 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
 
   // Locating a tile (binary search over the groups, reads of offs, integer divisions) costs microseconds, so
   // BATCH threads locate the next BATCH round-robin tiles of the workgroup at once and leave them in LDS for
-  // the tile loop to pick up.
+  // the tile loop to pick up.  From the queue one thread locates one tile at a time (two LDS reads and a division),
+  // with a ticket that it drew before the previous tile ran.
   for (int first = 0;; first += BATCH) {
     const int64_t mine = int64_t(blockIdx.x) + int64_t(first + tid) * gridDim.x;
-    if (tid < BATCH && mine < split_base) {
+    if (queue) {
+      if (tid == 0) {
+        split_flag = q.next >= 0 ? 1 : 0;
+        if (q.next >= 0) gmm_store_rec(&tiles[0], q.locate(p, cum_tall, cum_short, GMM_TILE_N), -1);
+      }
+    } else if (tid < BATCH && mine < split_base) {
       const int t = int(mine);
       const int tt = p.xcd_remap ? gmm_xcd_remap(t, split_base, gridDim.x) : t;
       gmm_store_rec(&tiles[tid], gmm_locate_tile2(p, cum_tall, cum_short, total_tall, tt, GMM_TILE_N), -1);
     }
     __syncthreads();
     const int64_t left = (int64_t(split_base) - blockIdx.x + gridDim.x - 1) / gridDim.x - first;  // tiles of this workgroup from `first` on
-    const int here = left < BATCH ? int(left) : BATCH;
+    const int here = queue ? split_flag : left < BATCH ? int(left) : BATCH;
     for (int j = 0; j < here; ++j) {
       // Everything the assembly wants per lane is a cheap function of the lane id.  Hidden from the
       // optimiser per tile, or it hoists those values out of the loop, keeps them alive across the
       // assembly (which clobbers most registers) and spills them to scratch memory.
       int lane_j = lane;
       asm volatile("" : "+v"(lane_j));
+      if (queue && tid == 0) q.draw(p);
       const GmmTileScalars t = gmm_load_rec(&tiles[j]);
       const GmmTileDesc dsc = gmm_describe_tile<A_TR, B_TR, ESZ, CDIV>(p, t);
       if constexpr (A_TR) {
@@ -505,9 +517,11 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
         else gmm_tile_compute<A_TR, B_TR, OUT_F32, 1, F16, 1, ACT>(dsc, lds_base, lane_j, wave);
       }
     }
-    if (left <= BATCH) break;
+    if (queue ? here == 0 : left <= BATCH) break;
     __syncthreads();  // everyone is done with this batch of located tiles
+    if (queue && tid == 0) q.advance(p);
   }
+  if (queue && tid == 0) q.leave(p);
 
   // The parts of the tiles that were cut: drawn from the ticket counter, one at a time, located by the thread
   // that draws.  Each part's whole fp32 tile goes to its workspace slot; gmm_split_finish does the rest.

@@ -70,6 +70,7 @@ constexpr int GMM_SPLIT_PART_COST = 20;      // what a part costs beyond its K t
                                              // measured, a round of 56 tiles of 64 K tiles cut four ways takes as long as uncut
 constexpr int GMM_WS_TICKET = 1020;          // header words beyond the arrival counters: next part to hand out,
 constexpr int GMM_WS_EXITED = 1021;          // workgroups that have left the ticket loop
+constexpr int GMM_WS_QUEUE_PITCH = 32;       // jagged contraction (no arrival counters): words between the XCDs' tile counters
 
 GMM_HD int gmm_cdiv(int a, int b) { return (a + b - 1) / b; }
 GMM_HD int gmm_min(int a, int b) { return a < b ? a : b; }
@@ -211,6 +212,18 @@ GMM_HD int gmm_group_rows(int jag, int lo, int hi, int M, int align) {
 GMM_HD int gmm_group_tile_cols(int jag, int lo, int hi, int N, int align, int bn) {
   if (jag != GMM_JAG_N) return gmm_cdiv(N, bn);
   return hi > lo ? gmm_cdiv(hi - (lo / align) * align, bn) : 0;
+}
+
+// Does a launch with a jagged contraction hand out its tiles longest group first, on demand (GmmKQueue), or deal them
+// round by round in group order?  A group with at least as many tiles as the launch has workgroups gives every one of
+// them the same share, and workgroups that run in step share operand panels: dealt, 8 groups of 896 tiles (4096 x
+// 14336, 16384 rows, fp32 result) take 1682 us, from the queue 1698.  Smaller groups make uneven shares: 128 skewed
+// groups of 24 tiles (2048 x 768, 32768 rows) take 258 us dealt, 211 from the queue.
+GMM_HD bool gmm_use_k_queue(const GmmParams& p, int bn, int num_wg) {
+  if (p.jag != GMM_JAG_K) return false;
+  int n_tall, n_short, rem_rows;
+  gmm_split_rows(p.M, p.tall, p.shrt, n_tall, n_short, rem_rows);
+  return int64_t(n_tall + n_short) * gmm_cdiv(p.N, bn) < num_wg;
 }
 
 // One output tile, in global coordinates of the operands.
