@@ -439,7 +439,9 @@ __device__ __forceinline__ GmmTileDesc gmm_describe_tile(const GmmParams& p, con
   return dsc;
 }
 
-template <int A_TR, int B_TR, int OUT_F32, int F16, int ACT = 0>
+// QUEUE = 1: jagged contraction, the longest groups' tiles first, drawn on demand (GmmKQueue).  A kernel of its own: with
+// both ways in one, every other launch took 1.6 us longer.
+template <int A_TR, int B_TR, int OUT_F32, int F16, int ACT = 0, int QUEUE = 0>
 __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   constexpr int WAVES = 4;
   constexpr bool SHORT_TILES = !A_TR;
@@ -459,19 +461,16 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   constexpr int ESZ = OUT_F32 ? 4 : 2;
   constexpr int CDIV = ACT ? 2 : 1;
 
-  // Jagged contraction: the groups' tiles take different times, so the longest come first and a workgroup that is
-  // done takes the next one (GmmKQueue).
-  const bool queue = gmm_use_k_queue(p, GMM_TILE_N, int(gridDim.x));
   int total_tall = 0, total_tiles = 0;
   GmmKQueue q;
-  if (queue) q.build<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short);
+  if constexpr (QUEUE) q.build<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short);
   else total_tiles = gmm_build_tile_table2<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, total_tall);
   // The tiles of the last, partly filled round may be cut along K into `nparts` parts each (gmm_tail_split).
   // Tiles before split_base are dealt round-robin (workgroup w takes w, w + grid, ...); the parts are taken
   // from a ticket counter in the workspace by whichever workgroup is free: part q is K part q / tail of tile
   // split_base + q % tail.
   int nparts = 1, tail = 0;
-  if (!ACT && p.ws_parts > 0 && p.jag != GMM_JAG_K) {
+  if (!ACT && !QUEUE && p.ws_parts > 0 && p.jag != GMM_JAG_K) {
     nparts = gmm_tail_split(total_tiles, int(gridDim.x), gmm_cdiv(p.K, GMM_TILE_K), p.ws_parts);
     if (nparts > 1) tail = total_tiles % int(gridDim.x);
   }
@@ -483,7 +482,7 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   // with a ticket that it drew before the previous tile ran.
   for (int first = 0;; first += BATCH) {
     const int64_t mine = int64_t(blockIdx.x) + int64_t(first + tid) * gridDim.x;
-    if (queue) {
+    if constexpr (QUEUE) {
       if (tid == 0) {
         split_flag = q.next >= 0 ? 1 : 0;
         if (q.next >= 0) gmm_store_rec(&tiles[0], q.locate(p, cum_tall, cum_short, GMM_TILE_N), -1);
@@ -495,14 +494,14 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
     }
     __syncthreads();
     const int64_t left = (int64_t(split_base) - blockIdx.x + gridDim.x - 1) / gridDim.x - first;  // tiles of this workgroup from `first` on
-    const int here = queue ? split_flag : left < BATCH ? int(left) : BATCH;
+    const int here = QUEUE ? split_flag : left < BATCH ? int(left) : BATCH;
     for (int j = 0; j < here; ++j) {
       // Everything the assembly wants per lane is a cheap function of the lane id.  Hidden from the
       // optimiser per tile, or it hoists those values out of the loop, keeps them alive across the
       // assembly (which clobbers most registers) and spills them to scratch memory.
       int lane_j = lane;
       asm volatile("" : "+v"(lane_j));
-      if (queue && tid == 0) q.draw(p);
+      if (QUEUE && tid == 0) q.draw(p);
       const GmmTileScalars t = gmm_load_rec(&tiles[j]);
       const GmmTileDesc dsc = gmm_describe_tile<A_TR, B_TR, ESZ, CDIV>(p, t);
       if constexpr (A_TR) {
@@ -517,15 +516,15 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
         else gmm_tile_compute<A_TR, B_TR, OUT_F32, 1, F16, 1, ACT>(dsc, lds_base, lane_j, wave);
       }
     }
-    if (queue ? here == 0 : left <= BATCH) break;
+    if (QUEUE ? here == 0 : left <= BATCH) break;
     __syncthreads();  // everyone is done with this batch of located tiles
-    if (queue && tid == 0) q.advance(p);
+    if (QUEUE && tid == 0) q.advance(p);
   }
-  if (queue && tid == 0) q.leave(p);
+  if (QUEUE && tid == 0) q.leave(p);
 
   // The parts of the tiles that were cut: drawn from the ticket counter, one at a time, located by the thread
   // that draws.  Each part's whole fp32 tile goes to its workspace slot; gmm_split_finish does the rest.
-  if constexpr (!ACT) {
+  if constexpr (!ACT && !QUEUE) {
     if (nparts > 1) {
       unsigned* const ws_header = static_cast<unsigned*>(p.ws);
       const int n_parts = tail * nparts;
@@ -578,11 +577,11 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   }
 }
 
-template <int OUT_F32, int F16>
+template <int OUT_F32, int F16, int QUEUE>
 int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
   const dim3 grid(p.num_wg), block(256);
   if (p.act) {
-    if constexpr (OUT_F32) {
+    if constexpr (OUT_F32 || QUEUE) {
       return -1;
     } else {
       if (!lay.a_kc) return -1;
@@ -594,13 +593,13 @@ int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
     }
   }
   if (lay.a_kc && lay.b_kc)
-    hipLaunchKernelGGL((gmm_asm_kernel<0, 0, OUT_F32, F16>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gmm_asm_kernel<0, 0, OUT_F32, F16, 0, QUEUE>), grid, block, 0, stream, p);
   else if (lay.a_kc && !lay.b_kc)
-    hipLaunchKernelGGL((gmm_asm_kernel<0, 1, OUT_F32, F16>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gmm_asm_kernel<0, 1, OUT_F32, F16, 0, QUEUE>), grid, block, 0, stream, p);
   else if (!lay.a_kc && lay.b_kc)
-    hipLaunchKernelGGL((gmm_asm_kernel<1, 0, OUT_F32, F16>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gmm_asm_kernel<1, 0, OUT_F32, F16, 0, QUEUE>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((gmm_asm_kernel<1, 1, OUT_F32, F16>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gmm_asm_kernel<1, 1, OUT_F32, F16, 0, QUEUE>), grid, block, 0, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -617,6 +616,11 @@ int launch_layout(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
   else
     hipLaunchKernelGGL((gmm_mfma_kernel<BM, BN, WAVES_M, WAVES_N, false, false, OutT>), grid, block, 0, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+template <int OUT_F32, int F16>
+int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
+  return gmm_use_k_queue(p, GMM_TILE_N, p.num_wg) ? launch_asm<OUT_F32, F16, 1>(p, lay, stream) : launch_asm<OUT_F32, F16, 0>(p, lay, stream);
 }
 
 }  // namespace
