@@ -137,6 +137,7 @@ int run(Problem& pr, hipStream_t stream) {
     p.xcd_remap = g_xcd_remap.load(std::memory_order_relaxed);
     int cfg = g_forced_config.load(std::memory_order_relaxed);
     if (cfg == GMM_CFG_ASM_256x256 && !can_asm) return GMM_ERR_UNSUPPORTED;
+    const bool automatic = forced == GMM_PATH_AUTO && (cfg < 0 || cfg >= GMM_CFG_COUNT);
     if (cfg < 0 || cfg >= GMM_CFG_COUNT) cfg = can_asm ? GMM_CFG_ASM_256x256 : GMM_CFG_REG_256x256;
     if ((p.gather || p.act) && cfg != GMM_CFG_ASM_256x256) return GMM_ERR_UNSUPPORTED;
     if (pr.in_dtype != GMM_DT_BF16 && cfg != GMM_CFG_ASM_256x256) return GMM_ERR_UNSUPPORTED;
@@ -162,7 +163,10 @@ int run(Problem& pr, hipStream_t stream) {
       const int fo = g_group_major.load(std::memory_order_relaxed);
       p.group_major = fo >= 0 ? fo : (p.tall == 128 ? 1 : 0);
     }
-    rc = gmm_launch_mfma(p, lay, pr.in_dtype, pr.out_dtype, cfg, cus, stream);
+    // small products of the automatic choice run on 128 x 128 tiles of the register-staged kernel
+    rc = automatic && cfg == GMM_CFG_ASM_256x256 && gmm_staged_preferred(p, cus)
+             ? gmm_launch_staged(p, pr.in_dtype, pr.out_dtype, cus, stream)
+             : gmm_launch_mfma(p, lay, pr.in_dtype, pr.out_dtype, cfg, cus, stream);
     t_last_path = GMM_PATH_MFMA;
     t_last_config = cfg;
   } else {

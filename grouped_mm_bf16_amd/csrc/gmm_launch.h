@@ -10,6 +10,8 @@ int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hi
 // Register-staged MFMA kernel for operands of any alignment (gmm_staged.hip): each operand contiguous along one of
 // its dimensions.  Returns like gmm_launch_generic.
 bool gmm_staged_eligible(const GmmParams& p);
+// Of the 16-bit products that the assembly tile could take: true for those that the register-staged kernel runs faster.
+bool gmm_staged_preferred(const GmmParams& p, int num_cus);
 int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream);
 
 // Operand layout facts the host derived from strides.

@@ -406,6 +406,14 @@ int64_t expected_tiles(const GmmParams& p, int edge) {
   return p.G * tm * tn;
 }
 
+// The same if every group boundary cuts a whole tile more.
+int64_t most_tiles(const GmmParams& p, int edge) {
+  const int64_t tm = (p.M + edge - 1) / edge, tn = (p.N + edge - 1) / edge;
+  if (p.jag == GMM_JAG_M) return (p.M / edge + (p.G < p.M ? p.G : p.M)) * tn;
+  if (p.jag == GMM_JAG_N) return tm * (p.N / edge + (p.G < p.N ? p.G : p.N));
+  return p.G * tm * tn;
+}
+
 // fp32: 64 x 64 tiles (four workgroups per CU) or 128 x 128 (two)?  A launch takes whole rounds of its grid, and a
 // round of large tiles takes 1.84 times a round of small ones (2048 x 2048 x 2048, four products: 2 rounds of 258 us
 // against 4 of 140 us), so the cheaper count wins.  Measured, us, small / large: 1024 rows, K 1024, 8192 columns in
@@ -422,6 +430,25 @@ bool small_tiles(const GmmParams& p, int in_dtype, int num_cus) {
 }
 
 }  // namespace
+
+// Aligned 16-bit products that this kernel runs faster than the assembly tile, which takes up to 256 x 256 elements
+// of output and needs 3.3 us before its first tile (1 us here): little work, spread over more and smaller tiles by four
+// times as many workgroups.  T tiles of 128 x 128 with nk K tiles each; us, assembly tile / here:
+//   A contiguous along K: six groups of 32 x 64 x 48 9.5 / 5.5; 131072 x 32 x 64 in 64 groups 28 / 13.7; 8192 x 256 x
+//   384 in 64 groups 13.5 / 9.9.  Over 260 random shapes, operands from memory, the ratio is 1.46 at nk = 1, 1.33 at 2, 1.17
+//   at 4, 1.12 at 6 and 1.05 with every third shape slower at 8, where the assembly tile has three K tiles in flight.  Past
+//   T nk = 3072 its larger tile moves less between L2 and LDS (16384 x 256 x 4096 in 8 groups 55 / 72), and groups shorter
+//   than its 64-row tile fill half a tile here (750 tiles of 264 x 424 x 1264 in 73 groups 26 / 29).
+//   A contiguous along M: the assembly tile always has 256 rows.  1256 x 824 x 456 in 11 groups 32 / 21; 1392 x 1312 x
+//   352 in 40 groups 47 / 37; 2160 tiles of 1880 x 144 x 1120 35 / 37.  It wins once there are rounds to fill.
+// Jagged contractions stay with the assembly tile, whose tiles are drawn from a queue.
+bool gmm_staged_preferred(const GmmParams& p, int num_cus) {
+  if (p.jag == GMM_JAG_K || p.act || !gmm_staged_eligible(p)) return false;
+  const int64_t tiles = most_tiles(p, 128), nk = (p.K + 63) / 64, cus = num_cus;
+  if (p.a_sk != 1 && tiles <= tile_wgs(128) * cus && nk <= 32) return true;
+  const bool rows_fill = p.jag == GMM_JAG_M ? p.M >= 64 * int64_t(p.G) : p.M >= 64;
+  return nk <= 6 && tiles * nk <= 12 * cus && (nk == 1 || rows_fill || tiles <= cus);
+}
 
 bool gmm_staged_eligible(const GmmParams& p) {
   // each operand contiguous along one of its dimensions; gathered rows only along K; element offsets are 64-bit, so

@@ -209,7 +209,9 @@ int gmm_moe_combine(const void* y, const int32_t* token_rows, const float* slot_
 int gmm_set_path(int path);
 int gmm_last_path(void);
 /* Tile configuration of the MFMA family: -1 = choose from the shapes, 0 = register-staged kernel,
- * 1 = assembly tile (256 / 128 / 64-row tiles).  Returns the previous setting. */
+ * 1 = assembly tile (256 / 128 / 64-row tiles).  Returns the previous setting.  With -1 and GMM_PATH_AUTO, calls that
+ * the assembly tile could take but that are too small for it run on 128 x 128 tiles of the kernel for operands of any
+ * alignment; gmm_last_mfma_config reports 1 for them as well. */
 int gmm_set_mfma_config(int config);
 int gmm_last_mfma_config(void);
 /* 0 / 1: renumber tiles per XCD (default 1). */

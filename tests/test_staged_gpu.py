@@ -121,3 +121,48 @@ def test_operands_smaller_than_a_chunk_and_strided_outputs():
     out = torch.full((2, 130, 70), float("nan"), device=DEV, dtype=torch.bfloat16).transpose(1, 2)
     K_.grouped_mm_3d3d(a.to(DEV), b.to(DEV), out)
     compare(out, a, b, None, "column-major output")
+
+
+# both sides of each line of the rule that sends small aligned products to these kernels: K 384 / 392 (6 K tiles), rows per
+# group 64 / 63 with more than 256 tiles, 128-row tiles times K tiles around 3072, first operand contiguous along M
+@pytest.mark.parametrize("variant,G,M,K,N,a_col,small", [
+    ("2d3d", 6, 32, 64, 48, False, True), ("2d3d", 3, 200, 384, 136, False, True), ("2d3d", 3, 200, 392, 136, False, False),
+    ("2d3d", 70, 4480, 72, 640, False, True), ("2d3d", 70, 4472, 72, 640, False, False), ("2d3d", 70, 4472, 64, 640, False, True),
+    ("3d3d", 48, 1000, 64, 1024, False, True), ("3d3d", 49, 1000, 64, 1024, False, False),
+    ("3d3d", 4, 136, 1032, 264, True, True), ("3d3d", 3, 40, 2056, 72, True, False),
+    ("3d2d", 5, 264, 384, 1000, False, True), ("3d2d", 5, 264, 776, 1000, True, True)])
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)])
+def test_small_aligned_products_take_these_kernels(variant, G, M, K, N, a_col, small, dtype, out_dtype):
+    gen = torch.Generator().manual_seed(G + M + K + N)
+    r = lambda *s: torch.randn(*s, generator=gen).to(dtype)
+    col = lambda x, c: x.to(DEV).transpose(-2, -1).contiguous().transpose(-2, -1) if c else x.to(DEV)
+    offs = None
+    if variant != "3d3d":
+        tot = M if variant == "2d3d" else N
+        cuts = torch.randint(0, tot + 1, (G,), generator=gen).sort().values
+        cuts[-1] = tot - 3                                # the last three rows or columns belong to nobody
+        offs = cuts.clamp(max=tot - 3).to(torch.int32)
+    if variant == "2d3d":
+        a, b, shape, fn = r(M, K), r(G, K, N), (M, N), K_.grouped_mm_2d3d
+    elif variant == "3d3d":
+        a, b, shape, fn = r(G, M, K), r(G, K, N), (G, M, N), K_.grouped_mm_3d3d
+    else:
+        a, b, shape, fn = r(G, M, K), r(K, N), (M, N), K_.grouped_mm_3d2d
+    for b_col in (False, True):
+        ad, bd = col(a, a_col), col(b, b_col)
+        args = (ad, bd) if offs is None else (ad, bd, offs.to(DEV))
+
+        def launch():
+            out = torch.full(shape, float("nan"), device=DEV, dtype=out_dtype)
+            fn(*args, out)
+            return out
+
+        got = launch()
+        assert K_.last_path() == "mfma"
+        if small:                                         # the same kernel, so the same bits
+            with K_.forced_path("generic"):
+                same = launch()
+            bits = torch.int32 if out_dtype == torch.float32 else torch.int16
+            assert torch.equal(got.view(bits), same.view(bits))
+        if G * M * N < 1 << 21:
+            compare(got, a, b, offs, f"{variant} {dtype} b_col={b_col}")
