@@ -7,8 +7,9 @@
 // Exclusive prefix sum of per-group tile counts into cum[0..G] (LDS), returns
 // the total.  All NT threads of the workgroup must call it; it ends with a
 // barrier.  For 3D x 3D there is no table: every group has the same grid.
+// chunk > 0: a group counts once for each of its parts along K (gmm_group_parts).
 template <int NT>
-__device__ __forceinline__ int gmm_build_tile_table(const GmmParams& p, int bm, int bn, int32_t* cum) {
+__device__ __forceinline__ int gmm_build_tile_table(const GmmParams& p, int bm, int bn, int32_t* cum, int chunk = 0) {
   const int tid = threadIdx.x;
   if (p.jag == GMM_JAG_NONE) return p.G * gmm_cdiv(p.M, bm) * gmm_cdiv(p.N, bn);
 
@@ -19,7 +20,7 @@ __device__ __forceinline__ int gmm_build_tile_table(const GmmParams& p, int bm, 
       int lo, hi, tm, tn;
       gmm_group_range(p.offs, g, extent, lo, hi);
       gmm_group_grid(p.jag, lo, hi, p.M, p.N, bm, bn, p.align, tm, tn);
-      cnt = tm * tn;
+      cnt = tm * tn * gmm_group_parts(hi - lo, chunk);
     }
     cum[g + 1] = cnt;
   }
@@ -99,7 +100,7 @@ struct GmmWaveGroups {
   int lo, hi, count, incl;   // of the lane's group: its range, its tiles, tiles up to and including it
 
   // Returns the total number of tiles.
-  __device__ __forceinline__ int build(const GmmParams& p, int bm, int bn) {
+  __device__ __forceinline__ int build(const GmmParams& p, int bm, int bn, int chunk = 0) {
     const int lane = threadIdx.x & 63;
     const int extent = p.jag == GMM_JAG_M ? p.M : (p.jag == GMM_JAG_N ? p.N : p.K);
     lo = hi = count = 0;
@@ -107,7 +108,7 @@ struct GmmWaveGroups {
       int tm, tn;
       gmm_group_range(p.offs, lane, extent, lo, hi);
       gmm_group_grid(p.jag, lo, hi, p.M, p.N, bm, bn, p.align, tm, tn);
-      count = tm * tn;
+      count = tm * tn * gmm_group_parts(hi - lo, chunk);
     }
     incl = gmm_wave_inclusive_scan(count);
     return __builtin_amdgcn_readlane(incl, 63);

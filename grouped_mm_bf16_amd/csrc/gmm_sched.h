@@ -60,6 +60,9 @@ struct GmmParams {
   // 1: group by group, a group's remainder tiles right after its tall tiles, while the group's second
   // operand is still in the Infinity Cache.
   int32_t group_major;
+  // Register-staged kernel, jagged contraction: elements of K per part of a group (gmm_group_parts) and the most parts
+  // that the workspace has room for; 0: no group is cut.
+  int32_t k_chunk, k_parts;
 };
 
 constexpr int GMM_WS_HEADER = 4096;          // 1024 int32: arrival counters, one per tile of the split round, ...
@@ -103,6 +106,13 @@ GMM_HD int gmm_tail_split(int total, int W, int nk, int max_parts) {
 GMM_HD void gmm_part_ktiles(int nk, int S, int part, int& first, int& last) {
   first = int(int64_t(part) * nk / S);
   last = int(int64_t(part + 1) * nk / S);
+}
+
+// Parts that a group of `len` elements is cut into along K.
+constexpr int GMM_K_PARTS_MAX = 64;     // of a group
+constexpr int GMM_K_CLUSTER = 8;        // parts whose partial tiles are added in one go
+GMM_HD int gmm_group_parts(int len, int chunk) {
+  return chunk > 0 && len > chunk ? gmm_min(gmm_cdiv(len, chunk), GMM_K_PARTS_MAX) : 1;
 }
 
 // [lo, hi) of group g along the jagged dimension, clamped into [0, extent] and

@@ -250,7 +250,105 @@ __device__ __forceinline__ void multiply(const uint4 (&a)[TM], const uint4 (&b)[
   }
 }
 
-template <typename T, typename OutT, bool A_TR, bool B_TR, int EDGE>
+// ---- jagged contractions cut along K ---------------------------------------------------------------- //
+// A weight gradient of small matrices has few tiles and a contraction as long as the group: 64 groups of 32 x 64 with 2048
+// elements each are 64 tiles, two groups of 88 x 48 over 64920 elements two.  A group longer than p.k_chunk is cut into
+// parts (gmm_group_parts); a tile of a part is an entry of the tile list like any other, number `id`, and leaves its
+// accumulators in slot `id` of the workspace as they lie in the registers.  Up to GMM_K_CLUSTER neighbouring parts form a
+// cluster: the part that finds all others of its cluster there adds the slots in the order of the parts, and so, one level
+// up, does the cluster that comes last.  The sum does not depend on timing, and nobody waits.  Counters (word `id` of the
+// workspace's header: of the cluster's first part for the cluster, of the tile's second part for the tile) are left
+// at zero.  A part's tiles are neighbours in the list, so that what they share of A and B is read together.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+template <int TM, int TN, int EDGE>
+struct Partial {
+  static constexpr int SLOT = EDGE * EDGE * 4;
+  __amdgpu_buffer_rsrc_t slots;
+  int rows, cols;    // 16 x 16 blocks of the wave that hold something
+
+  __device__ __forceinline__ Partial(const GmmParams& p, const GmmTile& tile, int wm, int wn) {
+    slots = __builtin_amdgcn_make_buffer_rsrc(static_cast<char*>(p.ws) + GMM_WS_HEADER, 0, 0x7fffffff, 0x00020000);
+    rows = gmm_min(gmm_max(gmm_cdiv(tile.m_hi - tile.m0 - wm, 16), 0), TM);
+    cols = gmm_min(gmm_max(gmm_cdiv(tile.n_hi - tile.n0 - wn, 16), 0), TN);
+  }
+  static __device__ __forceinline__ int at(int slot, int i, int j) {
+    return slot * SLOT + ((i * TN + j) * NT + int(threadIdx.x)) * 16;
+  }
+  // Stored through to memory at device scope and read past this XCD's L2 (sc1).
+  __device__ __forceinline__ void store(const f32x4 (&acc)[TM][TN], int slot) const {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        u32x4 v;
+        __builtin_memcpy(&v, &acc[i][j], 16);
+        if (i < rows && j < cols) __builtin_amdgcn_raw_buffer_store_b128(v, slots, at(slot, i, j), 0, 16 /* sc1 */);
+      }
+  }
+  // acc = sum of n slots `stride` apart.
+  __device__ __forceinline__ void add(f32x4 (&acc)[TM][TN], int slot, int stride, int n) const {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int x = 0; x < n; ++x) {
+      u32x4 v[TM][TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          v[i][j] = u32x4{0u, 0u, 0u, 0u};
+          if (i < rows && j < cols) v[i][j] = __builtin_amdgcn_raw_buffer_load_b128(slots, at(slot + x * stride, i, j), 0, 16 /* sc1 */);
+        }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          f32x4 f;
+          __builtin_memcpy(&f, &v[i][j], 16);
+          acc[i][j] += f;
+        }
+    }
+  }
+};
+
+// Count this workgroup in on counter `word`; true in all threads of the one that completes `n`.  Everything that the
+// workgroup stored before is visible to the device by then.
+__device__ __forceinline__ bool arrive(const GmmParams& p, int word, int n, int* flag) {
+  unsigned* const counter = static_cast<unsigned*>(p.ws) + word;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const bool last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == unsigned(n - 1);
+    if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = last ? 1 : 0;
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(*flag) != 0;
+}
+
+// Part `part` of `parts` of a tile whose first part is entry `id0` of the list and whose parts are `per` entries apart.
+// True if acc now holds the whole tile.
+template <int TM, int TN, int EDGE>
+__device__ __forceinline__ bool join_parts(const GmmParams& p, const GmmTile& tile, f32x4 (&acc)[TM][TN], int wm, int wn,
+                                           int id0, int per, int part, int parts, int* flag) {
+  const Partial<TM, TN, EDGE> partial(p, tile, wm, wn);
+  const int first = part / GMM_K_CLUSTER * GMM_K_CLUSTER, in_cluster = gmm_min(GMM_K_CLUSTER, parts - first);
+  const int clusters = gmm_cdiv(parts, GMM_K_CLUSTER);
+  partial.store(acc, id0 + part * per);
+  if (!arrive(p, id0 + first * per, in_cluster, flag)) return false;
+  partial.add(acc, id0 + first * per, per, in_cluster);
+  if (clusters == 1) return true;
+  partial.store(acc, id0 + first * per);
+  if (!arrive(p, id0 + per, clusters, flag)) return false;
+  partial.add(acc, id0, GMM_K_CLUSTER * per, clusters);
+  return true;
+}
+
+// SPLIT: a jagged contraction whose groups may be cut along K.
+template <typename T, typename OutT, bool A_TR, bool B_TR, int EDGE, bool SPLIT>
 __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const GmmParams p) {
   constexpr int BM = EDGE, BN = EDGE;
   constexpr int AHEAD = sizeof(T) == 4 ? 2 : 1;   // K tiles fetched ahead (see the top of the file)
@@ -264,6 +362,7 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
   constexpr int PIPE = 2 * (ImA::BYTES + ImB::BYTES), EPI = 4 * 16 * EPITCH;
   __shared__ __attribute__((aligned(16))) char lds[PIPE > EPI ? PIPE : EPI];
   __shared__ int32_t cum[GMM_MAX_GROUPS + 1];
+  __shared__ int flag;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -271,14 +370,36 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
   const int64_t lda = A_TR ? p.a_sk : p.a_sm, ldb = B_TR ? p.b_sk : p.b_sn;
   const bool in_registers = p.jag != GMM_JAG_NONE && p.G <= 64;
   GmmWaveGroups groups{0, 0, 0, 0};
-  const int total = __builtin_amdgcn_readfirstlane(in_registers ? groups.build(p, BM, BN) : gmm_build_tile_table<NT>(p, BM, BN, cum));
+  int chunk = SPLIT ? p.k_chunk : 0;
+  auto build = [&]() {
+    return __builtin_amdgcn_readfirstlane(in_registers ? groups.build(p, BM, BN, chunk) : gmm_build_tile_table<NT>(p, BM, BN, cum, chunk));
+  };
+  int total = build();
+  if (SPLIT && chunk && total > p.k_parts) {   // offsets that overlap: more parts than K elements have room for
+    chunk = 0;
+    __syncthreads();
+    total = build();
+  }
 
   for (int t = blockIdx.x; t < total; t += gridDim.x) {
     const int id = gmm_xcd_remap(t, total, gridDim.x);
     int g, local, lo, hi;
     if (in_registers) groups.find(id, g, local, lo, hi);
     else gmm_find_tile(p, cum, id, BM, BN, g, local, lo, hi);
-    const GmmTile tile = gmm_tile_of_group(p, g, local, lo, hi, BM, BN);
+    int part = 0, parts = 1, per = 1;
+    if constexpr (SPLIT) {
+      parts = gmm_group_parts(hi - lo, chunk);
+      per = gmm_cdiv(p.M, BM) * gmm_cdiv(p.N, BN);
+      part = local / per;
+      local -= part * per;
+    }
+    GmmTile tile = gmm_tile_of_group(p, g, local, lo, hi, BM, BN);
+    if (SPLIT && parts > 1) {
+      int first, last;
+      gmm_part_ktiles(gmm_cdiv(hi - lo, BK), parts, part, first, last);
+      tile.k_lo = lo + first * BK;
+      tile.k_hi = gmm_min(lo + last * BK, hi);
+    }
     const T* a = static_cast<const T*>(p.a) + int64_t(tile.g) * p.a_sg;
     const T* b = static_cast<const T*>(p.b) + int64_t(tile.g) * p.b_sg;
     OutT* c = static_cast<OutT*>(p.c) + int64_t(tile.g) * p.c_sg;
@@ -350,6 +471,8 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
       }
     }
 
+    if (SPLIT && parts > 1 && !join_parts<TM, TN, EDGE>(p, tile, acc, wm, wn, id - part * per, per, part, parts, &flag)) continue;
+
     // Block (i, j), register r: row 16 i + lane % 16, column 16 j + 4 (lane / 16) + r of the wave's part.
     char* const stage = lds + wave * (16 * EPITCH);
 #pragma unroll
@@ -382,20 +505,50 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
   }
 }
 
-template <typename T, typename OutT, int EDGE>
-int launch_layout(GmmParams p, bool a_tr, bool b_tr, int num_cus, hipStream_t stream) {
-  const int64_t bound = (gmm_tile_bound(p.jag, p.G, p.M, p.N, EDGE, EDGE) + 7) / 8 * 8, most = int64_t(tile_wgs(EDGE)) * num_cus;
-  p.num_wg = int(bound < most ? (bound < 8 ? 8 : bound) : most);
+template <typename T, typename OutT, int EDGE, bool SPLIT>
+int launch_layout(const GmmParams& p, bool a_tr, bool b_tr, hipStream_t stream) {
   const dim3 grid(p.num_wg), block(NT);
   if (a_tr && b_tr)
-    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, true, true, EDGE>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, true, true, EDGE, SPLIT>), grid, block, 0, stream, p);
   else if (a_tr)
-    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, true, false, EDGE>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, true, false, EDGE, SPLIT>), grid, block, 0, stream, p);
   else if (b_tr)
-    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, false, true, EDGE>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, false, true, EDGE, SPLIT>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, false, false, EDGE>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, false, false, EDGE, SPLIT>), grid, block, 0, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+// Cut the groups of a jagged contraction along K?  Into parts of an even share of one round of the grid each, so
+// that the chip is full whatever the groups' lengths, but not shorter than GMM_K_CHUNK_MIN: a part costs its start, a store
+// and a read of its partial tile.  Sets k_chunk and k_parts; returns the most entries of the list, 0 if nothing is cut.
+constexpr int GMM_K_CHUNK_MIN = 256;
+template <int EDGE>
+int64_t cut_contraction(GmmParams& p, int64_t most_wgs) {
+  p.k_chunk = p.k_parts = 0;
+  if (p.jag != GMM_JAG_K || p.ws_parts <= 0) return 0;
+  const int64_t per = int64_t((p.M + EDGE - 1) / EDGE) * ((p.N + EDGE - 1) / EDGE);
+  const int64_t share = (p.K * per + most_wgs - 1) / most_wgs;
+  const int64_t chunk = share < GMM_K_CHUNK_MIN ? GMM_K_CHUNK_MIN : (share + 63) / 64 * 64;
+  // entries of the list: every group's tiles once, and once more for every whole chunk; they need a counter and a slot
+  const int64_t entries = p.G * per + p.K / chunk * per;
+  int64_t room = int64_t(p.ws_parts) * GMM_WS_SLOT / (EDGE * EDGE * 4);
+  if (room > GMM_WS_TICKET) room = GMM_WS_TICKET;
+  if (entries > room || p.K < 2 * chunk) return 0;
+  p.k_chunk = int32_t(chunk);
+  p.k_parts = int32_t(room);
+  return entries;
+}
+
+template <typename T, typename OutT, int EDGE>
+int launch_layout(GmmParams p, bool a_tr, bool b_tr, int num_cus, hipStream_t stream) {
+  const int64_t most = int64_t(tile_wgs(EDGE)) * num_cus;
+  int64_t bound = cut_contraction<EDGE>(p, most);
+  if (bound == 0) bound = gmm_tile_bound(p.jag, p.G, p.M, p.N, EDGE, EDGE);
+  const int64_t want = (bound + 7) / 8 * 8;
+  p.num_wg = int(want < most ? (want < 8 ? 8 : want) : most);
+  return p.k_chunk ? launch_layout<T, OutT, EDGE, true>(p, a_tr, b_tr, stream)
+                   : launch_layout<T, OutT, EDGE, false>(p, a_tr, b_tr, stream);
 }
 
 // Tiles of a launch with square tiles of `edge`, the group boundaries taken to cut half a tile each on average.
@@ -441,10 +594,21 @@ bool small_tiles(const GmmParams& p, int in_dtype, int num_cus) {
 //   than its 64-row tile fill half a tile here (750 tiles of 264 x 424 x 1264 in 73 groups 26 / 29).
 //   A contiguous along M: the assembly tile always has 256 rows.  1256 x 824 x 456 in 11 groups 32 / 21; 1392 x 1312 x
 //   352 in 40 groups 47 / 37; 2160 tiles of 1880 x 144 x 1120 35 / 37.  It wins once there are rounds to fill.
-// Jagged contractions stay with the assembly tile, whose tiles are drawn from a queue.
+//   Jagged contraction: cut along K (above) it fills the chip whatever the groups' lengths.  A contiguous along M, up to 384
+//   tiles: 64 groups of 32 x 64 with 2048 elements each 46 / 13; 24 groups of 328 x 360, 95496 elements 201 / 98; two groups
+//   of 328 x 712, 40424 elements 652 / 62; past 384 the larger tile catches up (496 tiles of 184 x 464 in 62 even groups
+//   70 / 78), but for very short groups (1230 tiles of 104 x 1248 in 123 groups, 16464 elements 69 / 52).  A contiguous along
+//   K: its 16-byte loads start at any element here, which costs more than it gains unless the contraction is long and
+//   the tiles are few (28 tiles of 112 x 888 in 4 groups, 44536 elements 415 / 65; 80 tiles of 200 x 968 in 5 groups, 2960
+//   elements 19 / 26) or the groups are a K tile at most.
 bool gmm_staged_preferred(const GmmParams& p, int num_cus) {
-  if (p.jag == GMM_JAG_K || p.act || !gmm_staged_eligible(p)) return false;
+  if (p.act || !gmm_staged_eligible(p)) return false;
   const int64_t tiles = most_tiles(p, 128), nk = (p.K + 63) / 64, cus = num_cus;
+  if (p.jag == GMM_JAG_K) {
+    const bool short_groups = p.K <= 64 * int64_t(p.G);
+    if (p.a_sk != 1) return 2 * tiles <= 3 * cus || (short_groups && tiles <= 4 * cus);
+    return (2 * tiles <= cus && p.K >= 1024 * int64_t(p.G)) || (tiles <= cus && short_groups);
+  }
   if (p.a_sk != 1 && tiles <= tile_wgs(128) * cus && nk <= 32) return true;
   const bool rows_fill = p.jag == GMM_JAG_M ? p.M >= 64 * int64_t(p.G) : p.M >= 64;
   return nk <= 6 && tiles * nk <= 12 * cus && (nk == 1 || rows_fill || tiles <= cus);
