@@ -44,6 +44,16 @@ def test_routing_matches_the_oracle(T, E, k, dtype):
         check_routing(got, moe_oracle.route(logits, k, renorm))
 
 
+@pytest.mark.parametrize("T,E,k", [(1, 1, 1), (4096, 3, 1), (4097, 3, 1), (128, 1023, 32), (129, 1023, 32), (585, 65, 7),
+                                   (16, 128, 4), (1025, 64, 2)])
+def test_slots_at_the_edges_of_the_one_workgroup_sort(T, E, k):
+    """Up to 4096 slots one workgroup of 16 waves sorts, 64 slots of a wave at a time; above, one workgroup per 1024 slots."""
+    gen = torch.Generator().manual_seed(T + E + k)
+    logits = torch.randn(T, E, generator=gen)
+    logits[:, 0] += 2.0
+    check_routing(moe.moe_route(logits.to(DEV), k), moe_oracle.route(logits, k, True))
+
+
 def test_routing_fp16_skewed_padded_and_empty():
     gen = torch.Generator().manual_seed(3)
     # skew: most tokens pick expert 0, several experts stay empty
