@@ -37,6 +37,12 @@ def _require_gpu(*tensors) -> None:
             raise RuntimeError("grouped_mm_bf16 is GPU-only (CUDA/HIP); CPU tensors are not supported")
 
 
+def current_stream(device: torch.device) -> int:
+    """Handle of torch's current stream of `device`.  ``torch.cuda.current_stream().cuda_stream`` builds a Stream object
+    for it: 2.6 us of a 17 us call, this 0.1 us."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
 # One workspace per (device, stream): launches on one stream run one after the other, so they can share it;
 # launches on different streams may overlap and must not.  Allocated on first use and kept (the library leaves
 # the arrival counters at its head zero after every launch).
@@ -68,7 +74,7 @@ def _launch_now(variant: int, a: torch.Tensor, b: torch.Tensor, offs: Optional[t
     # the device guard costs microseconds; only switch when the tensors live on another device
     guard = torch.cuda.device(a.device) if a.device.index != torch.cuda.current_device() else contextlib.nullcontext()
     with guard:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = current_stream(a.device)
         pa, pb, po = a.data_ptr(), b.data_ptr(), out.data_ptr()
         poffs = offs.data_ptr() if offs is not None else None
         ws, ws_bytes = workspace(a.device, stream)

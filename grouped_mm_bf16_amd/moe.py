@@ -62,7 +62,7 @@ def _route_packed_now(router_logits: torch.Tensor, top_k: int, renormalize: bool
         rc = lib.gmm_moe_route(router_logits.data_ptr(), router_logits.stride(0) if T else E,
                                _dtype_code(router_logits.dtype), T, E, top_k, int(bool(renormalize)),
                                base, base + 4 * E, base + 4 * (E + S), base + 4 * (E + 2 * S), base + 4 * (E + 3 * S),
-                               ws.data_ptr(), ws_bytes, torch.cuda.current_stream().cuda_stream)
+                               ws.data_ptr(), ws_bytes, kernels.current_stream(dev))
     _lib.check(rc, "moe_route")
     return buf[:E + 4 * S]
 
@@ -143,7 +143,7 @@ def _gathered_now(a: torch.Tensor, row_index: torch.Tensor, b: torch.Tensor, off
         return out.zero_()
     lib = _lib.load()
     with _guard(a):
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = kernels.current_stream(a.device)
         ws, ws_bytes = kernels.workspace(a.device, stream)
         rc = lib.gmm_2d3d_gather(a.data_ptr(), row_index.data_ptr(), b.data_ptr(), out.data_ptr(), offs.data_ptr(),
                                  offs.numel(), a.size(0), M, N, a.size(1), a.stride(0), a.stride(1),
@@ -211,7 +211,7 @@ def _swiglu_now(a: torch.Tensor, row_index: torch.Tensor | None, b: torch.Tensor
         rc = lib.gmm_2d3d_swiglu(a.data_ptr(), row_index.data_ptr() if row_index is not None else None, b.data_ptr(),
                                  out.data_ptr(), offs.data_ptr(), offs.numel(), a.size(0), M, N, a.size(1),
                                  a.stride(0), a.stride(1), b.stride(0), b.stride(1), b.stride(2), out.stride(0), out.stride(1),
-                                 _dtype_code(a.dtype), torch.cuda.current_stream().cuda_stream)
+                                 _dtype_code(a.dtype), kernels.current_stream(a.device))
     _lib.check(rc, "grouped_mm_swiglu launch")
     return out
 
@@ -255,7 +255,7 @@ def _activation_now(h: torch.Tensor, kind: str = "swiglu", out: torch.Tensor | N
     with _guard(h):
         rc = lib.gmm_moe_activation(h.data_ptr(), out.data_ptr(), h.size(0), inner, h.stride(0) if h.size(0) else inner,
                                     out.stride(0) if h.size(0) else inner, code, _dtype_code(h.dtype),
-                                    torch.cuda.current_stream().cuda_stream)
+                                    kernels.current_stream(h.device))
     _lib.check(rc, "moe_activation")
     return out
 
@@ -299,7 +299,7 @@ def _combine_now(y: torch.Tensor, token_rows: torch.Tensor, slot_weight: torch.T
     with _guard(y):
         rc = lib.gmm_moe_combine(y.data_ptr(), token_rows.data_ptr(), slot_weight.data_ptr(), out.data_ptr(),
                                  tokens, top_k, H, y.size(0), y.stride(0) if y.size(0) else H, out.stride(0) if tokens else H,
-                                 _dtype_code(y.dtype), torch.cuda.current_stream().cuda_stream)
+                                 _dtype_code(y.dtype), kernels.current_stream(y.device))
     _lib.check(rc, "moe_combine")
     return out
 
