@@ -478,14 +478,18 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
 
   // Locating a tile (binary search over the groups, reads of offs, integer divisions) costs microseconds, so
   // BATCH threads locate the next BATCH round-robin tiles of the workgroup at once and leave them in LDS for
-  // the tile loop to pick up.  From the queue one thread locates one tile at a time (two LDS reads and a division),
-  // with a ticket that it drew before the previous tile ran.
+  // the tile loop to pick up.  Tiles that are drawn from the queue are located by one thread, one at a time (two LDS
+  // reads and a division), with a ticket that it drew before the previous tile ran.
   for (int first = 0;; first += BATCH) {
     const int64_t mine = int64_t(blockIdx.x) + int64_t(first + tid) * gridDim.x;
     if constexpr (QUEUE) {
-      if (tid == 0) {
-        split_flag = q.next >= 0 ? 1 : 0;
-        if (q.next >= 0) gmm_store_rec(&tiles[0], q.locate(p, cum_tall, cum_short, GMM_TILE_N), -1);
+      if (q.drawn) {
+        if (tid == 0) {
+          split_flag = q.next >= 0 ? 1 : 0;
+          if (q.next >= 0) gmm_store_rec(&tiles[0], q.locate(p, q.next, cum_tall, cum_short, GMM_TILE_N), -1);
+        }
+      } else if (tid < BATCH && first + tid < q.dealt()) {
+        gmm_store_rec(&tiles[tid], q.locate(p, q.tile_number(first + tid), cum_tall, cum_short, GMM_TILE_N), -1);
       }
     } else if (tid < BATCH && mine < split_base) {
       const int t = int(mine);
@@ -493,15 +497,16 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
       gmm_store_rec(&tiles[tid], gmm_locate_tile2(p, cum_tall, cum_short, total_tall, tt, GMM_TILE_N), -1);
     }
     __syncthreads();
-    const int64_t left = (int64_t(split_base) - blockIdx.x + gridDim.x - 1) / gridDim.x - first;  // tiles of this workgroup from `first` on
-    const int here = QUEUE ? split_flag : left < BATCH ? int(left) : BATCH;
+    // tiles of this workgroup from `first` on
+    const int64_t left = QUEUE ? int64_t(q.dealt()) - first : (int64_t(split_base) - blockIdx.x + gridDim.x - 1) / gridDim.x - first;
+    const int here = QUEUE && q.drawn ? split_flag : left < BATCH ? int(left) : BATCH;
     for (int j = 0; j < here; ++j) {
       // Everything the assembly wants per lane is a cheap function of the lane id.  Hidden from the
       // optimiser per tile, or it hoists those values out of the loop, keeps them alive across the
       // assembly (which clobbers most registers) and spills them to scratch memory.
       int lane_j = lane;
       asm volatile("" : "+v"(lane_j));
-      if (QUEUE && tid == 0) q.draw(p);
+      if (QUEUE && q.drawn && tid == 0) q.draw(p);
       const GmmTileScalars t = gmm_load_rec(&tiles[j]);
       const GmmTileDesc dsc = gmm_describe_tile<A_TR, B_TR, ESZ, CDIV>(p, t);
       if constexpr (A_TR) {
@@ -516,11 +521,11 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
         else gmm_tile_compute<A_TR, B_TR, OUT_F32, 1, F16, 1, ACT>(dsc, lds_base, lane_j, wave);
       }
     }
-    if (QUEUE ? here == 0 : left <= BATCH) break;
+    if (QUEUE && q.drawn ? here == 0 : left <= BATCH) break;
     __syncthreads();  // everyone is done with this batch of located tiles
-    if (QUEUE && tid == 0) q.advance(p);
+    if (QUEUE && q.drawn && tid == 0) q.advance(p);
   }
-  if (QUEUE && tid == 0) q.leave(p);
+  if (QUEUE && q.drawn && tid == 0) q.leave(p);
 
   // The parts of the tiles that were cut: drawn from the ticket counter, one at a time, located by the thread
   // that draws.  Each part's whole fp32 tile goes to its workspace slot; gmm_split_finish does the rest.

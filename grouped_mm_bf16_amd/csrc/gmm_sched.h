@@ -224,8 +224,8 @@ GMM_HD int gmm_group_tile_cols(int jag, int lo, int hi, int N, int align, int bn
   return hi > lo ? gmm_cdiv(hi - (lo / align) * align, bn) : 0;
 }
 
-// Does a launch with a jagged contraction hand out its tiles longest group first, on demand (GmmKQueue), or deal them
-// round by round in group order?  A group with at least as many tiles as the launch has workgroups gives every one of
+// Does a launch with a jagged contraction hand out its tiles longest group first (GmmKQueue, which also decides whether
+// on demand), or deal them round by round in group order?  A group with at least as many tiles as the launch has workgroups gives every one of
 // them the same share, and workgroups that run in step share operand panels: dealt, 8 groups of 896 tiles (4096 x
 // 14336, 16384 rows, fp32 result) take 1682 us, from the queue 1698.  Smaller groups make uneven shares: 128 skewed
 // groups of 24 tiles (2048 x 768, 32768 rows) take 258 us dealt, 211 from the queue.
