@@ -598,16 +598,13 @@ bool small_tiles(const GmmParams& p, int in_dtype, int num_cus) {
 //   tiles: 64 groups of 32 x 64 with 2048 elements each 46 / 13; 24 groups of 328 x 360, 95496 elements 201 / 98; two groups
 //   of 328 x 712, 40424 elements 652 / 62; past 384 the larger tile catches up (496 tiles of 184 x 464 in 62 even groups
 //   70 / 78), but for very short groups (1230 tiles of 104 x 1248 in 123 groups, 16464 elements 69 / 52).  A contiguous along
-//   K: its 16-byte loads start at any element here, which costs more than it gains unless the contraction is long and
-//   the tiles are few (28 tiles of 112 x 888 in 4 groups, 44536 elements 415 / 65; 80 tiles of 200 x 968 in 5 groups, 2960
-//   elements 19 / 26) or the groups are a K tile at most.
+//   K stays with the assembly tile, never cut: its 16-byte loads start at any element here (80 tiles of 200 x 968 in 5
+//   groups, 2960 elements 19 / 26), and the bits of such a product do not depend on there being a workspace.
 bool gmm_staged_preferred(const GmmParams& p, int num_cus) {
   if (p.act || !gmm_staged_eligible(p)) return false;
   const int64_t tiles = most_tiles(p, 128), nk = (p.K + 63) / 64, cus = num_cus;
   if (p.jag == GMM_JAG_K) {
-    const bool short_groups = p.K <= 64 * int64_t(p.G);
-    if (p.a_sk != 1) return 2 * tiles <= 3 * cus || (short_groups && tiles <= 4 * cus);
-    return (2 * tiles <= cus && p.K >= 1024 * int64_t(p.G)) || (tiles <= cus && short_groups);
+    return p.a_sk != 1 && (2 * tiles <= 3 * cus || (p.K <= 64 * int64_t(p.G) && tiles <= 4 * cus));
   }
   if (p.a_sk != 1 && tiles <= tile_wgs(128) * cus && nk <= 32) return true;
   const bool rows_fill = p.jag == GMM_JAG_M ? p.M >= 64 * int64_t(p.G) : p.M >= 64;
