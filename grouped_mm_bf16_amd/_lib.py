@@ -18,6 +18,8 @@ ABI_VERSION = 3
 PATH_AUTO, PATH_GENERIC, PATH_MFMA = 0, 1, 2
 DT_BF16, DT_F16, DT_F32 = 0, 1, 2
 OK = 0
+ERR_WORKSPACE = 4
+WORKSPACE_EAGER_ONLY = 1 << 62
 
 _i32, _i64, _vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p
 
@@ -26,6 +28,7 @@ SIGNATURES = {
     "gmm_abi_version": (ctypes.c_int, []),
     "gmm_status_string": (ctypes.c_char_p, [ctypes.c_int]),
     "gmm_workspace_bytes": (_i64, []),
+    "gmm_stream_capture": (_i64, [_vp]),
     "gmm_2d3d": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i32] + [_i64] * 3 + [_i64] * 7 + [_i32, _i32, _vp, _i64, _vp]),
     "gmm_2d3d_gather": (ctypes.c_int, [_vp] * 5 + [_i32] + [_i64] * 4 + [_i64] * 7 + [_i32, _i32, _vp, _i64, _vp]),
     "gmm_2d3d_swiglu": (ctypes.c_int, [_vp] * 5 + [_i32] + [_i64] * 4 + [_i64] * 7 + [_i32, _vp]),

@@ -44,13 +44,20 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 struct Problem {
   GmmParams p;
   int in_dtype, out_dtype;
+  bool eager_only;   // GMM_WORKSPACE_EAGER_ONLY
 };
 
 // Caller's workspace -> split parameters: the header must fit, the slots must be 16-byte aligned.
-void set_workspace(GmmParams& p, void* ws, int64_t bytes) {
+void set_workspace(Problem& pr, void* ws, int64_t bytes) {
+  GmmParams& p = pr.p;
   p.ws = nullptr;
   p.ws_parts = 0;
+  pr.eager_only = false;
   if (!g_tail_split.load(std::memory_order_relaxed)) return;
+  if (bytes >= GMM_WORKSPACE_EAGER_ONLY) {
+    pr.eager_only = true;
+    bytes -= GMM_WORKSPACE_EAGER_ONLY;
+  }
   if (!ws || !aligned16(ws) || bytes < GMM_WS_HEADER + 2 * int64_t(GMM_WS_SLOT)) return;
   const int64_t parts = (bytes - GMM_WS_HEADER) / GMM_WS_SLOT;
   p.ws = ws;
@@ -97,6 +104,24 @@ bool asm_tile_eligible(const Problem& pr, const GmmLayout& lay) {
     if (ldc >= ld_max / 2) return false;   // 255 rows of 4-byte elements must stay below 2^31 bytes from the tile's origin
   }
   return true;
+}
+
+// Id of the capture that `stream` takes part in, 0 if it takes part in none.
+uint64_t capture_id(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {
+    (void)hipGetLastError();   // the default stream while another stream captures: no capture of its own
+    return 0;
+  }
+  return status == hipStreamCaptureStatusActive ? uint64_t(id) : 0;
+}
+
+// Every workspace that a launch could use: what gmm_workspace_bytes has room for.
+GmmParams with_full_workspace(const GmmParams& p, int cus) {
+  GmmParams q = p;
+  q.ws_parts = 2 * cus;
+  return q;
 }
 
 int run(Problem& pr, hipStream_t stream) {
@@ -164,12 +189,20 @@ int run(Problem& pr, hipStream_t stream) {
       p.group_major = fo >= 0 ? fo : (p.tall == 128 ? 1 : 0);
     }
     // small products of the automatic choice run on 128 x 128 tiles of the register-staged kernel
-    rc = automatic && cfg == GMM_CFG_ASM_256x256 && gmm_staged_preferred(p, cus)
-             ? gmm_launch_staged(p, pr.in_dtype, pr.out_dtype, cus, stream)
-             : gmm_launch_mfma(p, lay, pr.in_dtype, pr.out_dtype, cfg, cus, stream);
+    const bool staged = automatic && cfg == GMM_CFG_ASM_256x256 && gmm_staged_preferred(p, cus);
+    if (pr.eager_only) {
+      const GmmParams q = with_full_workspace(p, cus);
+      if ((staged ? gmm_staged_uses_workspace(q, pr.in_dtype, cus) : gmm_mfma_uses_workspace(q, lay, cfg, cus)) && capture_id(stream))
+        return GMM_ERR_WORKSPACE;
+    }
+    rc = staged ? gmm_launch_staged(p, pr.in_dtype, pr.out_dtype, cus, stream)
+                : gmm_launch_mfma(p, lay, pr.in_dtype, pr.out_dtype, cfg, cus, stream);
     t_last_path = GMM_PATH_MFMA;
     t_last_config = cfg;
   } else {
+    if (pr.eager_only && gmm_staged_eligible(p) && gmm_staged_uses_workspace(with_full_workspace(p, cus), pr.in_dtype, cus) &&
+        capture_id(stream))
+      return GMM_ERR_WORKSPACE;
     rc = gmm_launch_generic(p, pr.in_dtype, pr.out_dtype, cus, stream);
     t_last_path = GMM_PATH_GENERIC;
     t_last_config = -1;
@@ -191,13 +224,15 @@ int64_t gmm_workspace_bytes(void) {
   return cus > 0 ? GMM_WS_HEADER + 2 * int64_t(cus) * GMM_WS_SLOT : 0;
 }
 
+int64_t gmm_stream_capture(void* stream) { return int64_t(capture_id(static_cast<hipStream_t>(stream))); }
+
 const char* gmm_status_string(int status) {
   switch (status) {
     case GMM_OK: return "ok";
     case GMM_ERR_BAD_ARGUMENT: return "bad argument (null pointer, size out of range or more than 1023 groups)";
     case GMM_ERR_UNSUPPORTED: return "unsupported dtype combination or forced kernel family not applicable";
     case GMM_ERR_LAUNCH: return "HIP launch failed";
-    case GMM_ERR_WORKSPACE: return "workspace too small for this problem";
+    case GMM_ERR_WORKSPACE: return "workspace too small for this problem, or shared and the stream is being captured";
     default: return "unknown status";
   }
 }
@@ -212,7 +247,7 @@ int gmm_2d3d(const void* a, const void* b, void* out, const int32_t* offs, int32
                    0, a_sm, a_sk, b_sg, b_sk, b_sn, 0, o_sm, o_sn, 0, 0};
   pr.in_dtype = in_dtype;
   pr.out_dtype = out_dtype;
-  set_workspace(pr.p, workspace, workspace_bytes);
+  set_workspace(pr, workspace, workspace_bytes);
   return run(pr, static_cast<hipStream_t>(stream));
 }
 
@@ -229,7 +264,7 @@ int gmm_2d3d_gather(const void* a, const int32_t* row_index, const void* b, void
   pr.p.a_rows = int32_t(a_rows);
   pr.in_dtype = in_dtype;
   pr.out_dtype = out_dtype;
-  set_workspace(pr.p, workspace, workspace_bytes);
+  set_workspace(pr, workspace, workspace_bytes);
   return run(pr, static_cast<hipStream_t>(stream));
 }
 
@@ -259,7 +294,7 @@ int gmm_3d3d(const void* a, const void* b, void* out, int32_t G, int64_t M, int6
                    a_sg, a_sm, a_sk, b_sg, b_sk, b_sn, o_sg, o_sm, o_sn, 0, 0};
   pr.in_dtype = in_dtype;
   pr.out_dtype = out_dtype;
-  set_workspace(pr.p, workspace, workspace_bytes);
+  set_workspace(pr, workspace, workspace_bytes);
   // the tile count G * tiles must fit an int32
   if (G > 0 && M > 0 && N > 0) {
     const int64_t tiles = int64_t(G) * ((M + 63) / 64) * ((N + 63) / 64);
@@ -278,7 +313,7 @@ int gmm_2d2d(const void* a, const void* b, void* out, const int32_t* offs, int32
                    0, a_sm, a_sk, 0, b_sk, b_sn, o_sg, o_sm, o_sn, 0, 0};
   pr.in_dtype = in_dtype;
   pr.out_dtype = out_dtype;
-  set_workspace(pr.p, workspace, workspace_bytes);
+  set_workspace(pr, workspace, workspace_bytes);
   return run(pr, static_cast<hipStream_t>(stream));
 }
 
@@ -292,7 +327,7 @@ int gmm_3d2d(const void* a, const void* b, void* out, const int32_t* offs, int32
                    a_sg, a_sm, a_sk, 0, b_sk, b_sn, 0, o_sm, o_sn, 0, 0};
   pr.in_dtype = in_dtype;
   pr.out_dtype = out_dtype;
-  set_workspace(pr.p, workspace, workspace_bytes);
+  set_workspace(pr, workspace, workspace_bytes);
   return run(pr, static_cast<hipStream_t>(stream));
 }
 

@@ -13,6 +13,8 @@ bool gmm_staged_eligible(const GmmParams& p);
 // Of the 16-bit products that the assembly tile could take: true for those that the register-staged kernel runs faster.
 bool gmm_staged_preferred(const GmmParams& p, int num_cus);
 int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream);
+// Would this launch use a workspace of p.ws_parts slots?
+bool gmm_staged_uses_workspace(const GmmParams& p, int in_dtype, int num_cus);
 
 // Operand layout facts the host derived from strides.
 struct GmmLayout {
@@ -28,3 +30,4 @@ enum GmmMfmaConfig : int { GMM_CFG_REG_256x256 = 0, GMM_CFG_ASM_256x256 = 1, GMM
 
 // bf16 inputs only; out_dtype bf16 or fp32.  Returns like gmm_launch_generic.
 int gmm_launch_mfma(GmmParams p, GmmLayout lay, int in_dtype, int out_dtype, int config, int num_cus, hipStream_t stream);
+bool gmm_mfma_uses_workspace(GmmParams p, GmmLayout lay, int config, int num_cus);

@@ -628,28 +628,38 @@ int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
   return gmm_use_k_queue(p, GMM_TILE_N, p.num_wg) ? launch_asm<OUT_F32, F16, 1>(p, lay, stream) : launch_asm<OUT_F32, F16, 0>(p, lay, stream);
 }
 
-}  // namespace
-
-int gmm_launch_mfma(GmmParams p, GmmLayout lay, int in_dtype, int out_dtype, int config, int num_cus, hipStream_t stream) {
+// Grid, tile heights and use of the workspace of a launch.
+void plan(GmmParams& p, GmmLayout lay, int config, int num_cus) {
   // persistent grid: one workgroup per CU, fewer (a multiple of 8, for the XCD renumbering) when the launch
   // cannot have that many tiles
-  {
-    const int64_t bound = gmm_tile_bound(p.jag, p.G, p.M, p.N, config == GMM_CFG_ASM_256x256 ? p.tall : 256, 256);
-    const int64_t want = ((bound + 7) / 8) * 8;
-    p.num_wg = int(want < num_cus ? (want < 8 ? 8 : want) : num_cus);
-    // the tiles of a partly filled last round can be cut along K (gmm_tail_split); a launch of few tiles with a
-    // long contraction gets the whole chip for that
-    const bool can_split = config == GMM_CFG_ASM_256x256 && p.ws_parts > 0 && !p.act && p.jag != GMM_JAG_K &&
-                           p.K >= 2 * GMM_SPLIT_PART_MIN * GMM_TILE_K;
-    if (can_split && p.K >= 96 * GMM_TILE_K) p.num_wg = num_cus;
-    if (!can_split) p.ws_parts = 0;
-  }
-  const bool out16 = out_dtype == in_dtype;   // else fp32
-  if (!out16 && out_dtype != GMM_DT_F32) return -1;
+  const int64_t bound = gmm_tile_bound(p.jag, p.G, p.M, p.N, config == GMM_CFG_ASM_256x256 ? p.tall : 256, 256);
+  const int64_t want = ((bound + 7) / 8) * 8;
+  p.num_wg = int(want < num_cus ? (want < 8 ? 8 : want) : num_cus);
+  // the tiles of a partly filled last round can be cut along K (gmm_tail_split); a launch of few tiles with a
+  // long contraction gets the whole chip for that
+  const bool can_split = config == GMM_CFG_ASM_256x256 && p.ws_parts > 0 && !p.act && p.jag != GMM_JAG_K &&
+                         p.K >= 2 * GMM_SPLIT_PART_MIN * GMM_TILE_K;
+  if (can_split && p.K >= 96 * GMM_TILE_K) p.num_wg = num_cus;
+  if (!can_split) p.ws_parts = 0;
   if (config == GMM_CFG_ASM_256x256) {
     // a column-major A has only the 256-row tile
     if (!lay.a_kc) { p.tall = 256; p.shrt = 0; }
     if (p.tall != 128) p.tall = 256;
+  }
+}
+
+}  // namespace
+
+bool gmm_mfma_uses_workspace(GmmParams p, GmmLayout lay, int config, int num_cus) {
+  plan(p, lay, config, num_cus);
+  return p.ws_parts > 0 || (config == GMM_CFG_ASM_256x256 && gmm_use_k_queue(p, GMM_TILE_N, p.num_wg));
+}
+
+int gmm_launch_mfma(GmmParams p, GmmLayout lay, int in_dtype, int out_dtype, int config, int num_cus, hipStream_t stream) {
+  plan(p, lay, config, num_cus);
+  const bool out16 = out_dtype == in_dtype;   // else fp32
+  if (!out16 && out_dtype != GMM_DT_F32) return -1;
+  if (config == GMM_CFG_ASM_256x256) {
     if (in_dtype == GMM_DT_BF16) return out16 ? launch_asm<0, 0>(p, lay, stream) : launch_asm<1, 0>(p, lay, stream);
     if (in_dtype == GMM_DT_F16) return out16 ? launch_asm<0, 1>(p, lay, stream) : launch_asm<1, 1>(p, lay, stream);
     return -1;

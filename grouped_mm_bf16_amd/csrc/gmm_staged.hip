@@ -625,6 +625,12 @@ bool gmm_staged_eligible(const GmmParams& p) {
   return lda >= 1 && ldb >= 1 && p.K >= 1 && rows >= 1 && a_len >= 8 && b_len >= 8;
 }
 
+bool gmm_staged_uses_workspace(const GmmParams& p, int in_dtype, int num_cus) {
+  GmmParams cut = p;
+  return (small_tiles(p, in_dtype, num_cus) ? cut_contraction<64>(cut, int64_t(tile_wgs(64)) * num_cus)
+                                            : cut_contraction<128>(cut, int64_t(tile_wgs(128)) * num_cus)) > 0;
+}
+
 int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream) {
   p.align = 1;
   const bool a_tr = p.a_sk != 1, b_tr = p.b_sk != 1;

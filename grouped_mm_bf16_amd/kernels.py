@@ -45,25 +45,61 @@ def current_stream(device: torch.device) -> int:
 
 # One workspace per (device, stream): launches on one stream run one after the other, so they can share it;
 # launches on different streams may overlap and must not.  Allocated on first use and kept (the library leaves
-# the arrival counters at its head zero after every launch).
+# the arrival counters at its head zero after every launch).  For eager launches only: a captured launch runs on
+# whatever stream its graph is replayed on, beside anything else.
 _workspaces: dict = {}
+
+# Last capture seen: its id, and whether torch gives allocations made inside it to the graph.
+_capture = (0, False)
 
 
 def workspace(device: torch.device, stream: int):
-    """(pointer, bytes) of the split workspace for launches on `stream` of `device`, or (None, 0) when none
-    can be had: inside a stream capture no new workspace is allocated (a captured allocation would belong to
-    the graph's memory pool), so a stream first used under capture launches without one."""
+    """(pointer, bytes) of the workspace for eager launches on `stream` of `device`, or (None, 0) when none can be
+    had."""
     key = (device.index, stream)
     ws = _workspaces.get(key)
     if ws is None:
-        if torch.cuda.is_current_stream_capturing():
-            return None, 0
         nbytes = _lib.load().gmm_workspace_bytes()
-        if nbytes <= 0:
+        if nbytes <= 0 or torch.cuda.is_current_stream_capturing():
             return None, 0
         ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
         _workspaces[key] = ws
     return ws.data_ptr(), ws.numel()
+
+
+def _captured_workspace(device: torch.device, stream: int) -> Optional[torch.Tensor]:
+    """A workspace for one launch inside a capture: allocated and cleared there, so that it belongs to the graph's memory
+    pool, which nothing but the graph uses (later allocations of the capture may share the memory: they follow on the
+    same stream).  None in a capture that torch does not know of: memory allocated there would go back to the common
+    pool."""
+    global _capture
+    lib = _lib.load()
+    capture = lib.gmm_stream_capture(stream)
+    known, owned = _capture
+    if capture != known:
+        # torch's ordinary allocations lie in pool (0, 0)
+        probe = torch.empty(1, device=device).data_ptr()
+        owned = any(s["address"] <= probe < s["address"] + s["total_size"] and tuple(s["segment_pool_id"]) != (0, 0)
+                    for s in torch.cuda.memory_snapshot() if s["device"] == device.index)
+        _capture = capture, owned
+    if not owned:
+        return None
+    ws = torch.empty(lib.gmm_workspace_bytes(), dtype=torch.uint8, device=device)
+    ws[:4096].zero_()
+    return ws
+
+
+def call_with_workspace(launcher, args: tuple, device: torch.device, stream: int) -> int:
+    """``launcher(*args, workspace, workspace_bytes, stream)`` with the stream's workspace, or with one of its own inside a
+    capture if the launch has a use for it; returns the status."""
+    ws, nbytes = workspace(device, stream)
+    rc = launcher(*args, ws, nbytes | _lib.WORKSPACE_EAGER_ONLY, stream)
+    if rc != _lib.ERR_WORKSPACE:
+        return rc
+    own = _captured_workspace(device, stream)
+    if own is None:
+        return launcher(*args, None, 0, stream)
+    return launcher(*args, own.data_ptr(), own.numel(), stream)
 
 
 def _launch_now(variant: int, a: torch.Tensor, b: torch.Tensor, offs: Optional[torch.Tensor],
@@ -77,25 +113,29 @@ def _launch_now(variant: int, a: torch.Tensor, b: torch.Tensor, offs: Optional[t
         stream = current_stream(a.device)
         pa, pb, po = a.data_ptr(), b.data_ptr(), out.data_ptr()
         poffs = offs.data_ptr() if offs is not None else None
-        ws, ws_bytes = workspace(a.device, stream)
         if variant == V_2D3D:
-            rc = lib.gmm_2d3d(pa, pb, po, poffs, offs.numel(), a.size(0), b.size(2), a.size(1),
-                              a.stride(0), a.stride(1), b.stride(0), b.stride(1), b.stride(2),
-                              out.stride(0), out.stride(1), in_dt, out_dt, ws, ws_bytes, stream)
+            launcher = lib.gmm_2d3d
+            args = (pa, pb, po, poffs, offs.numel(), a.size(0), b.size(2), a.size(1),
+                    a.stride(0), a.stride(1), b.stride(0), b.stride(1), b.stride(2),
+                    out.stride(0), out.stride(1), in_dt, out_dt)
         elif variant == V_3D3D:
-            rc = lib.gmm_3d3d(pa, pb, po, a.size(0), a.size(1), b.size(2), a.size(2),
-                              a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1), b.stride(2),
-                              out.stride(0), out.stride(1), out.stride(2), in_dt, out_dt, ws, ws_bytes, stream)
+            launcher = lib.gmm_3d3d
+            args = (pa, pb, po, a.size(0), a.size(1), b.size(2), a.size(2),
+                    a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1), b.stride(2),
+                    out.stride(0), out.stride(1), out.stride(2), in_dt, out_dt)
         elif variant == V_2D2D:
-            rc = lib.gmm_2d2d(pa, pb, po, poffs, offs.numel(), a.size(0), b.size(1), a.size(1),
-                              a.stride(0), a.stride(1), b.stride(0), b.stride(1),
-                              out.stride(0), out.stride(1), out.stride(2), in_dt, out_dt, ws, ws_bytes, stream)
+            launcher = lib.gmm_2d2d
+            args = (pa, pb, po, poffs, offs.numel(), a.size(0), b.size(1), a.size(1),
+                    a.stride(0), a.stride(1), b.stride(0), b.stride(1),
+                    out.stride(0), out.stride(1), out.stride(2), in_dt, out_dt)
         elif variant == V_3D2D:
-            rc = lib.gmm_3d2d(pa, pb, po, poffs, offs.numel(), a.size(1), b.size(1), a.size(2),
-                              a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1),
-                              out.stride(0), out.stride(1), in_dt, out_dt, ws, ws_bytes, stream)
+            launcher = lib.gmm_3d2d
+            args = (pa, pb, po, poffs, offs.numel(), a.size(1), b.size(1), a.size(2),
+                    a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1),
+                    out.stride(0), out.stride(1), in_dt, out_dt)
         else:
             raise RuntimeError(f"unknown variant {variant}")
+        rc = call_with_workspace(launcher, args, a.device, stream)
     _lib.check(rc, "grouped_mm launch")
 
 

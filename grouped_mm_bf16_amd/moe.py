@@ -144,11 +144,11 @@ def _gathered_now(a: torch.Tensor, row_index: torch.Tensor, b: torch.Tensor, off
     lib = _lib.load()
     with _guard(a):
         stream = kernels.current_stream(a.device)
-        ws, ws_bytes = kernels.workspace(a.device, stream)
-        rc = lib.gmm_2d3d_gather(a.data_ptr(), row_index.data_ptr(), b.data_ptr(), out.data_ptr(), offs.data_ptr(),
-                                 offs.numel(), a.size(0), M, N, a.size(1), a.stride(0), a.stride(1),
-                                 b.stride(0), b.stride(1), b.stride(2), out.stride(0), out.stride(1),
-                                 _dtype_code(a.dtype), _dtype_code(out.dtype), ws, ws_bytes, stream)
+        args = (a.data_ptr(), row_index.data_ptr(), b.data_ptr(), out.data_ptr(), offs.data_ptr(),
+                offs.numel(), a.size(0), M, N, a.size(1), a.stride(0), a.stride(1),
+                b.stride(0), b.stride(1), b.stride(2), out.stride(0), out.stride(1),
+                _dtype_code(a.dtype), _dtype_code(out.dtype))
+        rc = kernels.call_with_workspace(lib.gmm_2d3d_gather, args, a.device, stream)
     _lib.check(rc, "grouped_mm_gathered launch")
     return out
 

@@ -38,7 +38,8 @@ enum gmm_status {
   GMM_ERR_BAD_ARGUMENT = 1, /* null pointer, negative size, G out of range, bad stride */
   GMM_ERR_UNSUPPORTED = 2,  /* dtype combination or forced path not available */
   GMM_ERR_LAUNCH = 3,       /* the HIP runtime refused the launch */
-  GMM_ERR_WORKSPACE = 4     /* the workspace passed in is smaller than the problem needs */
+  GMM_ERR_WORKSPACE = 4     /* the workspace passed in is smaller than the problem needs, or shared (see
+                               GMM_WORKSPACE_EAGER_ONLY) */
 };
 
 enum gmm_dtype { GMM_DT_BF16 = 0, GMM_DT_F16 = 1, GMM_DT_F32 = 2 };
@@ -61,10 +62,21 @@ const char* gmm_status_string(int status);
  * limits the split, less than 4096 + 2 * 262144 bytes (or NULL) turns it off.  Rules for the caller:
  *   - 16-byte aligned; the first 4096 bytes zero before the first launch that uses it (the kernels leave
  *     them zero, so one hipMemset after allocation is enough); the rest need not be initialised;
- *   - launches that may run at the same time (different streams) need different workspaces.
+ *   - launches that may run at the same time (different streams) need different workspaces.  A captured launch
+ *     runs whenever and wherever its graph is replayed, so a graph needs a workspace that nothing outside it
+ *     uses, with the first 4096 bytes cleared by the graph itself or before its first replay.
+ *
+ * GMM_WORKSPACE_EAGER_ONLY, added to `workspace_bytes`, says that the workspace (or NULL) belongs to eager launches:
+ * on a stream that is being captured, a launch for which a workspace is of use then launches nothing and returns
+ * GMM_ERR_WORKSPACE, and the caller comes back with one that belongs to the graph (or with NULL, 0); every other launch
+ * runs as without it.
  * The reference has no counterpart (its launches create one program per tile, reference
  * kernels.py:636-659, and leave the balancing to the hardware dispatcher). */
 int64_t gmm_workspace_bytes(void);
+#define GMM_WORKSPACE_EAGER_ONLY (INT64_C(1) << 62)
+
+/* Id of the stream capture that `stream` takes part in, 0 if none.  Ids are unique in the process. */
+int64_t gmm_stream_capture(void* stream);
 
 /* 2D x 3D: out[s_g:e_g, :] = a[s_g:e_g, :] @ b[g]   (rows jagged)
  * a [M_total, K], b [G, K, N], out [M_total, N].
