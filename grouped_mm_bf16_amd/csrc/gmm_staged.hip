@@ -414,7 +414,7 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
     if (klen > 0) {
       Stage<T, A_TR, BM> sa;
       Stage<T, B_TR, BN> sb;
-      sa.init(a, lda, tile.m0, p.M, tile.k_lo, tile.k_hi, p.K, p.gather ? &p : nullptr, tile.m_hi);
+      sa.init(a, lda, tile.m0, p.M, tile.k_lo, tile.k_hi, p.K, SPLIT || !p.gather ? nullptr : &p, tile.m_hi);
       sb.init(b, ldb, tile.n0, p.N, tile.k_lo, tile.k_hi, p.K, nullptr, 0);
       const int n_fast = gmm_min(sa.n_fast, sb.n_fast), nk = (klen + BK - 1) / BK;
       // K tile t + 1 .. t + AHEAD are on their way in registers while K tile t is multiplied
