@@ -42,6 +42,7 @@ SIGNATURES = {
     "gmm_moe_combine": (ctypes.c_int, [_vp] * 4 + [_i64] * 6 + [_i32, _vp]),
     "gmm_set_path": (ctypes.c_int, [ctypes.c_int]),
     "gmm_last_path": (ctypes.c_int, []),
+    "gmm_last_kernel": (ctypes.c_int, []),
     "gmm_set_mfma_config": (ctypes.c_int, [ctypes.c_int]),
     "gmm_last_mfma_config": (ctypes.c_int, []),
     "gmm_set_xcd_remap": (ctypes.c_int, [ctypes.c_int]),

@@ -20,6 +20,7 @@ std::atomic<int> g_group_major{-1};   // -1 auto, 0 tall tiles of all groups fir
 std::atomic<int> g_tail_split{1};     // 0: ignore the workspace (no tile is cut along K)
 thread_local int t_last_path = 0;
 thread_local int t_last_config = -1;
+thread_local int t_last_kernel = GMM_KERNEL_NONE;
 
 constexpr int kMaxDevices = 64;
 std::atomic<int> g_num_cus[kMaxDevices];
@@ -162,7 +163,7 @@ int run(Problem& pr, hipStream_t stream) {
     p.xcd_remap = g_xcd_remap.load(std::memory_order_relaxed);
     int cfg = g_forced_config.load(std::memory_order_relaxed);
     if (cfg == GMM_CFG_ASM_256x256 && !can_asm) return GMM_ERR_UNSUPPORTED;
-    const bool automatic = forced == GMM_PATH_AUTO && (cfg < 0 || cfg >= GMM_CFG_COUNT);
+    bool automatic = forced == GMM_PATH_AUTO && (cfg < 0 || cfg >= GMM_CFG_COUNT) && p.xcd_remap;
     if (cfg < 0 || cfg >= GMM_CFG_COUNT) cfg = can_asm ? GMM_CFG_ASM_256x256 : GMM_CFG_REG_256x256;
     if ((p.gather || p.act) && cfg != GMM_CFG_ASM_256x256) return GMM_ERR_UNSUPPORTED;
     if (pr.in_dtype != GMM_DT_BF16 && cfg != GMM_CFG_ASM_256x256) return GMM_ERR_UNSUPPORTED;
@@ -180,6 +181,7 @@ int run(Problem& pr, hipStream_t stream) {
       const int ft = g_forced_tall.load(std::memory_order_relaxed), fs = g_forced_short.load(std::memory_order_relaxed);
       if (lay.a_kc && (ft == 256 || ft == 128)) p.tall = ft;
       if (lay.a_kc && (fs == 0 || fs == 64)) p.shrt = fs;
+      automatic = automatic && ft < 0 && fs < 0;
     }
     // Launch order: group by group in the fine-grained regime (many small groups: a group's remainder tile
     // then reads the second operand while its tall tiles have it in the caches; +4 % there), otherwise all
@@ -187,8 +189,9 @@ int run(Problem& pr, hipStream_t stream) {
     {
       const int fo = g_group_major.load(std::memory_order_relaxed);
       p.group_major = fo >= 0 ? fo : (p.tall == 128 ? 1 : 0);
+      automatic = automatic && fo < 0;
     }
-    // small products of the automatic choice run on 128 x 128 tiles of the register-staged kernel
+    // small products run on 128 x 128 tiles of the register-staged kernel, unless something of the assembly tile is forced
     const bool staged = automatic && cfg == GMM_CFG_ASM_256x256 && gmm_staged_preferred(p, cus);
     if (pr.eager_only) {
       const GmmParams q = with_full_workspace(p, cus);
@@ -199,11 +202,12 @@ int run(Problem& pr, hipStream_t stream) {
                 : gmm_launch_mfma(p, lay, pr.in_dtype, pr.out_dtype, cfg, cus, stream);
     t_last_path = GMM_PATH_MFMA;
     t_last_config = cfg;
+    t_last_kernel = staged ? GMM_KERNEL_ANY : cfg == GMM_CFG_ASM_256x256 ? GMM_KERNEL_ASSEMBLY : GMM_KERNEL_REGISTER;
   } else {
     if (pr.eager_only && gmm_staged_eligible(p) && gmm_staged_uses_workspace(with_full_workspace(p, cus), pr.in_dtype, cus) &&
         capture_id(stream))
       return GMM_ERR_WORKSPACE;
-    rc = gmm_launch_generic(p, pr.in_dtype, pr.out_dtype, cus, stream);
+    rc = gmm_launch_generic(p, pr.in_dtype, pr.out_dtype, cus, stream, t_last_kernel);
     t_last_path = GMM_PATH_GENERIC;
     t_last_config = -1;
   }
@@ -336,6 +340,7 @@ int gmm_set_path(int path) {
   return g_forced_path.exchange(path);
 }
 int gmm_last_path(void) { return t_last_path; }
+int gmm_last_kernel(void) { return t_last_kernel; }
 int gmm_set_mfma_config(int config) { return g_forced_config.exchange(config); }
 int gmm_last_mfma_config(void) { return t_last_config; }
 int gmm_set_xcd_remap(int on) { return g_xcd_remap.exchange(on ? 1 : 0); }

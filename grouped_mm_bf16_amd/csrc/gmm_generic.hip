@@ -216,12 +216,16 @@ int launch(const GmmParams& p, hipStream_t stream) {
 
 }  // namespace
 
-int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream) {
-  if (gmm_staged_eligible(p)) return gmm_launch_staged(p, in_dtype, out_dtype, num_cus, stream);
+int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream, int& kernel) {
+  if (gmm_staged_eligible(p)) {
+    kernel = GMM_KERNEL_ANY;
+    return gmm_launch_staged(p, in_dtype, out_dtype, num_cus, stream);
+  }
   p.align = 1;
   p.xcd_remap = 0;
   // at least one full 128 x 128 tile and a contraction worth pipelining: the matrix-core kernel
   const bool wide = p.M >= WT && p.N >= WT && p.K >= 64;
+  kernel = wide ? GMM_KERNEL_WIDE : GMM_KERNEL_ELEMENT;
   {
     const int edge = wide ? WT : GT;
     const int64_t bound = gmm_tile_bound(p.jag, p.G, p.M, p.N, edge, edge);

@@ -5,10 +5,11 @@
 #include "gmm_sched.h"
 
 // Each returns 0 on success, 1 if the launch failed, -1 if the dtype pair is unsupported.
-int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream);
+// `kernel`: the one that was launched (gmm_kernel).
+int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream, int& kernel);
 
 // Register-staged MFMA kernel for operands of any alignment (gmm_staged.hip): each operand contiguous along one of
-// its dimensions.  Returns like gmm_launch_generic.
+// its dimensions.  Returns like gmm_launch_generic, the kernel is GMM_KERNEL_ANY.
 bool gmm_staged_eligible(const GmmParams& p);
 // Of the 16-bit products that the assembly tile could take: true for those that the register-staged kernel runs faster.
 bool gmm_staged_preferred(const GmmParams& p, int num_cus);

@@ -241,3 +241,9 @@ def tail_split(on: bool):
 def last_path() -> str:
     """Kernel family used by this thread's last launch: "generic", "mfma" or "none"."""
     return {0: "none", _lib.PATH_GENERIC: "generic", _lib.PATH_MFMA: "mfma"}[_lib.load().gmm_last_path()]
+
+
+def last_kernel() -> str:
+    """Kernel of this thread's last launch: "none", "element", "wide", "any" (any alignment, staged through registers),
+    "register" or "assembly"."""
+    return ("none", "element", "wide", "any", "register", "assembly")[_lib.load().gmm_last_kernel()]

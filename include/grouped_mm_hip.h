@@ -220,10 +220,21 @@ int gmm_moe_combine(const void* y, const int32_t* token_rows, const float* slot_
  * takes that setting): they are for tests and tuning runs, not for serving code. */
 int gmm_set_path(int path);
 int gmm_last_path(void);
+/* The kernel that the calling thread's last launch used (a gmm_kernel; GMM_KERNEL_NONE before any launch). */
+enum gmm_kernel {
+  GMM_KERNEL_NONE = 0,
+  GMM_KERNEL_ELEMENT = 1,  /* any strides, element by element, fp32 products on the vector units */
+  GMM_KERNEL_WIDE = 2,     /* any strides, element by element, fp32 MFMA */
+  GMM_KERNEL_ANY = 3,      /* each operand contiguous along one dimension, any alignment, staged through registers */
+  GMM_KERNEL_REGISTER = 4, /* aligned bf16, staged through registers (MFMA configuration 0) */
+  GMM_KERNEL_ASSEMBLY = 5  /* assembly tile (MFMA configuration 1) */
+};
+int gmm_last_kernel(void);
 /* Tile configuration of the MFMA family: -1 = choose from the shapes, 0 = register-staged kernel,
- * 1 = assembly tile (256 / 128 / 64-row tiles).  Returns the previous setting.  With -1 and GMM_PATH_AUTO, calls that
- * the assembly tile could take but that are too small for it run on 128 x 128 tiles of the kernel for operands of any
- * alignment; gmm_last_mfma_config reports 1 for them as well. */
+ * 1 = assembly tile (256 / 128 / 64-row tiles).  Returns the previous setting.  With -1 and GMM_PATH_AUTO, and tile
+ * heights, launch order and renumbering (below) not forced either, calls that the assembly tile could take but that are too
+ * small for it run on 128 x 128 tiles of the kernel for operands of any alignment; gmm_last_mfma_config reports 1 for them
+ * as well, gmm_last_kernel GMM_KERNEL_ANY. */
 int gmm_set_mfma_config(int config);
 int gmm_last_mfma_config(void);
 /* 0 / 1: renumber tiles per XCD (default 1). */

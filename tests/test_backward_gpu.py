@@ -61,14 +61,17 @@ def make_case(variant, sizes, d1, d2, dtype, gen, scale_b=1.0, extra=0):
 
 
 class LaunchLog:
-    """Records (variant code, kernel family) of every launch inside the block."""
+    """Records (variant code, kernel family) of every launch inside the block, and the kernels."""
+    kernels: list = []                 # of the latest block
 
     def __enter__(self):
+        LaunchLog.kernels = []
         self.calls, self._orig = [], K_._launch_now
 
         def logged(variant, a, b, offs, out):
             self._orig(variant, a, b, offs, out)
             self.calls.append((variant, K_.last_path()))
+            LaunchLog.kernels.append(K_.last_kernel())
         K_._launch_now = logged
         return self
 
@@ -210,15 +213,19 @@ ALIGNED = {  # variant -> (sizes along the jagged dimension, d1, d2): every exte
 @pytest.mark.parametrize("layout", [(False, False), (True, False), (False, True), (True, True)])
 @pytest.mark.parametrize("variant", ["2d3d", "3d3d", "2d2d", "3d2d"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_backward_on_the_assembly_tile(variant, layout, dtype):
+@pytest.mark.parametrize("path", ["auto", "mfma"])
+def test_backward_on_the_assembly_tile(variant, layout, dtype, path):
     """bf16 / fp16 with aligned extents: the forward and both gradient launches take the MFMA family (the
-    gradients through transposed views, with jagged contractions starting at odd k)."""
+    gradients through transposed views, with jagged contractions starting at odd k), forced to the assembly tile or
+    on the kernels chosen for these sizes."""
     gen = torch.Generator().manual_seed(5)
     sizes, d1, d2 = ALIGNED[variant]
     extra = 0 if variant == "3d3d" else 8 - sum(sizes) % 8   # pad the jagged extent to a multiple of 8
     a, b, offs = make_case(variant, sizes, d1, d2, dtype, gen, scale_b=0.1, extra=extra)
-    got, want, calls = run_both(variant, a, b, offs, layout=layout, gen=gen)
-    assert len(calls) == 3 and all(path == "mfma" for _, path in calls), calls
+    with K_.forced_path(path):
+        got, want, calls = run_both(variant, a, b, offs, layout=layout, gen=gen)
+    assert len(calls) == 3 and all(family == "mfma" for _, family in calls), calls
+    assert path == "auto" or LaunchLog.kernels == ["assembly"] * 3
     assert_grads_forward_bar(variant, got, want, a, b, offs)
     tot = sum(sizes)
     owned = {"2d3d": (slice(0, tot),), "3d2d": (slice(None), slice(0, tot))}.get(variant, (slice(None),))

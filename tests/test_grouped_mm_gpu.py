@@ -133,8 +133,9 @@ def test_2d3d_boundary_lists_unaligned_shapes(sizes):
 
 @pytest.mark.parametrize("sizes", BOUNDARY_LISTS + [[300, 0, 1, 255, 256, 257, 33], [256, 256], [257, 255, 512]])
 @pytest.mark.parametrize("b_col", [False, True])
-def test_2d3d_boundary_lists_mfma(sizes, b_col):
-    """Same lists on aligned K / N so that the MFMA family and its 256-row tiles run."""
+@pytest.mark.parametrize("path", ["auto", "mfma"])
+def test_2d3d_boundary_lists_mfma(sizes, b_col, path):
+    """Same lists on aligned K / N: the 128 x 128 tiles that such small products take, and, forced, the assembly tile."""
     gen = torch.Generator().manual_seed(sum(sizes) + 1)
     m = sum(sizes)
     a, b = rnd(gen, m, 72), rnd(gen, len(sizes), 72, 264)
@@ -142,8 +143,10 @@ def test_2d3d_boundary_lists_mfma(sizes, b_col):
     if b_col:
         bd = bd.transpose(1, 2).contiguous().transpose(1, 2)
     out = torch.full((m, 264), float("nan"), device=DEV, dtype=torch.bfloat16)
-    K_.grouped_mm_2d3d(a.to(DEV), bd, offs_of(sizes).to(DEV), out)
+    with K_.forced_path(path):
+        K_.grouped_mm_2d3d(a.to(DEV), bd, offs_of(sizes).to(DEV), out)
     check(out, a, b, offs_of(sizes), 72, path="mfma")
+    assert K_.last_kernel() == ("any" if path == "auto" else "assembly")
 
 
 SMALL_GROUPS = [1, 15, 16, 17, 31, 33, 0, 1, 1, 63, 64, 65, 127, 129, 2]
@@ -169,6 +172,7 @@ def test_small_groups_on_every_tile_height(K, N, b_col, tall, shrt):
         K_.grouped_mm_2d3d(a.to(DEV), bd, offs_of(sizes).to(DEV), out)
         torch.cuda.synchronize()
     check(out, a, b, offs_of(sizes), K, path="mfma")
+    assert K_.last_kernel() == ("any" if (tall, K) == (-1, 72) else "assembly")
 
 
 def test_output_larger_than_4_gib():
@@ -244,7 +248,9 @@ def test_launch_replays_from_a_captured_graph():
 @pytest.mark.parametrize("a_col", [False, True])
 @pytest.mark.parametrize("b_col", [False, True])
 @pytest.mark.parametrize("variant", ["2d3d", "3d3d", "2d2d", "3d2d"])
-def test_all_layouts_all_variants_mfma(variant, a_col, b_col):
+@pytest.mark.parametrize("path", ["auto", "mfma"])
+def test_all_layouts_all_variants_mfma(variant, a_col, b_col, path):
+    """Every variant and layout, on the kernel chosen for the size and, forced, on the assembly tile."""
     gen = torch.Generator().manual_seed(17)
     sizes = [77, 0, 1, 130, 64, 200]  # sum 472
     offs = offs_of(sizes)
@@ -263,11 +269,13 @@ def test_all_layouts_all_variants_mfma(variant, a_col, b_col):
     if b_col:
         bd = bd.transpose(-2, -1).contiguous().transpose(-2, -1)
     out = torch.full(shape, float("nan"), device=DEV, dtype=torch.bfloat16)
-    if offs is None:
-        fn(ad, bd, out)
-    else:
-        fn(ad, bd, offs.to(DEV), out)
+    with K_.forced_path(path):
+        if offs is None:
+            fn(ad, bd, out)
+        else:
+            fn(ad, bd, offs.to(DEV), out)
     check(out, a, b, offs, k, path="mfma")
+    assert path == "auto" or K_.last_kernel() == "assembly"
 
 
 @pytest.mark.parametrize("tall,shrt", [(256, 64), (256, 0), (128, 64), (128, 0)])
@@ -289,6 +297,7 @@ def test_tile_heights_agree_bit_for_bit(tall, shrt, b_col):
         with K_.forced_tile_heights(*heights):
             K_.grouped_mm_2d3d(ad, bd, offs.to(DEV), out)
         torch.cuda.synchronize()
+        assert K_.last_kernel() == "assembly"
         outs.append(out.cpu())
     check(outs[0], a, b, offs, 328, path="mfma")
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
@@ -313,9 +322,10 @@ def test_3d2d_on_the_assembly_tile(sizes, in_dtype, out_dtype, a_col, b_col):
     if b_col:
         bd = bd.transpose(-2, -1).contiguous().transpose(-2, -1)
     out = torch.full((328, n_total + extra), float("nan"), device=DEV, dtype=out_dtype)
-    K_.grouped_mm_3d2d(ad, bd, offs.to(DEV), out)
+    with K_.forced_path("mfma"):
+        K_.grouped_mm_3d2d(ad, bd, offs.to(DEV), out)
     torch.cuda.synchronize()
-    assert K_.last_path() == "mfma" and K_._lib.load().gmm_last_mfma_config() == 1
+    assert K_.last_path() == "mfma" and K_._lib.load().gmm_last_mfma_config() == 1 and K_.last_kernel() == "assembly"
     got = out.cpu()
     assert torch.isnan(got[:, n_total:].float()).all()
     want = oracle.grouped_mm(a, b, offs, out_dtype=out_dtype)
@@ -486,12 +496,13 @@ def test_fp16_inputs_on_the_assembly_tile(variant, a_col, b_col, out_dtype):
     if b_col:
         bd = bd.transpose(-2, -1).contiguous().transpose(-2, -1)
     out = torch.full(shape, float("nan"), device=DEV, dtype=out_dtype)
-    if offs is None:
-        fn(ad, bd, out)
-    else:
-        fn(ad, bd, offs.to(DEV), out)
+    with K_.forced_path("mfma"):
+        if offs is None:
+            fn(ad, bd, out)
+        else:
+            fn(ad, bd, offs.to(DEV), out)
     torch.cuda.synchronize()
-    assert K_.last_path() == "mfma" and K_._lib.load().gmm_last_mfma_config() == 1
+    assert K_.last_path() == "mfma" and K_._lib.load().gmm_last_mfma_config() == 1 and K_.last_kernel() == "assembly"
     want = oracle.grouped_mm(a, b, offs, out_dtype=out_dtype)
     got = out.cpu()
     assert torch.equal(torch.isnan(got.float()), torch.isnan(want.float())), "ownership differs"
