@@ -403,12 +403,13 @@ static int64_t host_tile_list23(const int32_t* offs_host, int32_t G, int32_t jag
   std::vector<int32_t> order(size_t(G), 0);
   for (int g = 0; g < G; ++g) order[g] = g;
   if (gmm_use_k_queue(p, tile_n, num_workgroups)) {
-    std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
-      int xl, xh, yl, yh;
-      gmm_group_range(offs_host, x, extent, xl, xh);
-      gmm_group_range(offs_host, y, extent, yl, yh);
-      return xh - xl > yh - yl;
-    });
+    std::vector<uint32_t> keys(size_t(G), 0);
+    for (int g = 0; g < G; ++g) {
+      int lo, hi;
+      gmm_group_range(offs_host, g, K, lo, hi);
+      keys[g] = gmm_k_queue_key(g, hi - lo, K);
+    }
+    std::sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return keys[x] > keys[y]; });
     group_major = 1;   // every group's tall tiles, then its remainder tiles
     xcd_remap = 0;     // the tickets of an XCD are neighbours already
   }

@@ -215,10 +215,9 @@ __device__ __forceinline__ GmmTile gmm_locate_tile2(const GmmParams& p, const in
 
 // ---- tile queue of a jagged contraction -------------------------------------------------------------- //
 // Every group has the same grid of tiles, but its contraction is as long as the group, so dealing tiles round by round
-// leaves whole chips waiting for the workgroups that drew the long groups: 32768 rows in 128 skewed groups, 2048 x 768
-// each, keep the average workgroup busy for 141 us of 234 in a model of the kernel's tile times (258 us measured).  Here the groups are
-// sorted by length, longest first, and a workgroup draws its next tile when it is free (143 us in the model, 211 measured; sorted
-// but dealt round by round 199, drawn in group order 199).
+// leaves whole chips waiting for the workgroups that drew the long groups.  Here the groups are sorted by length, longest
+// first, and a workgroup draws its next tile when it is free.  128 groups, 20 of them empty, the others skewed (log-normal,
+// sigma 2.4), 32768 elements, 2048 x 768 each, bf16: dealt in group order 230 us, drawn 161; fp32 result 306 and 212.
 // The sorted list is cut into spans of one tile per workgroup and every span into one block per XCD, so that the tiles
 // an XCD runs together are neighbours; each XCD has a counter of its own, in the head of the workspace, and a workgroup
 // whose XCD has nothing left draws from the others.  The first tile needs no draw, the following ticket is drawn
@@ -226,8 +225,9 @@ __device__ __forceinline__ GmmTile gmm_locate_tile2(const GmmParams& p, const in
 // A drawn tile is located alone, on the critical path: 1.4 us each, where tiles that are dealt are located several at a
 // time.  Dealt round by round, the sorted list leaves workgroups apart by no more than the longest tile's time less the
 // shortest's, 1.5 us per K tile of 64.  So tiles are drawn when the longest group exceeds the mean by two K tiles a round
-// (at one a round, groups of 64 to 128 elements on average lost 4 to 8 %), and dealt otherwise or without a workspace (us, 2048 x 768 in 128 groups, every list drawn / dealt: 1280 elements
-// 108 / 91, 32768 of 256 each 153 / 147; 32768 in skewed groups 163, dealt in group order 191).
+// (at one a round, groups of 64 to 128 elements on average lost 4 to 8 %), and dealt otherwise or without a workspace.
+// Dealing what is not worth drawing, us, every list drawn / dealt, the matrices above: 1280 elements 108 / 91, 32768 of 256
+// each 153 / 147.
 // One thread of the workgroup uses the queue; it ends when all eight counters have run out.
 struct GmmKQueue {
   int per, total, chunk;   // tiles per group, of the launch, of an XCD's block in a span
@@ -237,22 +237,34 @@ struct GmmKQueue {
   int ticket;              // drawn ticket (index in the counter's part of the list)
 
   // order[i] = group of rank i, bound[g] .. bound[g + 1] = range of group g.  All threads; ends with a barrier.
+  // keys: room for G + 3 words, aligned to 16 bytes.  A group's rank is the number of greater keys (gmm_k_queue_key, no two
+  // are equal), counted four to a broadcast read, for two groups of a thread at a time.  Every workgroup does it, so it is part
+  // of every launch: 512 groups of 512 x 512, 16384 elements 71 us (67 in group order; 105 with lengths compared one by one).
+  // Up to about 450 groups a bitonic sort takes longer (128 groups 5 us more, 512 groups 1 us less than one group at a time).
   template <int NT>
-  __device__ __forceinline__ void build(const GmmParams& p, int bn, int32_t* order, int32_t* bound) {
+  __device__ __forceinline__ void build(const GmmParams& p, int bn, int32_t* order, int32_t* bound, uint32_t* keys) {
     const int tid = threadIdx.x;
-    for (int g = tid; g < p.G; g += NT) bound[g + 1] = gmm_min(gmm_max(p.offs[g], 0), p.K);
-    if (tid == 0) bound[0] = 0;
-    __syncthreads();
     for (int g = tid; g < p.G; g += NT) {
-      const int mine = gmm_max(bound[g + 1] - bound[g], 0);
-      int rank = 0, before = 0;
+      int lo, hi;
+      gmm_group_range(p.offs, g, p.K, lo, hi);
+      if (g == 0) bound[0] = 0;
+      bound[g + 1] = gmm_min(gmm_max(p.offs[g], 0), p.K);
+      keys[g] = gmm_k_queue_key(g, hi - lo, p.K);
+    }
+    if (tid < 3) keys[p.G + tid] = 0;
+    __syncthreads();
+    for (int g = tid; g < p.G; g += 2 * NT) {
+      const bool two = g + NT < p.G;
+      const uint32_t u = keys[g], v = two ? keys[g + NT] : ~0u;
+      int before_u = 0, before_v = 0;
 #pragma unroll 8
-      for (int h = 0; h < p.G; ++h) {
-        const int end = bound[h + 1], len = gmm_max(end - before, 0);
-        rank += (len > mine || (len == mine && h < g)) ? 1 : 0;
-        before = end;
+      for (int h = 0; h < p.G; h += 4) {
+        const uint4 k = *reinterpret_cast<const uint4*>(keys + h);
+        before_u += (k.x > u) + (k.y > u) + (k.z > u) + (k.w > u);
+        before_v += (k.x > v) + (k.y > v) + (k.z > v) + (k.w > v);
       }
-      order[rank] = g;
+      order[before_u] = g;
+      if (two) order[before_v] = g + NT;
     }
     __syncthreads();
     int n_tall, n_short, rem_rows;

@@ -463,7 +463,7 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
 
   int total_tall = 0, total_tiles = 0;
   GmmKQueue q;
-  if constexpr (QUEUE) q.build<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short);
+  if constexpr (QUEUE) q.build<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, reinterpret_cast<uint32_t*>(lds));
   else total_tiles = gmm_build_tile_table2<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, total_tall);
   // The tiles of the last, partly filled round may be cut along K into `nparts` parts each (gmm_tail_split).
   // Tiles before split_base are dealt round-robin (workgroup w takes w, w + grid, ...); the parts are taken

@@ -372,3 +372,28 @@ def test_fabric_traffic_floor_of_the_mixtral_launch_order():
     assert 3.4e9 < blocked < 3.55e9, blocked
     assert plain > 2.4 * blocked
     assert blocked > 2.5 * operands
+
+
+@pytest.mark.parametrize("groups,M,N,queue", [(130, 512, 256, True), (512, 64, 256, True), (513, 64, 256, False),
+                                              (900, 8, 8, False), (256, 8, 8, False), (257, 8, 8, True), (4, 4096, 4096, False)])
+def test_jagged_contraction_longest_first_where_it_pays(groups, M, N, queue):
+    """More than one tile for some workgroup, groups that are smaller than the launch and no more than 512 of them: longest
+    group first, equal ones in order; else in group order (sorting is part of every workgroup's start)."""
+    rng = np.random.default_rng(groups)
+    sizes = rng.integers(0, 40, groups).tolist()
+    rec = tile_list2(sizes, CONTRACTION, M, N, sum(sizes), 128, 64)
+    want = sorted(range(groups), key=lambda g: -sizes[g]) if queue else list(range(groups))
+    assert list(dict.fromkeys(rec[:, 0].tolist())) == want
+    per = len(rec) // groups
+    assert per * groups == len(rec) and (np.bincount(rec[:, 0], minlength=groups) == per).all()
+
+
+def test_jagged_contraction_order_of_lengths_beyond_22_bits():
+    """Lengths count by their 22 leading bits (of the whole contraction's)."""
+    sizes = [5, 1 << 22, (1 << 22) + 8, 1 << 29, 3, 0] + [1 << 20] * 251
+    rec = tile_list2(sizes, CONTRACTION, 64, 256, sum(sizes), 128, 64)
+    order = list(dict.fromkeys(rec[:, 0].tolist()))
+    assert order[:3] == [3, 1, 2]              # 8 elements of 2^30 are a tie
+    shift = max(0, sum(sizes).bit_length() - 22)
+    keys = [sizes[g] >> shift for g in order]
+    assert keys == sorted(keys, reverse=True)
