@@ -225,7 +225,10 @@ __device__ __forceinline__ GmmTile gmm_locate_tile2(const GmmParams& p, const in
 // A drawn tile is located alone, on the critical path: 1.4 us each, where tiles that are dealt are located several at a
 // time.  Dealt round by round, the sorted list leaves workgroups apart by no more than the longest tile's time less the
 // shortest's, 1.5 us per K tile of 64.  So tiles are drawn when the longest group exceeds the mean by two K tiles a round
-// (at one a round, groups of 64 to 128 elements on average lost 4 to 8 %), and dealt otherwise or without a workspace.
+// (at one a round, groups of 64 to 128 elements on average lost 4 to 8 %), and dealt otherwise or without a workspace.  Without
+// one, where the spread may be any, every other round is dealt backwards: the skewed groups above take 196 us (212 with every
+// round forwards, 226 in group order), 33 groups of 1208 x 352, 21600 elements 39 (51).  With a workspace, where the spread
+// is small, it gains as often as it loses (223 and 238 us for 201 groups of 1072 x 1360, 6432 elements).
 // Dealing what is not worth drawing, us, every list drawn / dealt, the matrices above: 1280 elements 108 / 91, 32768 of 256
 // each 153 / 147.
 // One thread of the workgroup uses the queue; it ends when all eight counters have run out.
@@ -233,6 +236,7 @@ struct GmmKQueue {
   int per, total, chunk;   // tiles per group, of the launch, of an XCD's block in a span
   int turn;                // counters that have run out, counted from the workgroup's own
   bool drawn;              // tiles are drawn, not dealt; the same in all threads
+  bool back;               // dealt: every other round backwards
   int next;                // drawn: tile to run, -1: none left
   int ticket;              // drawn ticket (index in the counter's part of the list)
 
@@ -274,17 +278,21 @@ struct GmmKQueue {
     chunk = int(gridDim.x) >> 3;
     const int longest = gmm_max(bound[order[0] + 1] - bound[order[0]], 0);
     drawn = p.ws && longest - p.K / p.G >= 128 * gmm_cdiv(total, int(gridDim.x));
+    back = p.ws == nullptr;
     turn = 0;
     ticket = int(blockIdx.x) >> 3;
     next = tile_of(int(blockIdx.x) & 7, ticket);
   }
 
-  // Tiles that the workgroup is dealt, and the i-th of them.
+  // Tiles that the workgroup is dealt, and the i-th of them.  Backwards, the workgroups with the longest tiles of one round
+  // get the shortest of the next.
   __device__ __forceinline__ int dealt() const {
-    return gmm_max(gmm_cdiv(total - tile_number(0), int(gridDim.x)), 0);
+    const int rounds = total / int(gridDim.x);
+    return rounds + (tile_number(rounds) < total ? 1 : 0);
   }
   __device__ __forceinline__ int tile_number(int i) const {
-    return i * int(gridDim.x) + (int(blockIdx.x) & 7) * chunk + (int(blockIdx.x) >> 3);
+    const int place = (int(blockIdx.x) & 7) * chunk + (int(blockIdx.x) >> 3);
+    return i * int(gridDim.x) + (back && (i & 1) ? int(gridDim.x) - 1 - place : place);
   }
 
   // Tile number `i` of an XCD's part of the list, or -1 past its end.
