@@ -217,7 +217,7 @@ int launch(const GmmParams& p, hipStream_t stream) {
 }  // namespace
 
 int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream, int& kernel) {
-  if (gmm_staged_eligible(p)) {
+  if (gmm_staged_eligible(p) && !gmm_element_preferred(p, in_dtype, num_cus)) {
     kernel = GMM_KERNEL_ANY;
     return gmm_launch_staged(p, in_dtype, out_dtype, num_cus, stream);
   }

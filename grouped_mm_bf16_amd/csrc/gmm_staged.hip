@@ -611,6 +611,15 @@ bool gmm_staged_preferred(const GmmParams& p, int num_cus) {
   return nk <= 6 && tiles * nk <= 12 * cus && (nk == 1 || rows_fill || tiles <= cus);
 }
 
+// Products without alignment, 16-bit, that are over before a tile of 128 x 128 has started: K up to 16, the first operand
+// contiguous along it, no more such tiles than half the compute units.  The element-wise kernel's 64 x 64 tiles are then
+// so many times as fast as the staged kernel (1500 random calls): K 1 and 2 1.12, 3 and 4 1.14, 5 to 8 1.15, 9 to 12 1.21, 13
+// to 16 1.08, 17 to 24 0.91 (16 products of 212 x 9 x 5 5.0 us against 8.5).  With 128 to 256 tiles it is 0.98, with the first
+// operand contiguous along M 1.05 at best, and in fp32 the staged kernel is as fast at any K.
+bool gmm_element_preferred(const GmmParams& p, int in_dtype, int num_cus) {
+  return in_dtype != GMM_DT_F32 && p.a_sk == 1 && p.K <= 16 && 2 * most_tiles(p, 128) <= num_cus;
+}
+
 bool gmm_staged_eligible(const GmmParams& p) {
   // each operand contiguous along one of its dimensions; gathered rows only along K; element offsets are 64-bit, so
   // no extent is too large

@@ -123,6 +123,23 @@ def test_operands_smaller_than_a_chunk_and_strided_outputs():
     compare(out, a, b, None, "column-major output")
 
 
+# both sides of each line of the rule that leaves small products with a very short contraction to the element-wise kernel:
+# K 16 / 17, 128 / 129 tiles of 128 x 128, the operands' types and the first one's layout
+@pytest.mark.parametrize("G,M,K,N,a_col,dtype,kernel", [
+    (16, 212, 5, 9, False, torch.bfloat16, "element"), (3, 129, 16, 131, False, torch.float16, "element"),
+    (3, 129, 17, 131, False, torch.float16, "any"), (3, 129, 16, 131, True, torch.bfloat16, "any"),
+    (3, 129, 16, 131, False, torch.float32, "any"), (64, 129, 3, 65, False, torch.bfloat16, "element"),
+    (129, 63, 3, 65, False, torch.bfloat16, "any"), (4, 2, 2, 3, False, torch.bfloat16, "element")])
+def test_very_short_contractions(G, M, K, N, a_col, dtype, kernel):
+    gen = torch.Generator().manual_seed(G + M + K + N)
+    a, b = torch.randn(G, M, K, generator=gen).to(dtype), torch.randn(G, K, N, generator=gen).to(dtype)
+    for b_col in (False, True):
+        out = torch.full((G, M, N), float("nan"), device=DEV, dtype=dtype)
+        K_.grouped_mm_3d3d(misaligned(a, a_col, 1), misaligned(b, b_col, 1), out)
+        assert K_.last_kernel() == kernel
+        compare(out, a, b, None, f"{G} of {M}x{K}x{N} {dtype}")
+
+
 # both sides of each line of the rule that sends small aligned products to these kernels: K 384 / 392 (6 K tiles), rows per
 # group 64 / 63 with more than 256 tiles, 128-row tiles times K tiles around 3072, first operand contiguous along M
 @pytest.mark.parametrize("variant,G,M,K,N,a_col,small", [
