@@ -1,10 +1,9 @@
-"""Jagged contractions whose groups are cut along K: parts, clusters of parts and their counters, against the oracle and
-against the same launch without a workspace (nothing is cut)."""
+"""Jagged contractions whose groups are cut along K: parts, clusters of parts and their counters, against fp64 and against
+the same launch without a workspace (nothing is cut)."""
 import pytest
 import torch
 
 import grouped_mm_bf16_amd.kernels as K_
-from oracle import grouped_mm_oracle as oracle
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -55,13 +54,20 @@ def test_parts_add_up(sizes, M, N, extra, dtype, out_dtype, a_col, b_col):
             assert ((out[g].double().cpu() - want).abs() <= bound).all(), f"group {g} of {sizes[g]}"
 
 
-def test_offsets_that_overlap_are_not_cut():
+@pytest.mark.parametrize("G", [60, 100])       # the table of the groups in registers, and in LDS
+def test_offsets_that_overlap_are_not_cut(G):
     """Offsets that go back: more parts than the workspace has counters for, so the launch runs uncut."""
     K, M, N = 32768, 32, 64
     gen = torch.Generator().manual_seed(3)
     a = torch.randn(M, K, generator=gen).bfloat16().to(DEV)
     b = torch.randn(K, N, generator=gen).bfloat16().to(DEV)
-    offs = torch.tensor([K, 0] * 30, dtype=torch.int32, device=DEV)
-    outs = _launches(a, b, offs, (60, M, N), torch.bfloat16)
+    offs = torch.tensor([K, 0] * (G // 2), dtype=torch.int32, device=DEV)
+    assert G // 2 * 64 > 1020                  # parts of the groups that hold all of K, counters
+    outs = _launches(a, b, offs, (G, M, N), torch.bfloat16)
     assert torch.equal(outs[0].view(torch.int16), outs[2].view(torch.int16))
-    assert torch.equal(outs[0][2].view(torch.int16), outs[0][0].view(torch.int16))
+    x, y = a.cpu().double(), b.cpu().double()
+    want, size = x @ y, x.abs() @ y.abs()
+    bound = (K + 1) * 2.0 ** -24 * size + 2.0 ** -8 * want.abs()     # as above
+    got = outs[0].double().cpu()
+    assert ((got[0::2] - want).abs() <= bound).all()
+    assert (outs[0][1::2] == 0).all()          # [K, 0): empty
