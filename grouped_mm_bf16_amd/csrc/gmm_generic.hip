@@ -1,9 +1,8 @@
-// Stride-generic grouped GEMM for gfx950: any row- or column-major operand,
-// any alignment, bf16 / fp16 / fp32 inputs, fp32 accumulation (on the vector
-// ALU for small problems, on the matrix cores with fp32 MFMAs otherwise),
-// output in the input dtype or fp32.  It covers everything the MFMA
-// kernels do not take (odd leading dimensions such as K = 33, N = 29, fp16 and
-// fp32 operands) and serves as the on-device cross-check for them.
+// Element-wise grouped GEMM for gfx950: any strides, any alignment, bf16 / fp16 / fp32 inputs, fp32 products and accumulation
+// (on the vector ALU for small problems, on the matrix cores with fp32 MFMAs otherwise), output in the input dtype or
+// fp32.  It takes what no other kernel takes: operands contiguous along neither dimension, operands of fewer than 16
+// bytes, rows gathered from a column-major source; and the unaligned products with a very short contraction that it
+// runs faster (gmm_element_preferred).  Everything else without alignment, and fp32, runs in gmm_staged.hip.
 //
 // One kernel handles the four variants; the tile list comes from gmm_sched.h.
 // Computes what grouped_mm_bf16/kernels.py:197-245, 248-301, 304-419 and 475-521

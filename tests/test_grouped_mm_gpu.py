@@ -368,8 +368,8 @@ def test_mfma_rate_diagnostic_runs():
 @pytest.mark.parametrize("variant", ["2d3d", "3d3d", "2d2d", "3d2d"])
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 3e-4), (torch.bfloat16, None)])
 def test_generic_family_on_the_matrix_cores(variant, a_col, b_col, dtype, tol):
-    """Problems with at least one 128 x 128 tile that the 16-bit MFMA tile does not take (fp32 operands;
-    bf16 with odd extents): the stride-generic kernel built on v_mfma_f32_32x32x2_f32."""
+    """Problems with at least one 128 x 128 tile that the aligned 16-bit tiles do not take (fp32 operands; bf16 with odd
+    extents): the register-staged kernel for operands of any alignment."""
     gen = torch.Generator().manual_seed(53)
     sizes = [77, 0, 1, 331, 64, 200]  # sum 673
     offs = offs_of(sizes)
@@ -393,7 +393,7 @@ def test_generic_family_on_the_matrix_cores(variant, a_col, b_col, dtype, tol):
     else:
         fn(ad, bd, offs.to(DEV), out)
     torch.cuda.synchronize()
-    assert K_.last_path() == "generic"
+    assert K_.last_path() == "generic" and K_.last_kernel() == "any"
     want = oracle.grouped_mm(a, b, offs, out_dtype=dtype)
     got = out.cpu()
     assert torch.equal(torch.isnan(got.float()), torch.isnan(want.float())), "ownership differs"
@@ -402,6 +402,37 @@ def test_generic_family_on_the_matrix_cores(variant, a_col, b_col, dtype, tol):
     else:
         owned = ~torch.isnan(want)
         torch.testing.assert_close(got[owned], want[owned], rtol=tol, atol=tol)
+
+
+# both sides of each line between the two element-wise kernels: 128 rows and columns, K 64
+@pytest.mark.parametrize("M,K,N,kernel", [(128, 64, 128, "wide"), (257, 71, 131, "wide"), (127, 70, 129, "element"),
+                                          (129, 63, 128, "element"), (130, 100, 65, "element")])
+@pytest.mark.parametrize("in_dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32),
+                                               (torch.float32, torch.float32)])
+def test_operands_contiguous_along_neither_dimension(M, K, N, kernel, in_dtype, out_dtype):
+    """Every second column of every operand, which only the launchers take: the two kernels that load element by element."""
+    gen = torch.Generator().manual_seed(M + K + N)
+    strided = lambda t: torch.stack([t, torch.full_like(t, float("nan"))], -1).to(DEV)[..., 0]
+    ends = torch.tensor([0, 3, 70, 70], dtype=torch.int32)
+    G = len(ends)
+    for fn, sa, sb, so, jag in ((K_.grouped_mm_3d3d, (G, M, K), (G, K, N), (G, M, N), 0),
+                                (K_.grouped_mm_2d3d, (M, K), (G, K, N), (M, N), M),
+                                (K_.grouped_mm_2d2d, (M, K), (K, N), (G, M, N), K),
+                                (K_.grouped_mm_3d2d, (G, M, K), (K, N), (M, N), N)):
+        a, b = rnd(gen, *sa).to(in_dtype), rnd(gen, *sb).to(in_dtype)
+        offs = ends.clamp(max=jag - 1) if jag else None
+        out = torch.full(so, float("nan"), device=DEV, dtype=out_dtype)
+        args = (strided(a), strided(b)) + (() if offs is None else (offs.to(DEV),))
+        fn(*args, out)
+        torch.cuda.synchronize()
+        assert K_.last_kernel() == kernel
+        want, got = oracle.grouped_mm(a, b, offs, out_dtype=torch.float32), out.cpu()
+        owned = ~torch.isnan(want)
+        assert torch.equal(torch.isnan(got.float()), ~owned), "ownership differs"
+        # products of the operands' values and sums in fp32, in any order, on both sides (u = 2^-24); one rounding to 16 bits
+        bound = 2 * (K + 1) * 2.0 ** -24 * oracle.grouped_mm(a.abs(), b.abs(), offs, out_dtype=torch.float32)
+        bound += 0 if out_dtype == torch.float32 else 2.0 ** -8 * want.abs()
+        assert ((got.float() - want).abs()[owned] <= bound[owned]).all(), fn.__name__
 
 
 # ------------------------------------------------------------------ seeded random sweep
