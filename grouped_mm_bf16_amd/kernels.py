@@ -226,8 +226,8 @@ def forced_tile_heights(tall: int, shrt: int):
 
 @contextlib.contextmanager
 def tail_split(on: bool):
-    """Inside the block launches do (True) or do not (False) cut the tiles of a sparse last round along the
-    contraction.  A cut tile adds its fp32 partial sums in a fixed order, so results are reproducible either
+    """Inside the block launches do (True) or do not (False) use their workspace: cut the tiles of a sparse last round or the
+    groups of a jagged contraction along the contraction, draw tiles from its counters.  A cut tile adds its fp32 partial sums in a fixed order, so results are reproducible either
     way, but they differ in the last bit from the uncut tile's: tests that compare two launches bit for bit
     across different tile lists switch the split off."""
     lib = _lib.load()

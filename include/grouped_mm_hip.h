@@ -14,9 +14,9 @@
  *     dimension (the first group starts at 0); it is read on the device only;
  *   - in_dtype / out_dtype are gmm_dtype values; out_dtype is in_dtype or
  *     GMM_DT_F32;
- *   - `workspace` / `workspace_bytes`: optional device memory (NULL / 0: none) that lets a launch whose
- *     last round of tiles would leave most of the chip idle cut those tiles along the contraction (see
- *     gmm_workspace_bytes below); the library itself never allocates;
+ *   - `workspace` / `workspace_bytes`: optional device memory (NULL / 0: none) that lets a launch cut tiles along the
+ *     contraction where whole tiles would leave most of the chip idle, and hand out tiles of uneven length on demand
+ *     (see gmm_workspace_bytes below); the library itself never allocates;
  *   - `stream` is a hipStream_t (NULL = the default stream);
  *   - the return value is a gmm_status; nothing is thrown across the boundary.
  *   - elements that no group owns (rows / columns at or beyond offs[G-1]) are
@@ -56,7 +56,13 @@ const char* gmm_status_string(int status);
  * 16384 x 14336 -> 4096 has 4.25 rounds of tiles on 256 units) its tiles are cut along the contraction into
  * up to 8 parts, every part stores an fp32 partial tile in the workspace, and the part that arrives last adds
  * the partials in part order and stores the output: the result does not depend on timing and is rounded
- * once.  Layout: 4096 bytes of arrival counters, then slots of 262144 bytes (one fp32 tile each); the more
+ * once.  gmm_2d2d uses it in two more ways: groups that are long beside the number of tiles are cut into parts in the same
+ * manner, and tiles of groups of uneven length are drawn from counters in it by whichever workgroup is free.
+ * With and without a workspace (or with one of another size) the last bits of a result may differ where tiles are cut: gmm_2d3d,
+ * gmm_3d3d and gmm_3d2d with a partly filled last round, gmm_2d2d with a first operand contiguous along its rows or with
+ * fp32 or unaligned operands; aligned 16-bit gmm_2d2d with a first operand contiguous along K is never cut.  Eager and
+ * captured launches that both have one of gmm_workspace_bytes() give the same bits.
+ * Layout: 4096 bytes of counters, then slots of 262144 bytes (one fp32 tile each); the more
  * slots, the more freedom to split.  gmm_workspace_bytes() returns the size the library can make full use
  * of on the current device (4096 + 2 * compute units * 262144; 128 MiB on MI355X); a smaller workspace
  * limits the split, less than 4096 + 2 * 262144 bytes (or NULL) turns it off.  Rules for the caller:
@@ -171,7 +177,8 @@ int gmm_3d2d(const void* a, const void* b, void* out, const int32_t* offs, int32
  *   token_rows  int32[tokens * top_k]   the row of each slot (inverse of the sort)
  * experts <= 1023, top_k <= min(experts, 32), tokens * top_k < 2^31.  `workspace` is device memory of at
  * least gmm_moe_route_workspace_bytes(...) bytes (per-workgroup expert histograms; contents need not be
- * initialised); too small a workspace returns GMM_ERR_WORKSPACE.  Four launches on `stream`, no host sync. */
+ * initialised); too small a workspace returns GMM_ERR_WORKSPACE.  Two launches on `stream` for up to 4096 slots, four for
+ * more; no host sync. */
 int64_t gmm_moe_route_workspace_bytes(int64_t tokens, int64_t experts, int64_t top_k);
 int gmm_moe_route(const void* logits, int64_t logits_stride, int32_t logits_dtype,
                   int64_t tokens, int64_t experts, int64_t top_k, int32_t renormalize,
@@ -243,8 +250,8 @@ int gmm_set_xcd_remap(int on);
  * 1 = group by group; -1 (default) = chosen from the shapes (group by group when the tall tiles are 128 rows,
  * the regime of many small groups).  Returns the previous setting. */
 int gmm_set_group_major(int mode);
-/* 0: later launches ignore their workspace, so no tile is cut along the contraction (tests compare launches
- * bit for bit that would otherwise split differently); 1 (default): use it.  Returns the previous setting. */
+/* 0: later launches ignore their workspace, so no tile is cut along the contraction and none is drawn on demand (tests compare
+ * launches bit for bit that would otherwise split differently); 1 (default): use it.  Returns the previous setting. */
 int gmm_set_tail_split(int on);
 /* Tile heights of the assembly tile: tall = 256 or 128 (-1: chosen from the shapes), shrt = 64 or 0
  * (-1: 64 whenever the first operand is contiguous along the contraction).  Returns the previous

@@ -99,6 +99,8 @@ def test_split_tiles_match_the_oracle(variant, a_col, b_col, dtype, out_dtype):
 
 
 def test_jagged_contraction_is_never_cut():
+    """Aligned, the first operand contiguous along K: the assembly tile, whose bits do not depend on a workspace.  (Other jagged
+    contractions may be cut: test_k_parts_gpu.py.)"""
     gen = torch.Generator().manual_seed(12)
     sizes = [3000, 0, 3144]
     a, b = rnd(gen, 300, 6144), rnd(gen, 6144, 520, scale=0.05)
@@ -107,6 +109,7 @@ def test_jagged_contraction_is_never_cut():
         out = torch.full((3, 300, 520), float("nan"), device=DEV, dtype=torch.float32)
         with K_.tail_split(on):
             K_.grouped_mm_2d2d(a.to(DEV), b.to(DEV), offs_of(sizes).to(DEV), out)
+        assert K_.last_kernel() == "assembly"
         outs.append(out.cpu())
     assert torch.equal(outs[0], outs[1])
     oracle.assert_close_grouped(outs[0], oracle.grouped_mm(a, b, offs_of(sizes), out_dtype=torch.float32), a, b, offs_of(sizes))
