@@ -49,6 +49,8 @@ def current_stream(device: torch.device) -> int:
 # whatever stream its graph is replayed on, beside anything else.
 _workspaces: dict = {}
 
+_EAGER_ONLY = _lib.WORKSPACE_EAGER_ONLY
+
 # Last capture seen: its id, and whether torch gives allocations made inside it to the graph.
 _capture = (0, False)
 
@@ -92,8 +94,12 @@ def _captured_workspace(device: torch.device, stream: int) -> Optional[torch.Ten
 def call_with_workspace(launcher, args: tuple, device: torch.device, stream: int) -> int:
     """``launcher(*args, workspace, workspace_bytes, stream)`` with the stream's workspace, or with one of its own inside a
     capture if the launch has a use for it; returns the status."""
-    ws, nbytes = workspace(device, stream)
-    rc = launcher(*args, ws, nbytes | _lib.WORKSPACE_EAGER_ONLY, stream)
+    ws = _workspaces.get((device.index, stream))     # as workspace() has it, without the call
+    if ws is not None:
+        rc = launcher(*args, ws.data_ptr(), ws.numel() | _EAGER_ONLY, stream)
+    else:
+        ws, nbytes = workspace(device, stream)
+        rc = launcher(*args, ws, nbytes | _EAGER_ONLY, stream)
     if rc != _lib.ERR_WORKSPACE:
         return rc
     own = _captured_workspace(device, stream)
@@ -106,36 +112,44 @@ def _launch_now(variant: int, a: torch.Tensor, b: torch.Tensor, offs: Optional[t
                 out: torch.Tensor) -> None:
     lib = _lib.load()
     _require_gpu(a, b, offs, out)
-    in_dt, out_dt = _dtype_code(a.dtype), _dtype_code(out.dtype)
+    device = a.device
     # the device guard costs microseconds; only switch when the tensors live on another device
-    guard = torch.cuda.device(a.device) if a.device.index != torch.cuda.current_device() else contextlib.nullcontext()
-    with guard:
-        stream = current_stream(a.device)
-        pa, pb, po = a.data_ptr(), b.data_ptr(), out.data_ptr()
-        poffs = offs.data_ptr() if offs is not None else None
-        if variant == V_2D3D:
-            launcher = lib.gmm_2d3d
-            args = (pa, pb, po, poffs, offs.numel(), a.size(0), b.size(2), a.size(1),
-                    a.stride(0), a.stride(1), b.stride(0), b.stride(1), b.stride(2),
-                    out.stride(0), out.stride(1), in_dt, out_dt)
-        elif variant == V_3D3D:
-            launcher = lib.gmm_3d3d
-            args = (pa, pb, po, a.size(0), a.size(1), b.size(2), a.size(2),
-                    a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1), b.stride(2),
-                    out.stride(0), out.stride(1), out.stride(2), in_dt, out_dt)
-        elif variant == V_2D2D:
-            launcher = lib.gmm_2d2d
-            args = (pa, pb, po, poffs, offs.numel(), a.size(0), b.size(1), a.size(1),
-                    a.stride(0), a.stride(1), b.stride(0), b.stride(1),
-                    out.stride(0), out.stride(1), out.stride(2), in_dt, out_dt)
-        elif variant == V_3D2D:
-            launcher = lib.gmm_3d2d
-            args = (pa, pb, po, poffs, offs.numel(), a.size(1), b.size(1), a.size(2),
-                    a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1),
-                    out.stride(0), out.stride(1), in_dt, out_dt)
-        else:
-            raise RuntimeError(f"unknown variant {variant}")
-        rc = call_with_workspace(launcher, args, a.device, stream)
+    if device.index != torch.cuda.current_device():
+        with torch.cuda.device(device):
+            _launch_here(lib, device, variant, a, b, offs, out)
+    else:
+        _launch_here(lib, device, variant, a, b, offs, out)
+
+
+def _launch_here(lib, device: torch.device, variant: int, a: torch.Tensor, b: torch.Tensor, offs: Optional[torch.Tensor],
+                 out: torch.Tensor) -> None:
+    in_dt, out_dt = _dtype_code(a.dtype), _dtype_code(out.dtype)
+    stream = current_stream(device)
+    pa, pb, po = a.data_ptr(), b.data_ptr(), out.data_ptr()
+    poffs = offs.data_ptr() if offs is not None else None
+    if variant == V_2D3D:
+        launcher = lib.gmm_2d3d
+        args = (pa, pb, po, poffs, offs.numel(), a.size(0), b.size(2), a.size(1),
+                a.stride(0), a.stride(1), b.stride(0), b.stride(1), b.stride(2),
+                out.stride(0), out.stride(1), in_dt, out_dt)
+    elif variant == V_3D3D:
+        launcher = lib.gmm_3d3d
+        args = (pa, pb, po, a.size(0), a.size(1), b.size(2), a.size(2),
+                a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1), b.stride(2),
+                out.stride(0), out.stride(1), out.stride(2), in_dt, out_dt)
+    elif variant == V_2D2D:
+        launcher = lib.gmm_2d2d
+        args = (pa, pb, po, poffs, offs.numel(), a.size(0), b.size(1), a.size(1),
+                a.stride(0), a.stride(1), b.stride(0), b.stride(1),
+                out.stride(0), out.stride(1), out.stride(2), in_dt, out_dt)
+    elif variant == V_3D2D:
+        launcher = lib.gmm_3d2d
+        args = (pa, pb, po, poffs, offs.numel(), a.size(1), b.size(1), a.size(2),
+                a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1),
+                out.stride(0), out.stride(1), in_dt, out_dt)
+    else:
+        raise RuntimeError(f"unknown variant {variant}")
+    rc = call_with_workspace(launcher, args, device, stream)
     _lib.check(rc, "grouped_mm launch")
 
 
