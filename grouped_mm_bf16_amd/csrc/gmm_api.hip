@@ -409,7 +409,10 @@ static int64_t host_tile_list23(const int32_t* offs_host, int32_t G, int32_t jag
       gmm_group_range(offs_host, g, K, lo, hi);
       keys[g] = gmm_k_queue_key(g, hi - lo, K);
     }
-    std::sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return keys[x] > keys[y]; });
+    int n_tall, n_short, rem_rows;
+    gmm_split_rows(M, tall, shrt, n_tall, n_short, rem_rows);
+    if (gmm_k_queue_sorts(int64_t(n_tall + n_short) * gmm_cdiv(N, tile_n), G, num_workgroups))
+      std::sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return keys[x] > keys[y]; });
     group_major = 1;   // every group's tall tiles, then its remainder tiles
     xcd_remap = 0;     // the tickets of an XCD are neighbours already
   }

@@ -256,6 +256,21 @@ struct GmmKQueue {
       keys[g] = gmm_k_queue_key(g, hi - lo, p.K);
     }
     if (tid < 3) keys[p.G + tid] = 0;
+    int n_tall, n_short, rem_rows;
+    gmm_split_rows(p.M, p.tall, p.shrt, n_tall, n_short, rem_rows);
+    per = (n_tall + n_short) * gmm_cdiv(p.N, bn);
+    total = p.G * per;
+    chunk = int(gridDim.x) >> 3;
+    turn = 0;
+    ticket = int(blockIdx.x) >> 3;
+    next = tile_of(int(blockIdx.x) & 7, ticket);
+    back = p.ws == nullptr;
+    drawn = false;
+    if (!gmm_k_queue_sorts(per, p.G, int(gridDim.x))) {
+      for (int g = tid; g < p.G; g += NT) order[g] = g;
+      __syncthreads();
+      return;
+    }
     __syncthreads();
     for (int g = tid; g < p.G; g += 2 * NT) {
       const bool two = g + NT < p.G;
@@ -271,17 +286,8 @@ struct GmmKQueue {
       if (two) order[before_v] = g + NT;
     }
     __syncthreads();
-    int n_tall, n_short, rem_rows;
-    gmm_split_rows(p.M, p.tall, p.shrt, n_tall, n_short, rem_rows);
-    per = (n_tall + n_short) * gmm_cdiv(p.N, bn);
-    total = p.G * per;
-    chunk = int(gridDim.x) >> 3;
     const int longest = gmm_max(bound[order[0] + 1] - bound[order[0]], 0);
     drawn = p.ws && longest - p.K / p.G >= 128 * gmm_cdiv(total, int(gridDim.x));
-    back = p.ws == nullptr;
-    turn = 0;
-    ticket = int(blockIdx.x) >> 3;
-    next = tile_of(int(blockIdx.x) & 7, ticket);
   }
 
   // Tiles that the workgroup is dealt, and the i-th of them.  Backwards, the workgroups with the longest tiles of one round

@@ -652,7 +652,11 @@ void plan(GmmParams& p, GmmLayout lay, int config, int num_cus) {
 
 bool gmm_mfma_uses_workspace(GmmParams p, GmmLayout lay, int config, int num_cus) {
   plan(p, lay, config, num_cus);
-  return p.ws_parts > 0 || (config == GMM_CFG_ASM_256x256 && gmm_use_k_queue(p, GMM_TILE_N, p.num_wg));
+  if (p.ws_parts > 0) return true;
+  if (config != GMM_CFG_ASM_256x256 || !gmm_use_k_queue(p, GMM_TILE_N, p.num_wg)) return false;
+  int n_tall, n_short, rem_rows;
+  gmm_split_rows(p.M, p.tall, p.shrt, n_tall, n_short, rem_rows);
+  return gmm_k_queue_sorts(int64_t(n_tall + n_short) * gmm_cdiv(p.N, GMM_TILE_N), p.G, p.num_wg);   // else nothing is drawn
 }
 
 int gmm_launch_mfma(GmmParams p, GmmLayout lay, int in_dtype, int out_dtype, int config, int num_cus, hipStream_t stream) {

@@ -228,19 +228,22 @@ GMM_HD int gmm_group_tile_cols(int jag, int lo, int hi, int N, int align, int bn
 // on demand), or deal them round by round in group order?
 //   - A group with at least as many tiles as the launch has workgroups gives every one of them the same share, and
 //     workgroups that run in step share operand panels: dealt, 8 groups of 896 tiles (4096 x 14336, 16384 rows, fp32
-//     result) take 1682 us, from the queue 1698.
-//   - Smaller groups make uneven shares (figures at GmmKQueue), but not where every workgroup has one tile at most: there
-//     sorting only costs, 25 groups of 32 x 8, 608 elements 14 us against 11.
+//     result) take 1682 us, from the queue 1698.  Smaller groups make uneven shares (figures at GmmKQueue).
 //   - Sorting costs the square of the groups: at 512 groups 4 us (2 at 300), at 900 groups 30 us (512 x 512 each, 16384
 //     elements 142 against 110).  Over 180 random calls of 8 to 300 groups the queue is 4.5 % faster on average, between
 //     1.76 and 0.78 times.
+//   - Where no workgroup has more than one tile nothing is sorted (gmm_k_queue_sorts), and the queue needs 2.5 us less to
+//     its first tile than the other kernel's table: 4 groups of 8 x 296, 144 elements 7.8 against 10.4, 414 random calls
+//     1.21 times as fast on average.
 GMM_HD bool gmm_use_k_queue(const GmmParams& p, int bn, int num_wg) {
   if (p.jag != GMM_JAG_K) return false;
   int n_tall, n_short, rem_rows;
   gmm_split_rows(p.M, p.tall, p.shrt, n_tall, n_short, rem_rows);
-  const int64_t per = int64_t(n_tall + n_short) * gmm_cdiv(p.N, bn);
-  return per < num_wg && per * p.G > num_wg && p.G <= 512;
+  return int64_t(n_tall + n_short) * gmm_cdiv(p.N, bn) < num_wg && p.G <= 512;
 }
+
+// Is the queue sorted?  `per` tiles per group.
+GMM_HD bool gmm_k_queue_sorts(int64_t per, int G, int num_wg) { return per * G > num_wg; }
 
 // Order of the groups in that queue: descending keys, that is by length, then by number.  22 bits of the length count.
 GMM_HD uint32_t gmm_k_queue_key(int g, int len, int K) {

@@ -20,8 +20,8 @@ def _sizes(groups, total, seed):
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("a_col,b_col", [(True, False), (False, True), (True, True)])
-@pytest.mark.parametrize("groups,M,N", [(70, 312, 528), (300, 256, 64), (9, 1280, 2048), (259, 8, 8), (512, 72, 8),
-                                           (513, 8, 8)])
+@pytest.mark.parametrize("groups,M,N", [(70, 312, 528), (300, 256, 64), (9, 1280, 2048), (256, 8, 8), (257, 8, 8),
+                                           (512, 72, 8), (513, 8, 8), (3, 40, 72)])
 def test_every_tile_once_and_counters_back_at_zero(groups, M, N, a_col, b_col, out_dtype):
     K = 3000
     gen = torch.Generator().manual_seed(groups)

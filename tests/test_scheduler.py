@@ -377,8 +377,8 @@ def test_fabric_traffic_floor_of_the_mixtral_launch_order():
 @pytest.mark.parametrize("groups,M,N,queue", [(130, 512, 256, True), (512, 64, 256, True), (513, 64, 256, False),
                                               (900, 8, 8, False), (256, 8, 8, False), (257, 8, 8, True), (4, 4096, 4096, False)])
 def test_jagged_contraction_longest_first_where_it_pays(groups, M, N, queue):
-    """More than one tile for some workgroup, groups that are smaller than the launch and no more than 512 of them: longest
-    group first, equal ones in order; else in group order (sorting is part of every workgroup's start)."""
+    """Where some workgroup has more than one tile, groups are smaller than the launch and no more than 512: longest group
+    first, equal ones in order; else in group order (sorting is part of every workgroup's start)."""
     rng = np.random.default_rng(groups)
     sizes = rng.integers(0, 40, groups).tolist()
     rec = tile_list2(sizes, CONTRACTION, M, N, sum(sizes), 128, 64)
