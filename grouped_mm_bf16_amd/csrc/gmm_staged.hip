@@ -61,12 +61,19 @@ __device__ __forceinline__ uint4 load_part(const T* p, const T* last, int n) {
   uint4 v = load16(cross ? last : p);
   const int shift = cross ? int(p - last) : 0;           // elements; only looked at when n > 0
   if (__ballot(n > 0 && shift > 0)) {
-    // the operand's very last chunks, down by 4, 2 and 1 elements (one element at a time it was 7 steps of 12 instructions)
-    if (sizeof(T) == 2 ? shift & 4 : shift & 2) v = make_uint4(v.z, v.w, 0u, 0u);
-    if (sizeof(T) == 2 ? shift & 2 : shift & 1) v = make_uint4(v.y, v.z, v.w, 0u);
-    if (sizeof(T) == 2 && (shift & 1))
-      v = make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
-                     __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16);
+    // rare (the operand's very last chunk): a loop over single elements.  Steps of 4, 2 and 1 elements are faster where it runs
+    // (3 products of 726 x 14 x 1 1 us of 10), but make the code longer and every other launch 0.2 us slower.
+#pragma unroll 1
+    for (int s = EPC - 1; s > 0; --s) {
+      const bool go = s <= shift;
+      uint4 w;
+      if constexpr (sizeof(T) == 2)
+        w = make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                       __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16);
+      else
+        w = make_uint4(v.y, v.z, v.w, 0u);
+      v.x = go ? w.x : v.x; v.y = go ? w.y : v.y; v.z = go ? w.z : v.z; v.w = go ? w.w : v.w;
+    }
   }
   uint32_t* w = &v.x;
 #pragma unroll
@@ -484,15 +491,23 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
         if (row < tile.m_lo || row >= tile.m_hi || col >= tile.n_hi || col + OEC <= tile.n_lo) continue;
         const char* src = stage + (x / ECPR) * EPITCH + (x % ECPR) * 16;
         OutT* dst = c + int64_t(row) * p.c_sm + int64_t(col) * p.c_sn;
-        const uint4 v = *reinterpret_cast<const uint4*>(src);
+        // The row's ragged end, or an output that is not contiguous along its columns, goes out element by element: out of
+        // registers, or with a loop over the elements there are, as each pair of types is faster (a loop over all elements that
+        // waits for the LDS for each of them takes 3 us of a launch).  us, that loop / this: bf16 2087 x 1034 in 80 groups of 3
+        // elements 130 / 123, 3 products of 1000 x 1001 x 515 28 / 26, fp32 60 of 300 x 65 x 131 16.1 / 14.9.
+        constexpr bool MIXED = sizeof(T) == 2 && OSZ == 4;
+        uint4 v;
+        if constexpr (sizeof(T) == 2) v = *reinterpret_cast<const uint4*>(src);   // fp32 has no registers to spare here
+        const void* const chunk = sizeof(T) == 2 ? static_cast<const void*>(&v) : __builtin_assume_aligned(src, 16);
         if (p.c_sn == 1 && col >= tile.n_lo && col + OEC <= tile.n_hi) {
-          __builtin_memcpy(dst, &v, 16);
+          __builtin_memcpy(dst, chunk, 16);
+        } else if constexpr (MIXED) {
+          const int first = gmm_max(tile.n_lo - col, 0), end = gmm_min(tile.n_hi - col, OEC);
+#pragma unroll 1
+          for (int e = first; e < end; ++e) __builtin_memcpy(dst + e * p.c_sn, src + e * OSZ, OSZ);
         } else {
-          // The row's ragged end, or an output that is not contiguous along its columns, element by element out of registers:
-          // out of LDS, with a wait for each element's read, 3 us of every launch with an odd number of columns (3 products of
-          // 726 x 14 x 1 12.0 us, now 8.8; 200 random odd-sized calls 9 % faster on average, none slower).
           OutT out[OEC];
-          __builtin_memcpy(out, &v, 16);
+          __builtin_memcpy(out, chunk, 16);
 #pragma unroll
           for (int e = 0; e < OEC; ++e)
             if (col + e >= tile.n_lo && col + e < tile.n_hi) dst[e * p.c_sn] = out[e];
