@@ -630,13 +630,13 @@ bool gmm_staged_preferred(const GmmParams& p, int num_cus) {
   return nk <= 6 && tiles * nk <= 12 * cus && (nk == 1 || rows_fill || tiles <= cus);
 }
 
-// Products without alignment, 16-bit, that are over before a tile of 128 x 128 has started: K up to 16, the first operand
-// contiguous along it, no more such tiles than half the compute units.  The element-wise kernel's 64 x 64 tiles are then
-// so many times as fast as the staged kernel (1500 random calls): K 1 and 2 1.12, 3 and 4 1.14, 5 to 8 1.15, 9 to 12 1.21, 13
-// to 16 1.08, 17 to 24 0.91 (16 products of 212 x 9 x 5 5.0 us against 8.5).  With 128 to 256 tiles it is 0.98, with the first
-// operand contiguous along M 1.05 at best, and in fp32 the staged kernel is as fast at any K.
+// Products without alignment, 16-bit, that are over before a tile of 128 x 128 has started: K up to 16 and no more such tiles
+// than compute units.  The element-wise kernel's 64 x 64 tiles are then so many times as fast as the staged kernel (3000 random
+// calls; first operand contiguous along K, 129 to 256 tiles / along M, up to 128): K 1 and 2 1.18 / 1.11, 3 and 4 1.27 / 1.13, 5
+// to 8 1.17 / 1.14, 9 to 12 1.13 / 1.21, 13 to 16 0.93 / 1.15; K 17 to 20 1.0 / 0.93; 257 to 512 tiles 1.07 / 0.99 (64 products of
+// 466 x 7 x 3 5.9 us against 11.3; at worst 53 of 5 x 7 x 186 8.0 against 6.3).  In fp32 the staged kernel is faster at any K.
 bool gmm_element_preferred(const GmmParams& p, int in_dtype, int num_cus) {
-  return in_dtype != GMM_DT_F32 && p.a_sk == 1 && p.K <= 16 && 2 * most_tiles(p, 128) <= num_cus;
+  return in_dtype != GMM_DT_F32 && p.K <= 16 && most_tiles(p, 128) <= num_cus;
 }
 
 bool gmm_staged_eligible(const GmmParams& p) {

@@ -124,12 +124,12 @@ def test_operands_smaller_than_a_chunk_and_strided_outputs():
 
 
 # both sides of each line of the rule that leaves small products with a very short contraction to the element-wise kernel:
-# K 16 / 17, 128 / 129 tiles of 128 x 128, the operands' types and the first one's layout
+# K 16 / 17, 256 / 257 tiles of 128 x 128, the operands' types
 @pytest.mark.parametrize("G,M,K,N,a_col,dtype,kernel", [
     (16, 212, 5, 9, False, torch.bfloat16, "element"), (3, 129, 16, 131, False, torch.float16, "element"),
-    (3, 129, 17, 131, False, torch.float16, "any"), (3, 129, 16, 131, True, torch.bfloat16, "any"),
-    (3, 129, 16, 131, False, torch.float32, "any"), (64, 129, 3, 65, False, torch.bfloat16, "element"),
-    (129, 63, 3, 65, False, torch.bfloat16, "any"), (4, 2, 2, 3, False, torch.bfloat16, "element")])
+    (3, 129, 17, 131, False, torch.float16, "any"), (3, 129, 16, 131, True, torch.bfloat16, "element"), (3, 129, 17, 131, True, torch.bfloat16, "any"),
+    (3, 129, 16, 131, False, torch.float32, "any"), (128, 129, 3, 65, False, torch.bfloat16, "element"),
+    (257, 63, 3, 65, False, torch.bfloat16, "any"), (4, 2, 2, 3, False, torch.bfloat16, "element")])
 def test_very_short_contractions(G, M, K, N, a_col, dtype, kernel):
     gen = torch.Generator().manual_seed(G + M + K + N)
     a, b = torch.randn(G, M, K, generator=gen).to(dtype), torch.randn(G, K, N, generator=gen).to(dtype)
