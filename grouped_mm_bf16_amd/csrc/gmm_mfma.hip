@@ -462,9 +462,11 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   constexpr int CDIV = ACT ? 2 : 1;
 
   int total_tall = 0, total_tiles = 0;
+  bool any_tall = true;
   GmmKQueue q;
   if constexpr (QUEUE) q.build<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, reinterpret_cast<uint32_t*>(lds));
-  else total_tiles = gmm_build_tile_table2<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, total_tall);
+  else total_tiles = gmm_build_tile_table2<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, total_tall, any_tall);
+  const bool renumber = p.xcd_remap && gmm_renumbered(any_tall, p.N);
   // The tiles of the last, partly filled round may be cut along K into `nparts` parts each (gmm_tail_split).
   // Tiles before split_base are dealt round-robin (workgroup w takes w, w + grid, ...); the parts are taken
   // from a ticket counter in the workspace by whichever workgroup is free: part q is K part q / tail of tile
@@ -493,7 +495,7 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
       }
     } else if (tid < BATCH && mine < split_base) {
       const int t = int(mine);
-      const int tt = p.xcd_remap ? gmm_xcd_remap(t, split_base, gridDim.x) : t;
+      const int tt = renumber ? gmm_xcd_remap(t, split_base, gridDim.x) : t;
       gmm_store_rec(&tiles[tid], gmm_locate_tile2(p, cum_tall, cum_short, total_tall, tt, GMM_TILE_N), -1);
     }
     __syncthreads();
