@@ -18,6 +18,7 @@ ABI_VERSION = 3
 PATH_AUTO, PATH_GENERIC, PATH_MFMA = 0, 1, 2
 DT_BF16, DT_F16, DT_F32 = 0, 1, 2
 OK = 0
+ERR_UNSUPPORTED = 2
 ERR_WORKSPACE = 4
 WORKSPACE_EAGER_ONLY = 1 << 62
 
@@ -32,6 +33,7 @@ SIGNATURES = {
     "gmm_2d3d": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i32] + [_i64] * 3 + [_i64] * 7 + [_i32, _i32, _vp, _i64, _vp]),
     "gmm_2d3d_gather": (ctypes.c_int, [_vp] * 5 + [_i32] + [_i64] * 4 + [_i64] * 7 + [_i32, _i32, _vp, _i64, _vp]),
     "gmm_2d3d_swiglu": (ctypes.c_int, [_vp] * 5 + [_i32] + [_i64] * 4 + [_i64] * 7 + [_i32, _vp]),
+    "gmm_2d3d_swiglu_apart": (ctypes.c_int, [_vp] * 5 + [_i32] + [_i64] * 4 + [_i64] * 7 + [_i32, _vp]),
     "gmm_3d3d": (ctypes.c_int, [_vp, _vp, _vp, _i32] + [_i64] * 3 + [_i64] * 9 + [_i32, _i32, _vp, _i64, _vp]),
     "gmm_2d2d": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i32] + [_i64] * 3 + [_i64] * 7 + [_i32, _i32, _vp, _i64, _vp]),
     "gmm_3d2d": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i32] + [_i64] * 3 + [_i64] * 7 + [_i32, _i32, _vp, _i64, _vp]),

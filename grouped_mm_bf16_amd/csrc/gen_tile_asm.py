@@ -135,9 +135,11 @@ class Variant:
     def __init__(self, a_tr, b_tr, out_f32, tm=4, f16=0, b_nt=0, act=0):
         """b_nt: B is copied with the non-temporal hint (a B panel that no other tile reads).
         act: SwiGLU epilogue -- of each 128 columns the first 64 are gates and the last 64 their partners;
-        the tile stores silu(gate) * partner, 128 columns of a 16-bit output per 256 columns of the product."""
+        the tile stores silu(gate) * partner, 128 columns of a 16-bit output per 256 columns of the product.
+        act == 3: the product is rounded to the output's type before the activation, as by a kernel of its own."""
         self.a_tr, self.b_tr, self.out_f32, self.tm, self.f16, self.b_nt = a_tr, b_tr, out_f32, tm, f16, b_nt
-        self.act = act == 1
+        self.act = act in (1, 3)
+        self.rounded = act == 3
         self.partial = act == 2      # fp32 partial tile of a tile cut along K: stored through to memory (sc1)
         assert not (self.act and (out_f32 or a_tr)) and not (self.partial and (not out_f32 or b_nt))
         self.dt = "f16" if f16 else "bf16"   # element type of A, B and of a 16-bit output
@@ -167,7 +169,7 @@ class Variant:
         self.b_stage = TR_STAGE if b_tr else KC_STAGE
         self.b_base = self.stages * self.a_stage   # LDS offset of B buffer 0
         self.name = "%s%s_%s_%s_m%d%s%s" % ("t" if a_tr else "k", "t" if b_tr else "k", self.dt, "f32" if out_f32 else self.dt, 64 * tm,
-                                            "_bnt" if b_nt else "", "_swiglu" if act == 1 else ("_partial" if act == 2 else ""))
+                                            "_bnt" if b_nt else "", ("", "_swiglu", "_partial", "_swiglu_rounded")[act])
 
     def acc(self, i, j):
         """First accumulator register of the wave's 16 x 16 block (i, j), i < 2 tm, j < 8."""
@@ -629,6 +631,20 @@ def gen_epilogue(v, e, L):
                         e("v_accvgpr_read_b32 %s, a%d" % (vr(b + r), g0 + r))
                     for r in range(4):
                         e("v_accvgpr_read_b32 %s, a%d" % (vr(b + 4 + r), u0 + r))
+                    if v.rounded:
+                        # to the output's type and back, two values to a register in between
+                        for r in range(0, 8, 2):
+                            e("v_cvt_pk_%s_f32 %s, %s, %s" % (v.dt, vr(b + 8 + r // 2), vr(b + r), vr(b + r + 1)))
+                        for r in range(0, 8, 2):
+                            if v.f16:
+                                e("v_cvt_f32_f16 %s, %s" % (vr(b + r), vr(b + 8 + r // 2)))
+                                e("v_lshrrev_b32 %s, 16, %s" % (vr(b + 8 + r // 2), vr(b + 8 + r // 2)))
+                            else:
+                                e("v_lshlrev_b32 %s, 16, %s" % (vr(b + r), vr(b + 8 + r // 2)))
+                                e("v_and_b32 %s, 0xffff0000, %s" % (vr(b + r + 1), vr(b + 8 + r // 2)))
+                        if v.f16:
+                            for r in range(0, 8, 2):
+                                e("v_cvt_f32_f16 %s, %s" % (vr(b + r + 1), vr(b + 8 + r // 2)))
                     for r in range(4):
                         e("v_mul_f32 %s, 0xbfb8aa3b, %s" % (vr(b + 8 + r), vr(b + r)))
                     for r in range(4):
@@ -638,10 +654,13 @@ def gen_epilogue(v, e, L):
                         e("v_add_f32 %s, 1.0, %s" % (vr(b + 8 + r), vr(b + 8 + r)))
                     for r in range(4):
                         e("v_rcp_f32 %s, %s" % (vr(b + 8 + r), vr(b + 8 + r)))
+                    # rounded: the gate's activation first, the order of the activation kernel (a gate far below zero
+                    # makes the result zero however large its partner is)
+                    first, second = (b + 8, b + 4) if v.rounded else (b + 4, b + 8)
                     for r in range(4):
-                        e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(b + r), vr(b + 4 + r)))
+                        e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(b + r), vr(first + r)))
                     for r in range(4):
-                        e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(b + r), vr(b + 8 + r)))
+                        e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(b + r), vr(second + r)))
                     e("v_cvt_pk_%s_f32 %s, %s, %s" % (v.dt, vr(b + 8), vr(b), vr(b + 1)))
                     e("v_cvt_pk_%s_f32 %s, %s, %s" % (v.dt, vr(b + 9), vr(b + 2), vr(b + 3)))
                     e("ds_write_b64 %s, %s offset:%d" % (vr(V_EPI), vr(b + 8, 2), rowoff + 16 * j * 2))
@@ -720,12 +739,12 @@ def main():
     out.append("#define GMM_TILE_PITCH_ACT %d" % PITCH_ACT)
     for f16 in (0, 1):
         for a_tr, b_tr, f32, tm, b_nt, act in [(a, b, f, t, n, c) for a in (0, 1) for b in (0, 1) for f in (0, 1) for t in (4, 2, 1)
-                                               for n in (0, 1) for c in (0, 1, 2)]:
+                                               for n in (0, 1) for c in (0, 1, 2, 3)]:
             if tm != 4 and a_tr:
                 continue
             if b_nt and tm == 4:
                 continue      # only remainder tiles can be the sole reader of a B panel often enough to matter
-            if act == 1 and (a_tr or f32):
+            if act in (1, 3) and (a_tr or f32):
                 continue      # the gated epilogue: K-contiguous first operand, 16-bit output
             if act == 2 and (not f32 or b_nt):
                 continue      # partial tiles: fp32, ordinary B copies

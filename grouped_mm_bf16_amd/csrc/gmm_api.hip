@@ -147,6 +147,15 @@ int run(Problem& pr, hipStream_t stream) {
   // the SwiGLU epilogue exists on the assembly tile only: K-contiguous first operand, 16-bit output, whole
   // blocks of 64 gates + 64 partners
   if (p.act && !(can_asm && lay.a_kc && pr.out_dtype == pr.in_dtype && (p.N & 127) == 0)) return GMM_ERR_UNSUPPORTED;
+  if (p.act == 3) {
+    // partner columns half the matrix away, both reached from one tile's origin
+    if (lay.b_kc && (int64_t(p.N) / 2 + 256) * p.b_sn * 2 >= (int64_t(1) << 31)) return GMM_ERR_UNSUPPORTED;
+    // Up to 64 rows a group the product is a stream of the second operand, and pieces of 256 bytes from two places come slower
+    // than 512 bytes from one where the matrices are large.  Product and activation in two kernels / in this one, us: 64 groups of
+    // 2048 x 4096 with 256 rows 148 / 160, 8 of 4096 x 28672 with 128 rows 304 / 317; smaller matrices: 128 groups of 2048 x
+    // 1536 with 512 rows 118 / 114, 8 of 1024 x 8192 with 128 rows 34.0 / 29.9; more rows: 16 of 2048 x 8192, 2048 rows 159 / 157.
+    if (int64_t(p.M) <= 64 * int64_t(p.G) && p.K >= 2048 && int64_t(p.K) * p.N >= (int64_t(1) << 23)) return GMM_ERR_UNSUPPORTED;
+  }
   if (p.gather) {
     // the assembly tile gathers rows of a K-contiguous first operand whose byte offsets fit 31 bits; the
     // register-staged MFMA kernel has no gather: everything else goes to the generic family
@@ -272,20 +281,33 @@ int gmm_2d3d_gather(const void* a, const int32_t* row_index, const void* b, void
   return run(pr, static_cast<hipStream_t>(stream));
 }
 
-int gmm_2d3d_swiglu(const void* a, const int32_t* row_index, const void* b, void* out, const int32_t* offs, int32_t G,
-                    int64_t a_rows, int64_t M_total, int64_t N, int64_t K, int64_t a_sm, int64_t a_sk, int64_t b_sg,
-                    int64_t b_sk, int64_t b_sn, int64_t o_sm, int64_t o_sn, int32_t dtype, void* stream) {
+// act: GmmParams::act
+static int swiglu(const void* a, const int32_t* row_index, const void* b, void* out, const int32_t* offs, int32_t G,
+                  int64_t a_rows, int64_t M_total, int64_t N, int64_t K, int64_t a_sm, int64_t a_sk, int64_t b_sg,
+                  int64_t b_sk, int64_t b_sn, int64_t o_sm, int64_t o_sn, int32_t dtype, int act, void* stream) {
   if (!dims_ok(M_total, N, K) || !fits_i32(a_rows)) return GMM_ERR_BAD_ARGUMENT;
   Problem pr{};
   pr.p = GmmParams{a, b, out, offs, G, GMM_JAG_M, int32_t(M_total), int32_t(N), int32_t(K), 1,
                    0, a_sm, a_sk, b_sg, b_sk, b_sn, 0, o_sm, o_sn, 0, 0};
   pr.p.gather = row_index;
   pr.p.a_rows = int32_t(row_index ? a_rows : M_total);
-  pr.p.act = 1;
+  pr.p.act = act;
   pr.in_dtype = dtype;
   pr.out_dtype = dtype;
   if (g_forced_path.load(std::memory_order_relaxed) == GMM_PATH_GENERIC) return GMM_ERR_UNSUPPORTED;
   return run(pr, static_cast<hipStream_t>(stream));
+}
+
+int gmm_2d3d_swiglu(const void* a, const int32_t* row_index, const void* b, void* out, const int32_t* offs, int32_t G,
+                    int64_t a_rows, int64_t M_total, int64_t N, int64_t K, int64_t a_sm, int64_t a_sk, int64_t b_sg,
+                    int64_t b_sk, int64_t b_sn, int64_t o_sm, int64_t o_sn, int32_t dtype, void* stream) {
+  return swiglu(a, row_index, b, out, offs, G, a_rows, M_total, N, K, a_sm, a_sk, b_sg, b_sk, b_sn, o_sm, o_sn, dtype, 1, stream);
+}
+
+int gmm_2d3d_swiglu_apart(const void* a, const int32_t* row_index, const void* b, void* out, const int32_t* offs, int32_t G,
+                          int64_t a_rows, int64_t M_total, int64_t N, int64_t K, int64_t a_sm, int64_t a_sk, int64_t b_sg,
+                          int64_t b_sk, int64_t b_sn, int64_t o_sm, int64_t o_sn, int32_t dtype, void* stream) {
+  return swiglu(a, row_index, b, out, offs, G, a_rows, M_total, N, K, a_sm, a_sk, b_sg, b_sk, b_sn, o_sm, o_sn, dtype, 3, stream);
 }
 
 int gmm_3d3d(const void* a, const void* b, void* out, int32_t G, int64_t M, int64_t N, int64_t K,

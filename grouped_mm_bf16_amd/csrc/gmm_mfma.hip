@@ -385,10 +385,11 @@ __device__ __forceinline__ GmmTileScalars gmm_load_rec(const GmmTileRec* d) {
   return t;
 }
 
-// Operands of a tile for the assembly.  CDIV = 2 for the SwiGLU epilogue (256 columns of the product become
-// 128 columns of the output), ESZ = bytes per output element.
-template <int A_TR, int B_TR, int ESZ, int CDIV>
+// Operands of a tile for the assembly.  ACT as there: with the SwiGLU epilogue 256 columns of the product become 128
+// columns of the output.  ESZ = bytes per output element.
+template <int A_TR, int B_TR, int ESZ, int ACT>
 __device__ __forceinline__ GmmTileDesc gmm_describe_tile(const GmmParams& p, const GmmTileScalars& t) {
+  constexpr int CDIV = ACT ? 2 : 1;
   const int lda = int(A_TR ? p.a_sk : p.a_sm);
   const int ldb = int(B_TR ? p.b_sk : p.b_sn);
   const int ldc = int(p.c_sm);
@@ -417,12 +418,16 @@ __device__ __forceinline__ GmmTileDesc gmm_describe_tile(const GmmParams& p, con
     dsc.a.base = a + int64_t(k_begin) * lda + t.m0;
     dsc.a.bytes = (int64_t(p.K - 1 - k_begin) * lda + (p.M - t.m0)) * 2;
   }
+  // gate and partner columns apart: the tile's first gate column; the last tile of an odd number of 64-column turns also
+  // fetches columns that are not its own, whose results are not stored
+  const int b_n0 = ACT == 3 ? t.n0 / 2 : t.n0;
+  if (ACT == 3) dsc.b.apart = p.N / 2;
   if (!B_TR) {
-    dsc.b.base = b + int64_t(t.n0) * ldb + k_begin;
-    dsc.b.bytes = (int64_t(p.N - 1 - t.n0) * ldb + (p.K - k_begin)) * 2;
+    dsc.b.base = b + int64_t(b_n0) * ldb + k_begin;
+    dsc.b.bytes = (int64_t(p.N - 1 - b_n0) * ldb + (p.K - k_begin)) * 2;
   } else {
-    dsc.b.base = b + int64_t(k_begin) * ldb + t.n0;
-    dsc.b.bytes = (int64_t(p.K - 1 - k_begin) * ldb + (p.N - t.n0)) * 2;
+    dsc.b.base = b + int64_t(k_begin) * ldb + b_n0;
+    dsc.b.bytes = (int64_t(p.K - 1 - k_begin) * ldb + (p.N - b_n0)) * 2;
   }
   dsc.c = static_cast<char*>(p.c) + (int64_t(t.g) * p.c_sg + int64_t(t.m0) * ldc + t.n0 / CDIV) * ESZ;
   dsc.ldc = ldc;
@@ -459,7 +464,6 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds;
   constexpr int ESZ = OUT_F32 ? 4 : 2;
-  constexpr int CDIV = ACT ? 2 : 1;
 
   int total_tall = 0, total_tiles = 0;
   bool any_tall = true;
@@ -510,7 +514,7 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
       asm volatile("" : "+v"(lane_j));
       if (QUEUE && q.drawn && tid == 0) q.draw(p);
       const GmmTileScalars t = gmm_load_rec(&tiles[j]);
-      const GmmTileDesc dsc = gmm_describe_tile<A_TR, B_TR, ESZ, CDIV>(p, t);
+      const GmmTileDesc dsc = gmm_describe_tile<A_TR, B_TR, ESZ, ACT>(p, t);
       if constexpr (A_TR) {
         gmm_tile_compute<A_TR, B_TR, OUT_F32, 4, F16>(dsc, lds_base, lane_j, wave);
       } else {
@@ -556,7 +560,7 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
         int lane_j = lane;
         asm volatile("" : "+v"(lane_j));
         const GmmTileScalars t = gmm_load_rec(&tiles[0]);
-        GmmTileDesc dsc = gmm_describe_tile<A_TR, B_TR, ESZ, 1>(p, t);
+        GmmTileDesc dsc = gmm_describe_tile<A_TR, B_TR, ESZ, 0>(p, t);
         const int tail_idx = t.part >> 8;
         dsc.c = static_cast<char*>(p.ws) + GMM_WS_HEADER + size_t((t.part & 0xff) * tail + tail_idx) * GMM_WS_SLOT;
         dsc.ldc = 256;
@@ -592,7 +596,11 @@ int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
       return -1;
     } else {
       if (!lay.a_kc) return -1;
-      if (lay.b_kc)
+      if (p.act == 3 && lay.b_kc)
+        hipLaunchKernelGGL((gmm_asm_kernel<0, 0, 0, F16, 3>), grid, block, 0, stream, p);
+      else if (p.act == 3)
+        hipLaunchKernelGGL((gmm_asm_kernel<0, 1, 0, F16, 3>), grid, block, 0, stream, p);
+      else if (lay.b_kc)
         hipLaunchKernelGGL((gmm_asm_kernel<0, 0, 0, F16, 1>), grid, block, 0, stream, p);
       else
         hipLaunchKernelGGL((gmm_asm_kernel<0, 1, 0, F16, 1>), grid, block, 0, stream, p);

@@ -49,7 +49,8 @@ struct GmmParams {
   // (which then has `a_rows` rows); null: row r reads row r.
   const int32_t* gather;
   int32_t a_rows;
-  // 1: SwiGLU epilogue (assembly tile, jagged rows, 16-bit output): `c` has N / 2 columns, see gmm_tile.h
+  // SwiGLU epilogue (assembly tile, jagged rows, 16-bit output): `c` has N / 2 columns, see gmm_tile.h.  1: gate and partner
+  // columns alternate in blocks of 64; 3: all gate columns, then all partner columns, the product rounded to 16 bits first
   int32_t act;
   // Split of the last, partly filled round of the launch along K (assembly tile; see gmm_tail_split): fp32
   // partial tiles go to `ws` (GMM_WS_HEADER bytes of arrival counters that are zero between launches, then

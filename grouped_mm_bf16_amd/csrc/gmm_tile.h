@@ -32,6 +32,8 @@ struct GmmTileRegs {
 // device scope (sc1), so that a workgroup on another XCD can read it without anybody flushing an L2.
 // ACT = 1: SwiGLU epilogue.  Of every 128 columns of the product the first 64 are gates g and the last 64
 // their partners u; the tile stores silu(g) * u: 128 columns of a 16-bit output per 256-column tile.
+// ACT = 3: the same with g and u rounded to the output's type first, for a B that has all gate columns before all partner
+// columns (GmmOperand::apart).
 template <int A_TR, int B_TR, int OUT_F32, int TM, int F16, int B_NT, int ACT>
 __device__ __forceinline__ void gmm_tile_asm(GmmTileRegs& r);
 
@@ -87,6 +89,8 @@ struct GmmOperand {
   // read as zeros.  Null: tile row r is row r from `base`.
   const int32_t* gather = nullptr;
   int gather_n = 0, src_rows = 0;
+  // ACT = 3, second operand: columns from a gate column to its partner; `base` points at the tile's first gate column.
+  int apart = 0;
 };
 
 // Description of one tile for the assembly.  klen = number of k elements from k_begin that count.
@@ -104,10 +108,15 @@ struct GmmTileDesc {
   int share, sharers;    // L2 prefetch of B: this tile touches share number `share` of `sharers` (0: none)
 };
 
+// Column of the matrix, from the tile's first gate column, that is column `c` of a SwiGLU tile: turns of 64 gate columns and
+// their 64 partners.  A wave's 128 columns then hold both factors of its 64 results in the same lanes, whichever way the
+// matrix has them: only the addresses of the copies differ (16-byte chunks and cache lines never cross a turn).
+__device__ __forceinline__ int gmm_apart_column(int c, int apart) { return (c >> 7) * 64 + (c & 63) + ((c & 64) ? apart : 0); }
+
 // NI = copy instructions per wave and K tile for this operand (8 for 256 rows, 2 per 64 rows).
 // klen, khead and nk are the same for all lanes: whether the first / last K tile is a whole one is a
 // scalar branch, and only partial ones pay for the per-lane selects.
-template <int TR, int NI>
+template <int TR, int NI, bool APART = false>
 __device__ __forceinline__ void gmm_copy_offsets(int lane, int wave, const GmmOperand& op, int klen, int khead, int nk,
                                                  gmm_v8i& head, gmm_v8i& full, gmm_v8i& tail) {
   const int ld = op.ld;
@@ -133,12 +142,13 @@ __device__ __forceinline__ void gmm_copy_offsets(int lane, int wave, const GmmOp
       const int row = wave * (NI * 8) + i * 8 + (lane >> 3);
       const int c = (lane & 7) ^ gmm_swz(row);
       kk[i] = c * 8;
-      const int r = op.gather ? src[i] : row;
+      const int r = APART ? gmm_apart_column(row, op.apart) : op.gather ? src[i] : row;
       full[i] = r >= 0 ? r * ld * 2 + c * 16 : (int)GMM_OOB;
     } else {
       const int blk = wave * 8 + i;
       kk[i] = 8 * (blk >> 2) + (blk & 3) + 4 * (lane >> 5);
-      full[i] = kk[i] * ld * 2 + (lane & 31) * 16;
+      const int c = (lane & 31) * 8;
+      full[i] = kk[i] * ld * 2 + (APART ? gmm_apart_column(c, op.apart) : c) * 2;
     }
   }
   head = full;
@@ -163,7 +173,7 @@ __device__ __forceinline__ void gmm_copy_offsets(int lane, int wave, const GmmOp
 template <int A_TR, int B_TR, int OUT_F32, int TM = 4, int F16 = 0, int B_NT = 0, int ACT = 0>
 __device__ __forceinline__ void gmm_tile_compute(const GmmTileDesc& t, unsigned lds_base, int lane, int wave) {
   static_assert(TM == 4 || !A_TR, "short tiles exist for a K-contiguous A only");
-  static_assert(ACT != 1 || (!A_TR && !OUT_F32), "the SwiGLU epilogue: K-contiguous A, 16-bit output");
+  static_assert(!(ACT & 1) || (!A_TR && !OUT_F32), "the SwiGLU epilogue: K-contiguous A, 16-bit output");
   static_assert(ACT != 2 || (OUT_F32 && !B_NT), "partial tiles are fp32");
   constexpr int WROWS = 32 * TM;  // rows of the tile per wave row
   constexpr int B_BASE = GmmTileLayout<A_TR, TM>::b_base;
@@ -171,7 +181,7 @@ __device__ __forceinline__ void gmm_tile_compute(const GmmTileDesc& t, unsigned 
   const int nk = (t.klen + GMM_TILE_K - 1) / GMM_TILE_K;
   GmmTileRegs r;
   gmm_copy_offsets<A_TR, 2 * TM>(lane, wave, t.a, t.klen, t.khead, nk, r.voa_head, r.voa, r.voa_tail);
-  gmm_copy_offsets<B_TR, 8>(lane, wave, t.b, t.klen, t.khead, nk, r.vob_head, r.vob, r.vob_tail);
+  gmm_copy_offsets<B_TR, 8, ACT == 3>(lane, wave, t.b, t.klen, t.khead, nk, r.vob_head, r.vob, r.vob_tail);
   // Fragment read addresses.  An MFMA fragment is 16 rows (or columns) x 32 k: lane l holds row l % 16,
   // k 8 (l / 16) .. + 7.  K-contiguous operand: one ds_read_b128 of chunk 4 sp + l / 16 of the lane's row
   // (sp = k half of the K tile; one address per half, 16-row blocks are immediate offsets).  Transposed
@@ -200,9 +210,9 @@ __device__ __forceinline__ void gmm_tile_compute(const GmmTileDesc& t, unsigned 
   // Epilogue: the wave stages its block in LDS and reads it back row by row, 16 bytes per lane (see
   // gen_tile_asm.py).  ESZ bytes per element: a lane's chunk is NEL = 16 / ESZ columns, a row of the wave's
   // 128 columns takes LPR lanes, a read-back instruction covers 64 / LPR rows.
-  constexpr int WCOLS = ACT == 1 ? 64 : 128;                   // output columns of a wave
+  constexpr int WCOLS = (ACT & 1) ? 64 : 128;                   // output columns of a wave
   constexpr int ESZ = OUT_F32 ? 4 : 2, NEL = 16 / ESZ, LPR = WCOLS / NEL;
-  constexpr int EPITCH = OUT_F32 ? GMM_TILE_PITCH32 : (ACT == 1 ? GMM_TILE_PITCH_ACT : GMM_TILE_PITCH);
+  constexpr int EPITCH = OUT_F32 ? GMM_TILE_PITCH32 : ((ACT & 1) ? GMM_TILE_PITCH_ACT : GMM_TILE_PITCH);
   constexpr int STAGE_ROWS = OUT_F32 ? 32 : WROWS;        // rows a wave stages per pass
   int partial = 0;
   {
@@ -233,7 +243,11 @@ __device__ __forceinline__ void gmm_tile_compute(const GmmTileDesc& t, unsigned 
       const int per_tile = (256 + t.sharers - 1) / t.sharers, per_wave = (per_tile + 3) >> 2;
       const int idx = wave * per_wave + lane, line = t.share * per_tile + idx;
       if (lane < per_wave && idx < per_tile && line < 256)
-        off_b = B_TR ? (line >> 2) * t.b.ld * 2 + (line & 3) * 128 : line * t.b.ld * 2;
+{
+        int col = B_TR ? (line & 3) * 64 : line;
+        if (ACT == 3) col = gmm_apart_column(col, t.b.apart);
+        off_b = B_TR ? (line >> 2) * t.b.ld * 2 + col * 2 : col * t.b.ld * 2;
+      }
     }
     r.touch[0] = (int)GMM_OOB;
     r.touch[1] = off_b;

@@ -127,6 +127,19 @@ int gmm_2d3d_swiglu(const void* a, const int32_t* row_index, const void* b, void
                     int64_t out_stride_m, int64_t out_stride_n,
                     int32_t dtype, void* stream);
 
+/* The same for b [G, K, N] with all gate columns first, then all partner columns (N / 2 a multiple of 64), and with the
+ * product rounded to the output's type before the activation, as gmm_2d3d_gather and gmm_moe_activation leave it:
+ *   out[r, c] = silu(h[r, c]) * h[r, N / 2 + c].
+ * With b contiguous along K also (N / 2 + 256) * b_stride_n * 2 < 2^31.  GMM_ERR_UNSUPPORTED as well where the two calls are
+ * faster: up to 64 rows a group on average with K >= 2048 and K * N >= 2^23. */
+int gmm_2d3d_swiglu_apart(const void* a, const int32_t* row_index, const void* b, void* out,
+                          const int32_t* offs, int32_t G, int64_t a_rows,
+                          int64_t M_total, int64_t N, int64_t K,
+                          int64_t a_stride_m, int64_t a_stride_k,
+                          int64_t b_stride_g, int64_t b_stride_k, int64_t b_stride_n,
+                          int64_t out_stride_m, int64_t out_stride_n,
+                          int32_t dtype, void* stream);
+
 /* 3D x 3D: out[g] = a[g] @ b[g]
  * a [G, M, K], b [G, K, N], out [G, M, N].
  * Replaces grouped_mm_3d3d(mat_a, mat_b, out), reference kernels.py:524-550. */

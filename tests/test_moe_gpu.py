@@ -5,6 +5,7 @@ small, Mixtral and fine-grained sizes."""
 import pytest
 import torch
 
+from grouped_mm_bf16_amd import _lib
 from grouped_mm_bf16_amd import kernels as K_
 from grouped_mm_bf16_amd import moe
 from oracle import grouped_mm_oracle as oracle
@@ -233,6 +234,43 @@ def test_fused_swiglu_product(dtype, K, N, gather, b_col):
         K_.grouped_mm_2d3d(a.to(DEV), w.to(DEV), offs.to(DEV), h16)
     two = moe.moe_activation(h16[:M], "swiglu").cpu()
     oracle.assert_close(got[:M], two, K)
+
+
+@pytest.mark.parametrize("b_col", [False, True])
+@pytest.mark.parametrize("dtype,K,N", [(torch.bfloat16, 136, 128), (torch.float16, 136, 384), (torch.bfloat16, 2048, 1536), (torch.float16, 64, 640)])
+def test_swiglu_with_gate_and_partner_columns_apart(dtype, K, N, b_col):
+    """The up projection of a layer with weights as published, in one kernel: the roundings of product and activation in
+    two, on every tile height, an odd number of 64-column turns, gathered rows of zeros and rows past offs[-1]."""
+    gen = torch.Generator().manual_seed(K * N)
+    G, M, S = len(SIZES), sum(SIZES), 401
+    a = rnd(gen, S, K, dtype=dtype).to(DEV)
+    w = rnd(gen, G, K, N, dtype=dtype, scale=K ** -0.5).to(DEV)
+    a[7], w[:, :, 1] = 60000.0 if dtype == torch.float16 else 1e30, -abs(w[:, :, 1])      # results that overflow
+    if b_col:
+        w = w.transpose(1, 2).contiguous().transpose(1, 2)
+    idx = torch.randint(0, S, (M + 9,), generator=gen).to(torch.int32)
+    idx[3], idx[M - 1] = S, -1
+    idx, offs = idx.to(DEV), offs_of(SIZES).to(DEV)
+    out = torch.full((M + 9, N // 2), 77.0, device=DEV, dtype=dtype)
+    rc = _lib.load().gmm_2d3d_swiglu_apart(a.data_ptr(), idx.data_ptr(), w.data_ptr(), out.data_ptr(), offs.data_ptr(), G, S, M + 9, N, K,
+                                           *a.stride(), *w.stride(), *out.stride(), K_._dtype_code(dtype),
+                                           torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and K_.last_kernel() == "assembly"
+    two = moe.moe_activation(moe.grouped_mm_gathered(a, idx, w, offs)[:M], "swiglu").cpu()
+    got = out.cpu()
+    assert (got[M:] == 77.0).all() and (got[3] == 0).all()
+    assert torch.equal(got[:M].isfinite(), two.isfinite()) and torch.equal(got[:M].isnan(), two.isnan()) and not two.isfinite().all()
+    ok = two.isfinite()
+    ulp_close(got[:M][ok], two[ok], dtype)
+
+
+def test_layers_whose_up_projection_stays_two_kernels():
+    """Few rows of large matrices, an inner size that is no multiple of 64, forced kernels: the same layer results."""
+    for T, H, I, E, k in [(40, 2048, 2048, 2, 1), (40, 64, 72, 4, 2)]:
+        run_layer(*layer_case(T, T, H, I, E, k, "swiglu"), k, "swiglu")
+    with K_.forced_path("generic"):
+        run_layer(*layer_case(1, 40, 64, 128, 4, 2, "swiglu"), 2, "swiglu")
+        assert K_.last_path() == "generic"
 
 
 def test_fused_swiglu_rejects_what_the_tile_cannot_do():
