@@ -11,6 +11,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/grouped_mm_hip.h"
 
@@ -85,62 +86,88 @@ __device__ __forceinline__ float key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
-// ---------------------------------------------------------------- routing 1/4: top-k and weights
+// ---------------------------------------------------------------- routing: top-k and weights
 // One wave per token.  Choice j of token t is slot t * k + j.  Ties go to the lower expert index (a stable
 // descending sort).  weight = softmax over the chosen k logits (renorm) or over all E logits.
-template <typename T>
+// Lane l holds the order keys of experts l, l + 64, ...: kPer of them, in registers (in LDS, with an index loop per round, a
+// token's 8 of 128 choices took a wave 2.3 us).  The wave's best key is found first, then the first expert that holds it.
+template <typename T, int kPer>
+struct MoeTopk {
+  uint32_t key[kPer];   // 0 beyond the last expert
+
+  __device__ __forceinline__ void load(const T* row, int E, int lane) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int e = lane + (i << 6);
+      key[i] = e < E ? order_key(to_float(row[e])) : 0u;
+    }
+  }
+
+  // Lane j < k returns choice j and its weight.
+  __device__ __forceinline__ void choose(int E, int k, int renorm, int lane, int& my_e, float& weight) const {
+    uint32_t free_keys = 0, my_key = 0, top_key = 0;   // free_keys: bit i: the lane's i-th expert exists and is not chosen yet
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) free_keys |= lane + (i << 6) < E ? 1u << i : 0u;
+    my_e = 0;
+    for (int j = 0; j < k; ++j) {
+      uint32_t best = 0;
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const uint32_t v = (free_keys >> i) & 1u ? key[i] : 0u;
+        best = v > best ? v : best;
+      }
+      const uint32_t win = wave_umax(best);
+      int e_win = 0;
+      bool found = false;
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const uint64_t holders = __ballot(((free_keys >> i) & 1u) && key[i] == win);
+        if (!found && holders) {
+          e_win = (i << 6) + __ffsll((unsigned long long)holders) - 1;
+          found = true;
+        }
+      }
+      if ((e_win & 63) == lane) free_keys &= ~(1u << (e_win >> 6));
+      if (lane == j) { my_e = e_win; my_key = win; }
+      if (j == 0) top_key = win;
+    }
+    // exp(x - m) with an infinite maximum m (a +inf logit, or a row of -inf: every expert masked) is the limit
+    // of the softmax: all weight, in equal shares, on the entries that equal the maximum (inf - inf is NaN)
+    const float m = key_value(top_key);
+    const bool inf_max = (__float_as_uint(m) & 0x7fffffffu) == 0x7f800000u;
+    const float p = lane < k ? (inf_max ? (my_key == top_key ? 1.0f : 0.0f) : __expf(key_value(my_key) - m)) : 0.0f;
+    float den;
+    if (renorm) {
+      den = wave_sum(p);
+    } else {
+      float s = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        if (lane + (i << 6) < E) s += inf_max ? (key[i] == top_key ? 1.0f : 0.0f) : __expf(key_value(key[i]) - m);
+      den = wave_sum(s);
+    }
+    weight = p / den;
+  }
+};
+
+template <typename T, int kPer>
 __global__ void __launch_bounds__(256) moe_topk_kernel(const T* __restrict__ logits, int64_t ld, int tokens, int E, int k,
                                                        int renorm, int32_t* __restrict__ slot_expert,
                                                        float* __restrict__ slot_weight) {
-  __shared__ uint32_t keys[4][1024];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t = blockIdx.x * 4 + wave;
+  const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= tokens) return;
-  const T* row = logits + int64_t(t) * ld;
-  uint32_t* kw = keys[wave];   // lane l reads and writes entries l, l + 64, ... only
-  for (int e = lane; e < E; e += 64) kw[e] = order_key(to_float(row[e]));
-  uint32_t taken = 0, my_key = 0, top_key = 0;
-  int my_e = 0;
-  const int per_lane = (E + 63) >> 6;
-  for (int j = 0; j < k; ++j) {
-    // this lane's best entry that is still free (lowest index among equals), then the wave's best key
-    uint32_t best = 0;
-    int best_i = -1;
-    for (int i = 0; i < per_lane; ++i) {
-      const int e = lane + (i << 6);
-      if (e < E && !((taken >> i) & 1u) && (best_i < 0 || kw[e] > best)) { best = kw[e]; best_i = i; }
-    }
-    const uint32_t key_win = wave_umax(best_i >= 0 ? best : 0u);
-    // lowest expert index among the lanes that hold that key: lowest i first, then lowest lane
-    int e_win = 0;
-    for (int i = 0; i < per_lane; ++i) {
-      const uint64_t holders = __ballot(best_i == i && best == key_win);
-      if (holders) { e_win = (i << 6) + __ffsll((unsigned long long)holders) - 1; break; }
-    }
-    if ((e_win & 63) == lane) taken |= 1u << (e_win >> 6);
-    if (lane == j) { my_e = e_win; my_key = key_win; }
-    if (j == 0) top_key = key_win;
-  }
-  // exp(x - m) with an infinite maximum m (a +inf logit, or a row of -inf: every expert masked) is the limit
-  // of the softmax: all weight, in equal shares, on the entries that equal the maximum (inf - inf is NaN)
-  const float m = key_value(top_key);
-  const bool inf_max = (__float_as_uint(m) & 0x7fffffffu) == 0x7f800000u;
-  const float p = lane < k ? (inf_max ? (my_key == top_key ? 1.0f : 0.0f) : __expf(key_value(my_key) - m)) : 0.0f;
-  float den;
-  if (renorm) {
-    den = wave_sum(p);
-  } else {
-    float s = 0.0f;
-    for (int e = lane; e < E; e += 64) s += inf_max ? (kw[e] == top_key ? 1.0f : 0.0f) : __expf(key_value(kw[e]) - m);
-    den = wave_sum(s);
-  }
+  MoeTopk<T, kPer> token;
+  int e;
+  float weight;
+  token.load(logits + int64_t(t) * ld, E, lane);
+  token.choose(E, k, renorm, lane, e, weight);
   if (lane < k) {
-    slot_expert[int64_t(t) * k + lane] = my_e;
-    slot_weight[int64_t(t) * k + lane] = p / den;
+    slot_expert[int64_t(t) * k + lane] = e;
+    slot_weight[int64_t(t) * k + lane] = weight;
   }
 }
 
-// ---------------------------------------------------------------- routing 2/4: per-workgroup histograms
+// ---------------------------------------------------------------- routing of many slots 1/3: per-workgroup histograms
 // Workgroup b counts the experts of slots [b * spb, (b + 1) * spb) into row b of the table.
 __global__ void __launch_bounds__(256) moe_hist_kernel(const int32_t* __restrict__ slot_expert, int slots, int spb, int E,
                                                        int32_t* __restrict__ table) {
@@ -153,7 +180,7 @@ __global__ void __launch_bounds__(256) moe_hist_kernel(const int32_t* __restrict
   for (int e = threadIdx.x; e < E; e += 256) table[int64_t(blockIdx.x) * E + e] = hist[e];
 }
 
-// ---------------------------------------------------------------- routing 3/4: column scan + offs
+// ---------------------------------------------------------------- routing of many slots 2/3: column scan + offs
 // One workgroup of 1024 threads, thread e owns expert e: the table's column e becomes its exclusive prefix
 // over the workgroups, and offs[e] the inclusive prefix of the expert totals.
 __global__ void __launch_bounds__(1024) moe_scan_kernel(int32_t* __restrict__ table, int nb, int E, int32_t* __restrict__ offs) {
@@ -186,7 +213,7 @@ __global__ void __launch_bounds__(1024) moe_scan_kernel(int32_t* __restrict__ ta
   if (e < E) offs[e] = base + incl;
 }
 
-// ---------------------------------------------------------------- routing 4/4: stable scatter
+// ---------------------------------------------------------------- routing of many slots 3/3: stable scatter
 // Workgroup b (one wave) places its slots, in slot order, behind what earlier workgroups hold of the same
 // expert: row = offs[e - 1] + (slots of expert e in earlier workgroups) + (earlier slots of e in this one).
 // 64 slots at a time: the lanes that hold the same expert find each other with one ballot per bit of the
@@ -231,43 +258,38 @@ __global__ void __launch_bounds__(64) moe_scatter_kernel(const int32_t* __restri
   }
 }
 
-// ---------------------------------------------------------------- routing 2 .. 4 of a few slots in one workgroup
-// Up to kSmallSlots slots are counted, scanned and placed by the 16 waves of one workgroup, each wave a run of consecutive
-// slots, with the table of counts in LDS: a decoding step's three launches of 4.6, 4.6 and 6.5 us did next to nothing but
-// start (64 tokens, 8 of 128 experts).  The placing is that of moe_scatter_kernel.
-constexpr int kSmallSlots = 4096;
-constexpr int kSortWaves = 16;
+// ---------------------------------------------------------------- routing of up to kPlaceSlots slots: one kernel
+// Workgroup b places slots [b * 1024, b * 1024 + 1024), each of its 16 waves 64 of them.  It counts the experts of all slots
+// itself, those before its own apart from the others (LDS atomics, four copies against conflicts), so there is no table of
+// counts to write, wait for and scan: histogram, scan and scatter were three launches.  The placing is that of
+// moe_scatter_kernel.  With the choice, us: 32768 slots of 128 experts 26 -> 12, 16384 of 8 18 -> 11.  Counting grows with the
+// slots, in every workgroup: at 131072 29 against 44, at 196608 and more the three kernels are as fast.
+constexpr int kPlaceWaves = 16;
+constexpr int kPlaceBlock = 64 * kPlaceWaves;
+constexpr int kPlaceCopies = 4;
+constexpr int kPlaceSlots = 131072;
 
-__global__ void __launch_bounds__(64 * kSortWaves) moe_sort_small_kernel(const int32_t* __restrict__ slot_expert, int slots, int E, int k,
-                                                                         int32_t* __restrict__ offs, int32_t* __restrict__ row_token,
-                                                                         int32_t* __restrict__ token_rows) {
-  __shared__ int32_t table[kSortWaves * kMaxExperts];   // row w: counts, then cursors, of wave w's slots
-  __shared__ int32_t part[kSortWaves];
-  constexpr int kRounds = kSmallSlots / (64 * kSortWaves);
+// Rows of E counts: copies of the slots before the workgroup's own, copies of those behind them, the waves' cursors.
+constexpr int kPlaceRows = 2 * kPlaceCopies + kPlaceWaves;
+
+// expert: of the thread's slot s0 + tid, -1 if there is none.  count: as above, the counts of the workgroup's own slots still
+// zero.
+__device__ __forceinline__ void moe_place(int32_t* count, int32_t* part, int expert, int s0, int E, int k, bool write_offs, int32_t* offs,
+                                          int32_t* row_token, int32_t* token_rows) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rounds = (slots + 64 * kSortWaves - 1) / (64 * kSortWaves);
-  const int s0 = wave * rounds * 64;
-  int ev[kRounds];
-#pragma unroll
-  for (int i = 0; i < kRounds; ++i) {
-    const int s = s0 + 64 * i + lane;
-    ev[i] = i < rounds && s < slots ? slot_expert[s] : -1;
-  }
-  for (int i = tid; i < kSortWaves * E; i += 64 * kSortWaves) table[i] = 0;
+  int32_t* const cursor = count + 2 * kPlaceCopies * E;
+  if (expert >= 0) atomicAdd(&cursor[wave * E + expert], 1);
   __syncthreads();
-  int32_t* const mine = table + wave * E;
-#pragma unroll
-  for (int i = 0; i < kRounds; ++i)
-    if (ev[i] >= 0) atomicAdd(&mine[ev[i]], 1);
-  __syncthreads();
-  // thread e owns expert e: prefix over the waves, then over the experts
-  int total = 0;
-  if (tid < E)
-    for (int w = 0; w < kSortWaves; ++w) {
-      const int c = table[w * E + tid];
-      table[w * E + tid] = total;
-      total += c;
+  // thread e owns expert e: prefix over the experts, then over the waves
+  int before = 0, total = 0;
+  if (tid < E) {
+    for (int c = 0; c < kPlaceCopies; ++c) {
+      before += count[c * E + tid];
+      total += count[(kPlaceCopies + c) * E + tid];
     }
+    total += before;
+    for (int w = 0; w < kPlaceWaves; ++w) total += cursor[w * E + tid];
+  }
   int incl = total;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -279,35 +301,89 @@ __global__ void __launch_bounds__(64 * kSortWaves) moe_sort_small_kernel(const i
   int base = 0;
   for (int w = 0; w < wave; ++w) base += part[w];
   if (tid < E) {
-    offs[tid] = base + incl;
-    for (int w = 0; w < kSortWaves; ++w) table[w * E + tid] += base + incl - total;
+    if (write_offs) offs[tid] = base + incl;
+    int at = base + incl - total + before;
+    for (int w = 0; w < kPlaceWaves; ++w) {
+      const int c = cursor[w * E + tid];
+      cursor[w * E + tid] = at;
+      at += c;
+    }
   }
   __syncthreads();
+  const bool live = expert >= 0;
   const int bits = E > 1 ? 32 - __clz(E - 1) : 0;
-  const uint64_t lower = (uint64_t(1) << lane) - 1;
-#pragma unroll
-  for (int i = 0; i < kRounds; ++i) {
-    const int s = s0 + 64 * i + lane, e = ev[i];
-    const bool live = e >= 0;
-    uint64_t same = __ballot(live);
-    if (same == 0) break;   // uniform over the wave: its slots have run out
-    for (int bit = 0; bit < bits; ++bit) {
-      const bool on = (e >> bit) & 1;
-      const uint64_t with_bit = __ballot(on && live);
-      same &= on ? with_bit : ~with_bit;
-    }
-    const int before = __popcll(same & lower), count = __popcll(same);
-    const int row = live ? mine[e] + before : 0;
-    asm volatile("" ::: "memory");   // the wave's LDS accesses complete in order; the compiler must keep it
-    __builtin_amdgcn_wave_barrier();
-    if (live) {
-      if (before == count - 1) mine[e] = row + 1;
-      row_token[row] = s / k;
-      token_rows[s] = row;
-    }
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
+  uint64_t same = __ballot(live);
+  for (int bit = 0; bit < bits; ++bit) {
+    const bool on = (expert >> bit) & 1;
+    const uint64_t with_bit = __ballot(on && live);
+    same &= on ? with_bit : ~with_bit;
   }
+  if (live) {
+    const int row = cursor[wave * E + expert] + __popcll(same & ((uint64_t(1) << lane) - 1));
+    row_token[row] = (s0 + tid) / k;
+    token_rows[s0 + tid] = row;
+  }
+}
+
+__global__ void __launch_bounds__(kPlaceBlock) moe_place_kernel(const int32_t* __restrict__ slot_expert, int slots, int E, int k,
+                                                                int32_t* __restrict__ offs, int32_t* __restrict__ row_token,
+                                                                int32_t* __restrict__ token_rows) {
+  __shared__ int32_t count[kPlaceRows * kMaxExperts];
+  __shared__ int32_t part[kPlaceWaves];
+  const int tid = threadIdx.x, copy = (tid >> 6) & (kPlaceCopies - 1), own = blockIdx.x;
+  const int expert = own * kPlaceBlock + tid < slots ? slot_expert[own * kPlaceBlock + tid] : -1;
+  for (int i = tid; i < kPlaceRows * E; i += kPlaceBlock) count[i] = 0;
+  __syncthreads();
+  const int blocks = gridDim.x;
+  for (int b0 = 0; b0 < blocks; b0 += 8) {
+    int e[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int s = (b0 + i) * kPlaceBlock + tid;
+      e[i] = b0 + i != own && s < slots ? slot_expert[s] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (e[i] >= 0) atomicAdd(&count[(b0 + i < own ? copy : kPlaceCopies + copy) * E + e[i]], 1);
+  }
+  moe_place(count, part, expert, own * kPlaceBlock, E, k, own == 0, offs, row_token, token_rows);
+}
+
+// The whole routing of a decoding step, one launch: 16 tokens at a time, one to a wave, the next one's logits on their way while
+// one chooses.  Worth it while no wave makes more than kRouteChoices choices beyond its first token's: a choice takes 0.28 us,
+// the second launch 3 us.  1 token, 8 of 128 experts 8.9 -> 5.0 us, 32 tokens, 2 of 8 6.9 -> 4.8; 64 tokens, 8 of 128 13.6 (24
+// choices more) against 7.7 in two launches.
+constexpr int kRouteChoices = 8;
+bool route_in_one(int64_t tokens, int64_t top_k) {
+  return tokens * top_k <= kPlaceBlock && ((tokens + kPlaceWaves - 1) / kPlaceWaves - 1) * top_k <= kRouteChoices;
+}
+
+template <typename T, int kPer>
+__global__ void __launch_bounds__(kPlaceBlock) moe_route_kernel(const T* __restrict__ logits, int64_t ld, int tokens, int E, int k, int renorm,
+                                                                int32_t* __restrict__ offs, int32_t* __restrict__ slot_expert,
+                                                                float* __restrict__ slot_weight, int32_t* __restrict__ row_token,
+                                                                int32_t* __restrict__ token_rows) {
+  __shared__ int32_t count[kPlaceRows * kMaxExperts];
+  __shared__ int32_t part[kPlaceWaves];
+  __shared__ int32_t chosen[kPlaceBlock];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  MoeTopk<T, kPer> next;
+  if (wave < tokens) next.load(logits + int64_t(wave) * ld, E, lane);
+  for (int i = tid; i < kPlaceRows * E; i += kPlaceBlock) count[i] = 0;
+  for (int t = wave; t < tokens; t += kPlaceWaves) {
+    const MoeTopk<T, kPer> token = next;
+    if (t + kPlaceWaves < tokens) next.load(logits + int64_t(t + kPlaceWaves) * ld, E, lane);
+    int e;
+    float weight;
+    token.choose(E, k, renorm, lane, e, weight);
+    if (lane < k) {
+      chosen[t * k + lane] = e;
+      slot_expert[t * k + lane] = e;
+      slot_weight[t * k + lane] = weight;
+    }
+  }
+  __syncthreads();
+  moe_place(count, part, tid < tokens * k ? chosen[tid] : -1, 0, E, k, true, offs, row_token, token_rows);
 }
 
 // ---------------------------------------------------------------- activation
@@ -397,21 +473,30 @@ int route_checked(const void* logits, int64_t ld, int dtype, int64_t tokens, int
   if (size_t(pl.nb) * size_t(E) * sizeof(int32_t) > table_bytes) return GMM_ERR_WORKSPACE;
   if (pl.nb > 0 && !table) return GMM_ERR_BAD_ARGUMENT;
   if (tokens > 0) {
-    const dim3 grid(unsigned((tokens + 3) / 4)), block(256);
-    if (dtype == GMM_DT_BF16)
-      hipLaunchKernelGGL(moe_topk_kernel<Bf16>, grid, block, 0, stream, static_cast<const Bf16*>(logits), ld, int(tokens), int(E),
-                         int(top_k), renorm, slot_expert, slot_weight);
-    else if (dtype == GMM_DT_F16)
-      hipLaunchKernelGGL(moe_topk_kernel<F16>, grid, block, 0, stream, static_cast<const F16*>(logits), ld, int(tokens), int(E),
-                         int(top_k), renorm, slot_expert, slot_weight);
-    else
-      hipLaunchKernelGGL(moe_topk_kernel<float>, grid, block, 0, stream, static_cast<const float*>(logits), ld, int(tokens), int(E),
-                         int(top_k), renorm, slot_expert, slot_weight);
-    if (pl.slots <= kSmallSlots) {
-      hipLaunchKernelGGL(moe_sort_small_kernel, dim3(1), dim3(64 * kSortWaves), 0, stream, slot_expert, pl.slots, int(E), int(top_k),
-                         offs, row_token, token_rows);
-      return hipGetLastError() == hipSuccess ? GMM_OK : GMM_ERR_LAUNCH;
-    }
+    const bool one = route_in_one(tokens, top_k);
+    const auto launch = [&](const auto* rows, auto per) {
+      using T = std::remove_const_t<std::remove_pointer_t<decltype(rows)>>;
+      constexpr int kPer = decltype(per)::value;
+      if (one)
+        hipLaunchKernelGGL((moe_route_kernel<T, kPer>), dim3(1), dim3(kPlaceBlock), 0, stream, rows, ld, int(tokens), int(E), int(top_k),
+                           renorm, offs, slot_expert, slot_weight, row_token, token_rows);
+      else
+        hipLaunchKernelGGL((moe_topk_kernel<T, kPer>), dim3(unsigned((tokens + 3) / 4)), dim3(256), 0, stream, rows, ld, int(tokens),
+                           int(E), int(top_k), renorm, slot_expert, slot_weight);
+    };
+    const auto topk = [&](const auto* rows) {
+      if (E <= 64) launch(rows, std::integral_constant<int, 1>{});
+      else if (E <= 128) launch(rows, std::integral_constant<int, 2>{});
+      else if (E <= 256) launch(rows, std::integral_constant<int, 4>{});
+      else launch(rows, std::integral_constant<int, 16>{});
+    };
+    if (dtype == GMM_DT_BF16) topk(static_cast<const Bf16*>(logits));
+    else if (dtype == GMM_DT_F16) topk(static_cast<const F16*>(logits));
+    else topk(static_cast<const float*>(logits));
+    if (!one && pl.slots <= kPlaceSlots)
+      hipLaunchKernelGGL(moe_place_kernel, dim3((pl.slots + kPlaceBlock - 1) / kPlaceBlock), dim3(kPlaceBlock), 0, stream, slot_expert,
+                         pl.slots, int(E), int(top_k), offs, row_token, token_rows);
+    if (one || pl.slots <= kPlaceSlots) return hipGetLastError() == hipSuccess ? GMM_OK : GMM_ERR_LAUNCH;
     hipLaunchKernelGGL(moe_hist_kernel, dim3(pl.nb), dim3(256), 0, stream, slot_expert, pl.slots, pl.spb, int(E), table);
   }
   hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(1024), 0, stream, table, pl.nb, int(E), offs);

@@ -190,8 +190,8 @@ int gmm_3d2d(const void* a, const void* b, void* out, const int32_t* offs, int32
  *   token_rows  int32[tokens * top_k]   the row of each slot (inverse of the sort)
  * experts <= 1023, top_k <= min(experts, 32), tokens * top_k < 2^31.  `workspace` is device memory of at
  * least gmm_moe_route_workspace_bytes(...) bytes (per-workgroup expert histograms; contents need not be
- * initialised); too small a workspace returns GMM_ERR_WORKSPACE.  Two launches on `stream` for up to 4096 slots, four for
- * more; no host sync. */
+ * initialised); too small a workspace returns GMM_ERR_WORKSPACE.  One launch on `stream` for a few
+ * tokens, two for up to 131072 slots, four for more (the workspace is theirs); no host sync. */
 int64_t gmm_moe_route_workspace_bytes(int64_t tokens, int64_t experts, int64_t top_k);
 int gmm_moe_route(const void* logits, int64_t logits_stride, int32_t logits_dtype,
                   int64_t tokens, int64_t experts, int64_t top_k, int32_t renormalize,
@@ -204,8 +204,8 @@ int gmm_moe_route(const void* logits, int64_t logits_stride, int32_t logits_dtyp
  * loops, harnesses that forbid hipMalloc).  The histogram table lives in a 256 KiB array that the library
  * holds on every GPU it runs on until the process ends; the call allocates nothing.  Problems whose
  * gmm_moe_route_workspace_bytes(...) exceeds 262144 bytes are refused with GMM_ERR_WORKSPACE (any problem
- * with experts <= 256 fits; with 1023 experts up to 65536 slots).  All calls on one GPU share that array:
- * calls that may overlap on one GPU (different streams, different threads) race and must be serialised by
+ * with experts <= 256 fits; with 1023 experts up to 65536 slots).  All calls on one GPU with more than 131072
+ * slots share that array: such calls that may overlap on one GPU (different streams, different threads) race and must be serialised by
  * the caller.  The first call on a device looks the array's device address up (hipGetSymbolAddress, no
  * allocation): make that first call outside a stream capture -- one eager call per device at start-up is
  * enough -- and every later call, captured or not, only launches.  Outputs and everything else as

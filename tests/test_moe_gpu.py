@@ -48,11 +48,25 @@ def test_routing_matches_the_oracle(T, E, k, dtype):
 @pytest.mark.parametrize("T,E,k", [(1, 1, 1), (4096, 3, 1), (4097, 3, 1), (128, 1023, 32), (129, 1023, 32), (585, 65, 7),
                                    (16, 128, 4), (1025, 64, 2)])
 def test_slots_at_the_edges_of_the_one_workgroup_sort(T, E, k):
-    """Up to 4096 slots one workgroup of 16 waves sorts, 64 slots of a wave at a time; above, one workgroup per 1024 slots."""
+    """A workgroup of 16 waves places 1024 slots, 64 to a wave."""
     gen = torch.Generator().manual_seed(T + E + k)
     logits = torch.randn(T, E, generator=gen)
     logits[:, 0] += 2.0
     check_routing(moe.moe_route(logits.to(DEV), k), moe_oracle.route(logits, k, True))
+
+
+@pytest.mark.parametrize("T,E,k", [(16, 64, 8), (17, 65, 8), (32, 128, 8), (33, 129, 8), (144, 5, 1), (145, 5, 1), (32, 1023, 32), (16, 256, 32),
+                                   (80, 257, 2), (81, 1023, 2), (1023, 9, 1), (341, 9, 3), (1024, 7, 1), (1025, 7, 1), (131072, 5, 1),
+                                   (131073, 5, 1)])
+def test_routing_at_the_edges_of_its_kernels(T, E, k):
+    """One launch while no wave chooses more than eight times beyond its first token, then 1024 slots to a workgroup, from
+    131073 slots on a table of counts; 64, 128 and 256 experts to a lane's registers.  Ties and masked experts among them."""
+    gen = torch.Generator().manual_seed(T + E + k)
+    logits = torch.randn(T, E, generator=gen).round(decimals=1)
+    logits[:, 0] += 1.0
+    logits[T // 2, E // 2:] = float("-inf")
+    for renorm in (True, False):
+        check_routing(moe.moe_route(logits.to(DEV), k, renormalize=renorm), moe_oracle.route(logits, k, renorm))
 
 
 def test_routing_fp16_skewed_padded_and_empty():
