@@ -438,7 +438,6 @@ static int64_t host_tile_list23(const int32_t* offs_host, int32_t G, int32_t jag
     group_major = 1;   // every group's tall tiles, then its remainder tiles
     xcd_remap = 0;     // the tickets of an XCD are neighbours already
   }
-  bool any_tall = false;
   std::vector<int32_t> ct(size_t(G) + 1, 0), cs(size_t(G) + 1, 0);
   for (int i = 0; i < G; ++i) {
     const int g = order[i];
@@ -446,12 +445,10 @@ static int64_t host_tile_list23(const int32_t* offs_host, int32_t G, int32_t jag
     if (jagged != GMM_JAG_NONE) gmm_group_range(offs_host, g, extent, lo, hi);
     gmm_split_rows(gmm_group_rows(jagged, lo, hi, M, align), tall, shrt, n_tall, n_short, rem_rows);
     const int tn = gmm_group_tile_cols(jagged, lo, hi, N, align, tile_n);
-    any_tall = any_tall || n_tall * tn > 0;
     ct[i + 1] = ct[i] + n_tall * tn + (group_major ? n_short * tn : 0);
     cs[i + 1] = cs[i] + (group_major ? 0 : n_short * tn);
   }
   const int total_tall = ct[G], total_tiles = ct[G] + cs[G];
-  if (!gmm_renumbered(any_tall, N)) xcd_remap = 0;
   // the split of the last round, as gmm_asm_kernel decides it
   const int nk = gmm_cdiv(K, 64);
   int nparts = 1, tail = 0;

@@ -147,17 +147,16 @@ __device__ __forceinline__ void gmm_scan_table(int32_t* cum) {
 
 // Returns the total number of tiles; total_tall gets the number of tall ones (they come first in the launch
 // order: the workgroups of all XCDs then work on tiles of one height in every round and stay in step, which
-// keeps the operand panels they share in the Infinity Cache).  any_tall: is there a tall tile at all?
+// keeps the operand panels they share in the Infinity Cache).
 template <int NT>
 __device__ __forceinline__ int gmm_build_tile_table2(const GmmParams& p, int bn, int32_t* cum_tall, int32_t* cum_short,
-                                                     int& total_tall, bool& any_tall) {
+                                                     int& total_tall) {
   const int tid = threadIdx.x;
   if (p.jag == GMM_JAG_NONE) {
     const int tn = gmm_cdiv(p.N, bn);
     int n_tall, n_short, rem_rows;
     gmm_split_rows(p.M, p.tall, p.shrt, n_tall, n_short, rem_rows);
     total_tall = p.G * n_tall * tn;
-    any_tall = n_tall > 0;
     return total_tall + p.G * n_short * tn;
   }
   const int extent = p.jag == GMM_JAG_M ? p.M : (p.jag == GMM_JAG_N ? p.N : p.K);
@@ -172,7 +171,7 @@ __device__ __forceinline__ int gmm_build_tile_table2(const GmmParams& p, int bn,
       cs = n_short * tn;
     }
     cum_tall[g + 1] = p.group_major ? ct + cs : ct;
-    cum_short[g + 1] = p.group_major ? ct : cs;
+    cum_short[g + 1] = p.group_major ? 0 : cs;
   }
   if (tid == 0) { cum_tall[0] = 0; cum_short[0] = 0; }
   __syncthreads();
@@ -180,12 +179,7 @@ __device__ __forceinline__ int gmm_build_tile_table2(const GmmParams& p, int bn,
   gmm_scan_table<NT>(cum_short);
   __syncthreads();
   total_tall = cum_tall[p.G];
-  if (p.group_major) {   // everything is in the first table, the second counts the tall tiles
-    any_tall = cum_short[p.G] > 0;
-    return total_tall;
-  }
-  any_tall = total_tall > 0;
-  return total_tall + cum_short[p.G];
+  return total_tall + cum_short[p.G];   // group-major order: everything is in the first table
 }
 
 // Tile id -> tile, per lane (ids differ between lanes).

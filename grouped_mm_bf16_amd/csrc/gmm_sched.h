@@ -179,13 +179,6 @@ GMM_HD int gmm_xcd_remap(int t, int total, int num_wg) {
   return base + start + (r >> 3);
 }
 
-// Launches that are renumbered.  Without a tall tile (decoding: every group is one row of tiles) there is nothing worth an
-// L2, the second operand is read once.  If a group's row of tiles is at least an XCD's share of a round, the chip then reads
-// 128 KB that lie side by side in memory in launch order, and eight times 16 KB renumbered: 8 groups of 4096 x 28672, 64 rows
-// in all, 303 -> 290 us (6.5 TB/s; plain reads of such pieces 6.3 and 6.0).  Narrower groups: 128 of 2048 x 1536, 512 rows,
-// a decoding step with them 201.8 us in launch order, 200.4 renumbered.
-GMM_HD bool gmm_renumbered(bool any_tall, int N) { return any_tall || N < 32 * 256; }
-
 // Group that holds linear tile id t, given the exclusive prefix sum cum[0..G]:
 // the g with cum[g] <= t < cum[g + 1] (empty groups are skipped by construction).
 GMM_HD int gmm_find_group(const int32_t* cum, int G, int t) {

@@ -175,6 +175,28 @@ def test_small_groups_on_every_tile_height(K, N, b_col, tall, shrt):
     assert K_.last_kernel() == ("any" if (tall, K) == (-1, 72) else "assembly")
 
 
+@pytest.mark.parametrize("sizes,N,K", [([8] * 8, 12288, 1024), ([30, 0, 1, 33, 64, 0, 3, 125], 12288, 1024), ([64] * 2, 28672, 1032),
+                                       ([8] * 8, 12280, 1024), ([8] * 8, 12288, 1016)])
+def test_launch_order_of_wide_decoding_products(sizes, N, K):
+    """Both sides of the line between launches in order and renumbered ones: the same bits."""
+    gen = torch.Generator(device=DEV).manual_seed(N + K)
+    a = torch.randn(sum(sizes), K, device=DEV, generator=gen).bfloat16()
+    b = torch.randn(len(sizes), K, N, device=DEV, generator=gen).bfloat16()
+    outs = []
+    for remap in (1, 0):
+        prev = K_._lib.load().gmm_set_xcd_remap(remap)
+        try:
+            outs.append(torch.full((sum(sizes), N), float("nan"), device=DEV, dtype=torch.bfloat16))
+            with K_.tail_split(False):
+                K_.grouped_mm_2d3d(a, b, offs_of(sizes).to(DEV), outs[-1])
+        finally:
+            K_._lib.load().gmm_set_xcd_remap(prev)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    g = len(sizes) - 1
+    lo = sum(sizes[:g])
+    oracle.assert_close(outs[0][lo:, :512].cpu(), (a[lo:].float() @ b[g, :, :512].float()).bfloat16().cpu(), K)
+
+
 def test_output_larger_than_4_gib():
     """70000 x 32768 bf16 output (4.6 GB): every tile's address arithmetic must be 64-bit up to the tile's
     origin.  Rows on both sides of the 2 GiB and 4 GiB marks and of the group boundaries against the oracle."""

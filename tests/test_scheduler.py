@@ -397,16 +397,3 @@ def test_jagged_contraction_order_of_lengths_beyond_22_bits():
     shift = max(0, sum(sizes).bit_length() - 22)
     keys = [sizes[g] >> shift for g in order]
     assert keys == sorted(keys, reverse=True)
-
-
-def test_launches_without_a_tall_tile_keep_launch_order():
-    """One wide row of tiles per group, whatever its height: the renumbering for the XCDs stays out; a tall tile or narrower
-    groups bring it back."""
-    def launch(sizes, remap, N=28672):
-        return tile_list2(sizes, ROWS, sum(sizes), N, 4096, 256, 64, remap=remap)
-
-    for sizes in ([64] * 8, [1, 0, 63, 17] * 20):
-        assert (launch(sizes, 1) == launch(sizes, 0)).all()
-    assert (launch([256] + [64] * 8, 1) != launch([256] + [64] * 8, 0)).any()
-    for N, plain in ((8192, True), (8184, False)):
-        assert (launch([64] * 40, 1, N) == launch([64] * 40, 0, N)).all() == plain
