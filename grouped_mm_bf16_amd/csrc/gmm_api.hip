@@ -155,6 +155,10 @@ int run(Problem& pr, hipStream_t stream) {
     // 2048 x 4096 with 256 rows 148 / 160, 8 of 4096 x 28672 with 128 rows 304 / 317; smaller matrices: 128 groups of 2048 x
     // 1536 with 512 rows 118 / 114, 8 of 1024 x 8192 with 128 rows 34.0 / 29.9; more rows: 16 of 2048 x 8192, 2048 rows 159 / 157.
     if (int64_t(p.M) <= 64 * int64_t(p.G) && p.K >= 2048 && int64_t(p.K) * p.N >= (int64_t(1) << 23)) return GMM_ERR_UNSUPPORTED;
+    // few tiles: the product alone is cut along K (2 rows of 8 groups, 4096 x 2048: 42 us with the activation, 53 in this kernel)
+    GmmParams product = with_full_workspace(p, cus);
+    product.act = 0;
+    if (gmm_staged_cut_preferred(product, cus)) return GMM_ERR_UNSUPPORTED;
   }
   if (p.gather) {
     // the assembly tile gathers rows of a K-contiguous first operand whose byte offsets fit 31 bits; the

@@ -13,6 +13,8 @@ int gmm_launch_generic(GmmParams p, int in_dtype, int out_dtype, int num_cus, hi
 bool gmm_staged_eligible(const GmmParams& p);
 // Of the 16-bit products that the assembly tile could take: true for those that the register-staged kernel runs faster.
 bool gmm_staged_preferred(const GmmParams& p, int num_cus);
+// Those among them that are cut along K for it (needs a workspace).
+bool gmm_staged_cut_preferred(const GmmParams& p, int num_cus);
 // Of the products without alignment: true for those that the element-wise kernel runs faster.
 bool gmm_element_preferred(const GmmParams& p, int in_dtype, int num_cus);
 int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream);

@@ -64,6 +64,8 @@ struct GmmParams {
   // Register-staged kernel, jagged contraction: elements of K per part of a group (gmm_group_parts) and the most parts
   // that the workspace has room for; 0: no group is cut.
   int32_t k_chunk, k_parts;
+  // Register-staged kernel, any other product: the most parts that a tile is cut into along K.
+  int32_t k_split;
 };
 
 constexpr int GMM_WS_HEADER = 4096;          // 1024 int32: arrival counters, one per tile of the split round, ...

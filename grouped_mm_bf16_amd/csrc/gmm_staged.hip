@@ -113,7 +113,7 @@ struct Stage {
 
   // base: element (row 0, k 0) of the group's operand; the tile's rows start at row0; `ext` rows exist.
   __device__ __forceinline__ void init(const T* base, int64_t ld, int row0, int ext, int k_lo, int k_hi, int k_ext,
-                                       const GmmParams* gather, int gather_end) {
+                                       const int32_t* gather, int gather_end, int src_rows) {
     const int tid = threadIdx.x;
     zero_rows = 0;
     const int whole = (k_hi - k_lo) / Im::BK;          // K tiles that lie inside the range
@@ -123,13 +123,13 @@ struct Stage {
         const int q = i * NT + tid, row = q >> 3, c = q & 7;
         int src = gmm_min(row0 + row, ext - 1);
         if (gather) {
-          src = row0 + row < gather_end ? gmm_gather_row(*gather, row0 + row) : -1;
-          if (src < 0) { zero_rows |= 1 << i; src = 0; }
+          src = row0 + row < gather_end ? gather[row0 + row] : -1;
+          if (src < 0 || src >= src_rows) { zero_rows |= 1 << i; src = 0; }
         }
         ptr[i] = base + int64_t(src) * ld + k_lo + c * EPC;
       }
       any_zero = gather ? __ballot(zero_rows != 0) != 0 : 0;
-      last = base + int64_t((gather ? gather->a_rows : ext) - 1) * ld + k_ext - EPC;
+      last = base + int64_t((gather ? src_rows : ext) - 1) * ld + k_ext - EPC;
       step = Im::BK;
       n_fast = whole;
     } else {
@@ -348,8 +348,8 @@ __device__ __forceinline__ bool join_parts(const GmmParams& p, const GmmTile& ti
   return true;
 }
 
-// SPLIT: a jagged contraction whose groups may be cut along K.
-template <typename T, typename OutT, bool A_TR, bool B_TR, int EDGE, bool SPLIT>
+// SPLIT = 1: a jagged contraction whose groups may be cut along K.  SPLIT = 2: any other product, few tiles cut along K.
+template <typename T, typename OutT, bool A_TR, bool B_TR, int EDGE, int SPLIT>
 __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const GmmParams p) {
   constexpr int BM = EDGE, BN = EDGE;
   constexpr int AHEAD = sizeof(T) == 4 ? 2 : 1;   // K tiles fetched ahead (see the top of the file)
@@ -371,12 +371,16 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
   const int64_t lda = A_TR ? p.a_sk : p.a_sm, ldb = B_TR ? p.b_sk : p.b_sn;
   const bool in_registers = p.jag != GMM_JAG_NONE && p.G <= 64;
   GmmWaveGroups groups{0, 0, 0, 0};
-  int chunk = SPLIT ? p.k_chunk : 0;
+  int chunk = SPLIT == 1 ? p.k_chunk : 0;
   auto build = [&]() {
     return __builtin_amdgcn_readfirstlane(in_registers ? groups.build(p, BM, BN, chunk) : gmm_build_tile_table<NT>(p, BM, BN, cum, chunk));
   };
   int total = build();
-  if (SPLIT && chunk && total > p.k_parts) {   // offsets that overlap: more parts than K elements have room for
+  // few tiles: each in as many parts as there are workgroups for
+  const int tiles = gmm_max(total, 1);
+  const int split = SPLIT == 2 ? gmm_max(gmm_min(p.k_split, gmm_min(int(gridDim.x), p.k_parts) / tiles), 1) : 1;
+  if (SPLIT == 2) total *= split;
+  if (SPLIT == 1 && chunk && total > p.k_parts) {   // offsets that overlap: more parts than K elements have room for
     chunk = 0;
     __syncthreads();
     total = build();
@@ -385,10 +389,16 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
   for (int t = blockIdx.x; t < total; t += gridDim.x) {
     const int id = gmm_xcd_remap(t, total, gridDim.x);
     int g, local, lo, hi;
-    if (in_registers) groups.find(id, g, local, lo, hi);
-    else gmm_find_tile(p, cum, id, BM, BN, g, local, lo, hi);
-    int part = 0, parts = 1, per = 1;
-    if constexpr (SPLIT) {
+    int part = 0, parts = 1, per = 1, number = id;
+    if (SPLIT == 2) {
+      per = tiles;
+      parts = split;
+      part = id / tiles;
+      number = id - part * tiles;
+    }
+    if (in_registers) groups.find(number, g, local, lo, hi);
+    else gmm_find_tile(p, cum, number, BM, BN, g, local, lo, hi);
+    if (SPLIT == 1) {
       parts = gmm_group_parts(hi - lo, chunk);
       per = gmm_cdiv(p.M, BM) * gmm_cdiv(p.N, BN);
       part = local / per;
@@ -396,10 +406,11 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
     }
     GmmTile tile = gmm_tile_of_group(p, g, local, lo, hi, BM, BN);
     if (SPLIT && parts > 1) {
+      const int k_lo = tile.k_lo, k_hi = tile.k_hi;
       int first, last;
-      gmm_part_ktiles(gmm_cdiv(hi - lo, BK), parts, part, first, last);
-      tile.k_lo = lo + first * BK;
-      tile.k_hi = gmm_min(lo + last * BK, hi);
+      gmm_part_ktiles(gmm_cdiv(k_hi - k_lo, BK), parts, part, first, last);
+      tile.k_lo = k_lo + first * BK;
+      tile.k_hi = gmm_min(k_lo + last * BK, k_hi);
     }
     const T* a = static_cast<const T*>(p.a) + int64_t(tile.g) * p.a_sg;
     const T* b = static_cast<const T*>(p.b) + int64_t(tile.g) * p.b_sg;
@@ -415,8 +426,8 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
     if (klen > 0) {
       Stage<T, A_TR, BM> sa;
       Stage<T, B_TR, BN> sb;
-      sa.init(a, lda, tile.m0, p.M, tile.k_lo, tile.k_hi, p.K, SPLIT || !p.gather ? nullptr : &p, tile.m_hi);
-      sb.init(b, ldb, tile.n0, p.N, tile.k_lo, tile.k_hi, p.K, nullptr, 0);
+      sa.init(a, lda, tile.m0, p.M, tile.k_lo, tile.k_hi, p.K, SPLIT == 1 ? nullptr : p.gather, tile.m_hi, p.a_rows);
+      sb.init(b, ldb, tile.n0, p.N, tile.k_lo, tile.k_hi, p.K, nullptr, 0, 0);
       const int n_fast = gmm_min(sa.n_fast, sb.n_fast), nk = (klen + BK - 1) / BK;
       // K tile t + 1 .. t + AHEAD are on their way in registers while K tile t is multiplied
       uint4 ra[AHEAD][sa.NCH], rb[AHEAD][sb.NCH];
@@ -520,7 +531,7 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
   }
 }
 
-template <typename T, typename OutT, int EDGE, bool SPLIT>
+template <typename T, typename OutT, int EDGE, int SPLIT>
 int launch_layout(const GmmParams& p, bool a_tr, bool b_tr, hipStream_t stream) {
   const dim3 grid(p.num_wg), block(NT);
   if (a_tr && b_tr)
@@ -532,6 +543,22 @@ int launch_layout(const GmmParams& p, bool a_tr, bool b_tr, hipStream_t stream) 
   else
     hipLaunchKernelGGL((gmm_staged_kernel<T, OutT, false, false, EDGE, SPLIT>), grid, block, 0, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+// Tiles of a launch with square tiles of `edge`, the group boundaries taken to cut half a tile each on average.
+int64_t expected_tiles(const GmmParams& p, int edge) {
+  const int64_t tm = (p.M + edge - 1) / edge, tn = (p.N + edge - 1) / edge;
+  if (p.jag == GMM_JAG_M) return (p.M / edge + (p.G + 1) / 2) * tn;
+  if (p.jag == GMM_JAG_N) return tm * (p.N / edge + (p.G + 1) / 2);
+  return p.G * tm * tn;
+}
+
+// The same if every group boundary cuts a whole tile more.
+int64_t most_tiles(const GmmParams& p, int edge) {
+  const int64_t tm = (p.M + edge - 1) / edge, tn = (p.N + edge - 1) / edge;
+  if (p.jag == GMM_JAG_M) return (p.M / edge + (p.G < p.M ? p.G : p.M)) * tn;
+  if (p.jag == GMM_JAG_N) return tm * (p.N / edge + (p.G < p.N ? p.G : p.N));
+  return p.G * tm * tn;
 }
 
 // Cut the groups of a jagged contraction along K?  A group longer than a chunk is cut into even parts of up to a chunk (more
@@ -556,31 +583,46 @@ int64_t cut_contraction(GmmParams& p, int64_t most_wgs) {
   return entries;
 }
 
+// Rows of a group on average: the tiles of one are full, the other's mostly hold rows that do not exist.
+bool full_rows(const GmmParams& p) { return p.jag == GMM_JAG_M ? int64_t(p.M) >= 96 * int64_t(p.G) : p.M >= 96; }
+
+// Cut the tiles of any other product along K?  A launch of few tiles with a long contraction leaves most of the chip idle and
+// takes as long as one tile: each is cut into as many parts as there are workgroups for (the device knows the number of tiles),
+// of at least GMM_K_SPLIT_MIN elements, joined like those of a jagged contraction.  Joining costs 8 to 12 us.  us, whole / cut:
+// 16 rows, 8 groups of 4001 x 2047 112 / 47; 3 x 4 tiles of 331 x 517 x 4099, four products 86 / 40; fp32 500 x 500 x 8000, two
+// 173 / 92.  Over 350 random launches of up to half the workgroups 2.3 (16-bit) and 2.1 (fp32) times as fast; the line leaves
+// out what lost there or at sizes that fit the tiles exactly: K up to 1024 (two products of 512 x 1024 x 1024 17 / 22), more
+// than 64 full tiles with a first operand contiguous along M up to 2048 (0.97), more than 80 fp32 tiles up to 3072 (0.9 to 1.4).
+constexpr int GMM_K_SPLIT_MIN = 256;
+template <int EDGE>
+bool split_tiles(GmmParams& p, int64_t most_wgs) {
+  p.k_split = 0;
+  if (p.jag == GMM_JAG_K || p.ws_parts <= 0) return false;
+  const int64_t tiles = most_tiles(p, EDGE);
+  int64_t room = int64_t(p.ws_parts) * GMM_WS_SLOT / (EDGE * EDGE * 4);
+  if (room > GMM_WS_TICKET) room = GMM_WS_TICKET;
+  if (tiles > 256 || 2 * tiles > most_wgs || 2 * tiles > room) return false;
+  int least = 1024;
+  if (EDGE == 64 && tiles > 80) least = 3072;
+  if (EDGE == 128 && tiles > 128) least = 1536;
+  if (EDGE == 128 && tiles > 64 && p.a_sk != 1 && full_rows(p)) least = 2048;
+  if (p.K <= least) return false;
+  p.k_split = int32_t(p.K / GMM_K_SPLIT_MIN < GMM_K_PARTS_MAX ? p.K / GMM_K_SPLIT_MIN : GMM_K_PARTS_MAX);
+  p.k_parts = int32_t(room);
+  return true;
+}
+
 template <typename T, typename OutT, int EDGE>
 int launch_layout(GmmParams p, bool a_tr, bool b_tr, int num_cus, hipStream_t stream) {
   const int64_t most = int64_t(tile_wgs(EDGE)) * num_cus;
   int64_t bound = cut_contraction<EDGE>(p, most);
   if (bound == 0) bound = gmm_tile_bound(p.jag, p.G, p.M, p.N, EDGE, EDGE);
+  const bool split = split_tiles<EDGE>(p, most);
+  if (split) bound = gmm_tile_bound(p.jag, p.G, p.M, p.N, EDGE, EDGE) * p.k_split;
   const int64_t want = (bound + 7) / 8 * 8;
   p.num_wg = int(want < most ? (want < 8 ? 8 : want) : most);
-  return p.k_chunk ? launch_layout<T, OutT, EDGE, true>(p, a_tr, b_tr, stream)
-                   : launch_layout<T, OutT, EDGE, false>(p, a_tr, b_tr, stream);
-}
-
-// Tiles of a launch with square tiles of `edge`, the group boundaries taken to cut half a tile each on average.
-int64_t expected_tiles(const GmmParams& p, int edge) {
-  const int64_t tm = (p.M + edge - 1) / edge, tn = (p.N + edge - 1) / edge;
-  if (p.jag == GMM_JAG_M) return (p.M / edge + (p.G + 1) / 2) * tn;
-  if (p.jag == GMM_JAG_N) return tm * (p.N / edge + (p.G + 1) / 2);
-  return p.G * tm * tn;
-}
-
-// The same if every group boundary cuts a whole tile more.
-int64_t most_tiles(const GmmParams& p, int edge) {
-  const int64_t tm = (p.M + edge - 1) / edge, tn = (p.N + edge - 1) / edge;
-  if (p.jag == GMM_JAG_M) return (p.M / edge + (p.G < p.M ? p.G : p.M)) * tn;
-  if (p.jag == GMM_JAG_N) return tm * (p.N / edge + (p.G < p.N ? p.G : p.N));
-  return p.G * tm * tn;
+  if (split) return launch_layout<T, OutT, EDGE, 2>(p, a_tr, b_tr, stream);
+  return p.k_chunk ? launch_layout<T, OutT, EDGE, 1>(p, a_tr, b_tr, stream) : launch_layout<T, OutT, EDGE, 0>(p, a_tr, b_tr, stream);
 }
 
 // fp32: 64 x 64 tiles (four workgroups per CU) or 128 x 128 (two)?  A launch takes whole rounds of its grid, and a
@@ -610,6 +652,11 @@ bool small_tiles(const GmmParams& p, int in_dtype, int num_cus) {
 //   than its 64-row tile fill half a tile here (750 tiles of 264 x 424 x 1264 in 73 groups 26 / 29).
 //   A contiguous along M: the assembly tile always has 256 rows.  1256 x 824 x 456 in 11 groups 32 / 21; 1392 x 1312 x
 //   352 in 40 groups 47 / 37; 2160 tiles of 1880 x 144 x 1120 35 / 37.  It wins once there are rounds to fill.
+//   Few tiles, K past 1024: cut along K (split_tiles).  The assembly tile cuts its own tiles from K = 4096 on, into longer
+//   parts.  us, assembly tile / here: one row each of 8 groups of 2048 x 1536 30 / 20; 8 products of 64 x 1024 x 4096 49 / 29;
+//   512 rows, 8 groups of 4096 x 1024 57 / 31; A contiguous along M, two products of 1024 x 1024 x 8192 89 / 58.  Full tiles want
+//   more K or fewer of them (two products of 1024 x 1024 x 2048 26 / 32).  Random launches, ragged sizes / sizes of whole tiles:
+//   few rows, five parts and more to a tile 1.6 / 1.6, full rows 1.5 / 1.4, A contiguous along M 2.2 / 1.7.
 //   Jagged contraction: cut along K (above) it fills the chip whatever the groups' lengths.  A contiguous along M, up to 384
 //   tiles: 64 groups of 32 x 64 with 2048 elements each 46 / 13; 24 groups of 328 x 360, 95496 elements 201 / 98; two groups
 //   of 328 x 712, 40424 elements 652 / 62; past 384 the larger tile catches up (496 tiles of 184 x 464 in 62 even groups
@@ -625,9 +672,20 @@ bool gmm_staged_preferred(const GmmParams& p, int num_cus) {
   if (p.jag == GMM_JAG_K) {
     return p.a_sk != 1 && (2 * tiles <= 3 * cus || (p.K <= 64 * int64_t(p.G) && tiles <= 4 * cus));
   }
+  if (gmm_staged_cut_preferred(p, num_cus)) return true;
   if (p.a_sk != 1 && tiles <= tile_wgs(128) * cus && nk <= 32) return true;
   const bool rows_fill = p.jag == GMM_JAG_M ? p.M >= 64 * int64_t(p.G) : p.M >= 64;
   return nk <= 6 && tiles * nk <= 12 * cus && (nk == 1 || rows_fill || tiles <= cus);
+}
+
+bool gmm_staged_cut_preferred(const GmmParams& p, int num_cus) {
+  GmmParams cut = p;
+  if (!gmm_staged_eligible(p) || !split_tiles<128>(cut, tile_wgs(128) * int64_t(num_cus))) return false;
+  const int64_t tiles = most_tiles(p, 128), parts = tile_wgs(128) * int64_t(num_cus) / tiles;
+  if (p.a_sk != 1) return p.K >= 2560 && (parts >= 4 || p.K <= 6144);
+  if (parts >= 16) return true;
+  if (full_rows(p)) return p.K > 2048 && (parts >= 8 || (parts >= 4 && p.K <= 4096));
+  return parts >= 5 && p.K <= 6144;
 }
 
 // Products without alignment, 16-bit, that are over before a tile of 128 x 128 has started: K up to 16 and no more such tiles
@@ -655,8 +713,9 @@ bool gmm_staged_eligible(const GmmParams& p) {
 
 bool gmm_staged_uses_workspace(const GmmParams& p, int in_dtype, int num_cus) {
   GmmParams cut = p;
-  return (small_tiles(p, in_dtype, num_cus) ? cut_contraction<64>(cut, int64_t(tile_wgs(64)) * num_cus)
-                                            : cut_contraction<128>(cut, int64_t(tile_wgs(128)) * num_cus)) > 0;
+  if (small_tiles(p, in_dtype, num_cus))
+    return cut_contraction<64>(cut, int64_t(tile_wgs(64)) * num_cus) > 0 || split_tiles<64>(cut, int64_t(tile_wgs(64)) * num_cus);
+  return cut_contraction<128>(cut, int64_t(tile_wgs(128)) * num_cus) > 0 || split_tiles<128>(cut, int64_t(tile_wgs(128)) * num_cus);
 }
 
 int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream) {
