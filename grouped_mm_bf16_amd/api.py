@@ -200,31 +200,25 @@ class _GroupedMM(torch.autograd.Function):
 
         a_is_2d, b_is_2d = mat_a.dim() == 2, mat_b.dim() == 2
         grad_a = grad_b = None
+        # Elements of a jagged operand that no group owns get a zero gradient: rows or columns past the last offset.
         if need_a:
-            # Elements of a jagged operand that no group owns get a zero gradient.
-            jagged_a = (a_is_2d and not b_is_2d) or (a_is_2d and b_is_2d)
-            grad_a = (torch.zeros if jagged_a else torch.empty)(
-                mat_a.shape, device=mat_a.device, dtype=mat_a.dtype)
-            if not a_is_2d and not b_is_2d:
-                _k.grouped_mm_3d3d(grad_out, _t(mat_b), grad_a)
-            elif a_is_2d and not b_is_2d:
-                _k.grouped_mm_2d3d(grad_out, _t(mat_b), offs, grad_a)
-            elif a_is_2d and b_is_2d:
-                _k.grouped_mm_3d2d(grad_out, _t(mat_b), offs, grad_a)
+            if a_is_2d:
+                grad_a = _k.launch_zeroed(_k.V_3D2D if b_is_2d else _k.V_2D3D, grad_out, _t(mat_b), offs, mat_a.shape)
             else:
-                _k.grouped_mm_2d2d(grad_out, _t(mat_b), offs, grad_a)
+                grad_a = torch.empty(mat_a.shape, device=mat_a.device, dtype=mat_a.dtype)
+                if b_is_2d:
+                    _k.grouped_mm_2d2d(grad_out, _t(mat_b), offs, grad_a)
+                else:
+                    _k.grouped_mm_3d3d(grad_out, _t(mat_b), grad_a)
         if need_b:
-            jagged_b = b_is_2d
-            grad_b = (torch.zeros if jagged_b else torch.empty)(
-                mat_b.shape, device=mat_b.device, dtype=mat_b.dtype)
-            if not a_is_2d and not b_is_2d:
-                _k.grouped_mm_3d3d(_t(mat_a), grad_out, grad_b)
-            elif a_is_2d and not b_is_2d:
-                _k.grouped_mm_2d2d(_t(mat_a), grad_out, offs, grad_b)
-            elif a_is_2d and b_is_2d:
-                _k.grouped_mm_2d3d(_t(mat_a), grad_out, offs, grad_b)
+            if b_is_2d:
+                grad_b = _k.launch_zeroed(_k.V_2D3D if a_is_2d else _k.V_3D2D, _t(mat_a), grad_out, offs, mat_b.shape)
             else:
-                _k.grouped_mm_3d2d(_t(mat_a), grad_out, offs, grad_b)
+                grad_b = torch.empty(mat_b.shape, device=mat_b.device, dtype=mat_b.dtype)
+                if a_is_2d:
+                    _k.grouped_mm_2d2d(_t(mat_a), grad_out, offs, grad_b)
+                else:
+                    _k.grouped_mm_3d3d(_t(mat_a), grad_out, grad_b)
         return grad_a, grad_b, None, None, None
 
 

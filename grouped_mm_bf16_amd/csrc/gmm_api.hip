@@ -361,6 +361,18 @@ int gmm_3d2d(const void* a, const void* b, void* out, const int32_t* offs, int32
   return run(pr, static_cast<hipStream_t>(stream));
 }
 
+int gmm_zero_unowned(void* out, const int32_t* offs, int32_t G, int32_t by_columns, int64_t M, int64_t N, int64_t o_sm, int64_t o_sn,
+                     int32_t dtype, void* stream) {
+  if (!dims_ok(M, N, G) || G >= GMM_MAX_GROUPS) return GMM_ERR_BAD_ARGUMENT;
+  if (dtype < GMM_DT_BF16 || dtype > GMM_DT_F32) return GMM_ERR_UNSUPPORTED;
+  if (M == 0 || N == 0) return GMM_OK;
+  if (!out || (G > 0 && !offs)) return GMM_ERR_BAD_ARGUMENT;
+  GmmParams p{};
+  p.c = out; p.offs = offs; p.G = G; p.jag = by_columns ? GMM_JAG_N : GMM_JAG_M;
+  p.M = int32_t(M); p.N = int32_t(N); p.c_sm = o_sm; p.c_sn = o_sn;
+  return gmm_launch_zero_unowned(p, dtype, static_cast<hipStream_t>(stream)) == 0 ? GMM_OK : GMM_ERR_LAUNCH;
+}
+
 int gmm_set_path(int path) {
   if (path < GMM_PATH_AUTO || path > GMM_PATH_MFMA) return -1;
   return g_forced_path.exchange(path);

@@ -21,6 +21,9 @@ int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hip
 // Would this launch use a workspace of p.ws_parts slots?
 bool gmm_staged_uses_workspace(const GmmParams& p, int in_dtype, int num_cus);
 
+// Zeros in the rows (jagged rows) or columns (jagged columns) of the output that no group owns.
+int gmm_launch_zero_unowned(const GmmParams& p, int out_dtype, hipStream_t stream);
+
 // Operand layout facts the host derived from strides.
 struct GmmLayout {
   bool a_kc;  // A contiguous along K (row-major); otherwise contiguous along M

@@ -171,6 +171,32 @@ def _launch(variant: int, a: torch.Tensor, b: torch.Tensor, offs: Optional[torch
         _launch_now(variant, a, b, offs, out)
 
 
+# Bytes from which a gradient is not cleared first: torch's fill of 32 MiB takes as long as the kernel that looks at the offsets
+# (6 us; 134 MB 18.5), and a smaller one costs less host time than that launch.
+_CLEAR_FIRST_BELOW = 32 << 20
+
+
+def launch_zeroed(variant: int, a: torch.Tensor, b: torch.Tensor, offs: torch.Tensor, shape) -> torch.Tensor:
+    """A new tensor with the product of a variant with jagged rows or columns in it, zeros where no group owns anything: what a
+    gradient has to be.  A large one is not cleared as a whole, which wrote it twice."""
+    if torch.compiler.is_compiling() or shape[0] * shape[1] * a.element_size() < _CLEAR_FIRST_BELOW:
+        out = torch.zeros(shape, device=a.device, dtype=a.dtype)
+        if out.numel():
+            _launch(variant, a, b, offs, out)
+        return out
+    out = torch.empty(shape, device=a.device, dtype=a.dtype)
+    _launch_now(variant, a, b, offs, out)
+    _zero_unowned(out, offs, variant == V_3D2D)
+    return out
+
+
+def _zero_unowned(out: torch.Tensor, offs: torch.Tensor, by_columns: bool) -> None:
+    with torch.cuda.device(out.device) if out.device.index != torch.cuda.current_device() else contextlib.nullcontext():
+        rc = _lib.load().gmm_zero_unowned(out.data_ptr(), offs.data_ptr(), offs.numel(), int(by_columns), out.size(0), out.size(1),
+                                          out.stride(0), out.stride(1), _dtype_code(out.dtype), current_stream(out.device))
+    _lib.check(rc, "zeros past the last offset")
+
+
 def grouped_mm_3d3d(mat_a: torch.Tensor, mat_b: torch.Tensor, out: torch.Tensor) -> None:
     """out[g] = mat_a[g] @ mat_b[g]  (reference ``kernels.py:524-550``)."""
     if mat_a.size(0) != mat_b.size(0):

@@ -173,6 +173,12 @@ int gmm_3d2d(const void* a, const void* b, void* out, const int32_t* offs, int32
              int32_t in_dtype, int32_t out_dtype,
              void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Zeros in what no group owns of the output of gmm_2d3d (by_columns 0: the rows past the largest offset) or of gmm_3d2d
+ * (by_columns 1: the columns past it).  out [M, N], dtype a gmm_dtype; the rest of `out` is not touched.  With G == 0 nothing is
+ * owned.  What a gradient with respect to a jagged operand needs beside the product. */
+int gmm_zero_unowned(void* out, const int32_t* offs, int32_t G, int32_t by_columns, int64_t M, int64_t N,
+                     int64_t out_stride_m, int64_t out_stride_n, int32_t dtype, void* stream);
+
 /* ---- The mixture-of-experts step either side of the grouped product.  The reference has no such code;
  * its benchmark builds the sorted rows and `offs` with torch on the host side (bench/bench_2d3d.py:124-149:
  * randint / bincount / cumsum and an offs[-1].item() round trip).  Here everything stays on the device.

@@ -268,3 +268,60 @@ def test_1023_groups_backward_bf16_mfma():
     assert len(calls) == 3 and all(path == "mfma" for _, path in calls), calls
     assert_grads_forward_bar("2d3d", got, want, a, b, offs)
     assert (got[2][1::2] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("extent,other", [(40, 33), (3, 1), (257, 130)])
+@pytest.mark.parametrize("rows", [True, False])
+def test_what_no_group_owns_is_zeroed(rows, extent, other, dtype):
+    """Every place the owned part can end, offsets that go back or past the extent among them, into
+    contiguous, padded and transposed outputs: the rest is zero, the owned part and what lies around the output untouched."""
+    K = 24
+    gen = torch.Generator(device="cuda").manual_seed(extent)
+    G = 3
+    for offs in ([0, 0, 0], [1, 2, extent - 1], [2, 1, 1], [extent] * 3, [1, extent + 50, 2], [-5, 1, 1]):
+        od = torch.tensor(offs, dtype=torch.int32, device="cuda")
+        end = min(max(max(offs), 0), extent)
+        a = torch.randn((extent, K) if rows else (G, other, K), device="cuda", generator=gen).to(dtype)
+        b = torch.randn((G, K, other) if rows else (K, extent), device="cuda", generator=gen).to(dtype)
+        shape = (extent, other) if rows else (other, extent)
+        for padded, transposed in ((0, False), (5, False), (0, True)):
+            m, n = shape[::-1] if transposed else shape
+            stored = [torch.full((m, n + padded), 7.0, device="cuda", dtype=dtype) for _ in range(2)]
+            views = [t[:, :n].t() if transposed else t[:, :n] for t in stored]
+            for view in views:
+                K_._launch_now(K_.V_2D3D if rows else K_.V_3D2D, a, b, od, view)
+            K_._zero_unowned(views[1], od, not rows)
+            plain, zeroed = (v if rows else v.t() for v in views)
+            assert torch.equal(plain[:end], zeroed[:end]) and (plain[end:] == 7).all() and (zeroed[end:] == 0).all(), (offs, padded)
+            assert all((t[:, n:] == 7).all() for t in stored)
+    out = torch.full((4, 8), 7.0, device="cuda", dtype=dtype)
+    K_._zero_unowned(out, torch.empty(0, device="cuda", dtype=torch.int32), not rows)       # no groups: nothing is owned
+    assert (out == 0).all()
+
+
+@pytest.mark.parametrize("variant", ["2d3d", "2d2d", "3d2d"])
+@pytest.mark.parametrize("clear_first", [True, False])
+def test_gradients_past_the_last_offset(variant, clear_first, monkeypatch):
+    """Either way of clearing, with elements past the last offset: zeros there, the loop's gradients elsewhere."""
+    monkeypatch.setattr(K_, "_CLEAR_FIRST_BELOW", 1 << 40 if clear_first else 0)
+    gen = torch.Generator().manual_seed(11)
+    sizes = [5, 0, 20, 13]
+    tot, ends = sum(sizes) + 6, offs_of(sizes)
+    shapes = {"2d3d": ((tot, 40), (4, 40, 24)), "2d2d": ((32, tot), (tot, 24)), "3d2d": ((4, 32, 40), (40, tot))}[variant]
+    a, b = (rnd(gen, *s).to(torch.bfloat16) for s in shapes)
+    ad, bd = a.to(DEV).requires_grad_(), b.to(DEV).requires_grad_()
+    junk = torch.full((1 << 22,), float("nan"), device=DEV)     # what torch.empty hands out next holds NaN
+    del junk
+    out = grouped_mm(ad, bd, offs=ends.to(DEV))
+    go = rnd(gen, *out.shape).to(torch.bfloat16)
+    out.backward(go.to(DEV))
+    ar, br = a.float().requires_grad_(), b.float().requires_grad_()
+    loop_reference(variant, ar, br, ends).backward(go.float())
+    for got, want in ((ad.grad, ar.grad), (bd.grad, br.grad)):
+        torch.testing.assert_close(got.float().cpu(), want, rtol=4e-2, atol=4e-2)
+    end = sum(sizes)
+    if variant != "3d2d":
+        assert (ad.grad[end:] == 0).all() if variant == "2d3d" else (ad.grad[:, end:] == 0).all() and (bd.grad[end:] == 0).all()
+    else:
+        assert (bd.grad[:, end:] == 0).all()
