@@ -348,7 +348,8 @@ __device__ __forceinline__ bool join_parts(const GmmParams& p, const GmmTile& ti
   return true;
 }
 
-// SPLIT = 1: a jagged contraction whose groups may be cut along K.  SPLIT = 2: any other product, few tiles cut along K.
+// SPLIT = 1: a jagged contraction whose groups may be cut along K.  SPLIT = 2: any other product, the tiles of the last round
+// cut along K.
 template <typename T, typename OutT, bool A_TR, bool B_TR, int EDGE, int SPLIT>
 __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const GmmParams p) {
   constexpr int BM = EDGE, BN = EDGE;
@@ -376,10 +377,14 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
     return __builtin_amdgcn_readfirstlane(in_registers ? groups.build(p, BM, BN, chunk) : gmm_build_tile_table<NT>(p, BM, BN, cum, chunk));
   };
   int total = build();
-  // few tiles: each in as many parts as there are workgroups for
-  const int tiles = gmm_max(total, 1);
-  const int split = SPLIT == 2 ? gmm_max(gmm_min(p.k_split, gmm_min(int(gridDim.x), p.k_parts) / tiles), 1) : 1;
-  if (SPLIT == 2) total *= split;
+  // the tiles of the last, partly filled round: each in as many parts as there are places for, and behind whole rounds only if
+  // that makes four of each.  Places: the workgroups; behind whole rounds of 64 x 64 tiles, four of which share a CU's matrix
+  // cores, half of them (a tile that is alone on its CU already runs three times as fast as in a full round).
+  const int tail = SPLIT == 2 ? total % int(gridDim.x) : 0, whole = total - tail;
+  const int places = EDGE == 64 && whole ? int(gridDim.x) / 2 : int(gridDim.x);
+  int split = SPLIT == 2 && tail ? gmm_max(gmm_min(p.k_split, gmm_min(places, p.k_parts) / tail), 1) : 1;
+  if (SPLIT == 2 && whole && split < 4) split = 1;
+  if (SPLIT == 2) total = whole + tail * split;
   if (SPLIT == 1 && chunk && total > p.k_parts) {   // offsets that overlap: more parts than K elements have room for
     chunk = 0;
     __syncthreads();
@@ -387,14 +392,15 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
   }
 
   for (int t = blockIdx.x; t < total; t += gridDim.x) {
-    const int id = gmm_xcd_remap(t, total, gridDim.x);
+    int id = gmm_xcd_remap(t, total, gridDim.x);
     int g, local, lo, hi;
     int part = 0, parts = 1, per = 1, number = id;
-    if (SPLIT == 2) {
-      per = tiles;
+    if (SPLIT == 2 && id >= whole) {
+      per = tail;
       parts = split;
-      part = id / tiles;
-      number = id - part * tiles;
+      id -= whole;
+      part = id / tail;
+      number = whole + id - part * tail;
     }
     if (in_registers) groups.find(number, g, local, lo, hi);
     else gmm_find_tile(p, cum, number, BM, BN, g, local, lo, hi);
@@ -612,12 +618,28 @@ bool split_tiles(GmmParams& p, int64_t most_wgs) {
   return true;
 }
 
+// Cut the tiles of the last round along K where it holds only a few?  The device knows how many; launches of one to four
+// rounds with at least 24 K tiles can have a use for it.  us, whole / cut: fp32 1024 x 1024 x 8192 columns in 8 groups (2.1
+// rounds) 165 / 157, 8192 x 1024 x 4096 in 8 groups 617 / 577; bf16 8191 x 2047 x 2047 in 8 groups 157 / 148, 5 products of 7 x
+// 13204 x 2148 (520 tiles, 512 workgroups) 99 / 71.  400 random launches: 1.4 at best, 0.96 at worst, uncut ones among them.
+template <int EDGE>
+bool split_tail(GmmParams& p, int64_t most_wgs, int esz) {
+  if (p.jag == GMM_JAG_K || p.ws_parts <= 0 || int64_t(p.K) * esz < 24 * ROW_BYTES) return false;
+  const int64_t tiles = expected_tiles(p, EDGE);
+  int64_t room = int64_t(p.ws_parts) * GMM_WS_SLOT / (EDGE * EDGE * 4);
+  if (room > GMM_WS_TICKET) room = GMM_WS_TICKET;
+  if (tiles <= most_wgs || tiles > 4 * most_wgs) return false;
+  p.k_split = p.K / (GMM_K_SPLIT_MIN / 2) < GMM_K_CLUSTER ? p.K / (GMM_K_SPLIT_MIN / 2) : GMM_K_CLUSTER;
+  p.k_parts = int32_t(room);
+  return true;
+}
+
 template <typename T, typename OutT, int EDGE>
 int launch_layout(GmmParams p, bool a_tr, bool b_tr, int num_cus, hipStream_t stream) {
   const int64_t most = int64_t(tile_wgs(EDGE)) * num_cus;
   int64_t bound = cut_contraction<EDGE>(p, most);
   if (bound == 0) bound = gmm_tile_bound(p.jag, p.G, p.M, p.N, EDGE, EDGE);
-  const bool split = split_tiles<EDGE>(p, most);
+  const bool split = split_tiles<EDGE>(p, most) || split_tail<EDGE>(p, most, sizeof(T));
   if (split) bound = gmm_tile_bound(p.jag, p.G, p.M, p.N, EDGE, EDGE) * p.k_split;
   const int64_t want = (bound + 7) / 8 * 8;
   p.num_wg = int(want < most ? (want < 8 ? 8 : want) : most);
@@ -711,11 +733,16 @@ bool gmm_staged_eligible(const GmmParams& p) {
   return lda >= 1 && ldb >= 1 && p.K >= 1 && rows >= 1 && a_len >= 8 && b_len >= 8;
 }
 
+template <int EDGE>
+static bool uses_workspace(GmmParams& p, int64_t most_wgs, int esz) {
+  return cut_contraction<EDGE>(p, most_wgs) > 0 || split_tiles<EDGE>(p, most_wgs) || split_tail<EDGE>(p, most_wgs, esz);
+}
+
 bool gmm_staged_uses_workspace(const GmmParams& p, int in_dtype, int num_cus) {
   GmmParams cut = p;
   if (small_tiles(p, in_dtype, num_cus))
-    return cut_contraction<64>(cut, int64_t(tile_wgs(64)) * num_cus) > 0 || split_tiles<64>(cut, int64_t(tile_wgs(64)) * num_cus);
-  return cut_contraction<128>(cut, int64_t(tile_wgs(128)) * num_cus) > 0 || split_tiles<128>(cut, int64_t(tile_wgs(128)) * num_cus);
+    return uses_workspace<64>(cut, int64_t(tile_wgs(64)) * num_cus, 4);
+  return uses_workspace<128>(cut, int64_t(tile_wgs(128)) * num_cus, in_dtype == GMM_DT_F32 ? 4 : 2);
 }
 
 int gmm_launch_staged(GmmParams p, int in_dtype, int out_dtype, int num_cus, hipStream_t stream) {

@@ -117,3 +117,18 @@ def test_gathered_rows_of_cut_tiles():
         for out in outs:
             check(out[lo:hi], padded[idx[lo:hi].long()], b[g])
     assert (outs[0][3] == 0).all()
+
+
+# the last round behind whole ones: 512 workgroups of 128 x 128 tiles, 1024 of 64 x 64 (fp32); tiles past it that are cut, that
+# are too many to be cut, none at all; K at the line of 24 K tiles and below it
+@pytest.mark.parametrize("dtype,G,M,N,K", [(torch.bfloat16, 13, 130, 2570, 1537), (torch.float16, 26, 100, 2570, 1601), (torch.bfloat16, 16, 250, 2040, 1543),
+                                           (torch.bfloat16, 13, 130, 2570, 1535), (torch.float32, 26, 130, 2500, 801), (torch.float32, 27, 130, 2500, 769)])
+def test_last_round_behind_whole_ones(dtype, G, M, N, K):
+    gen = torch.Generator(device=DEV).manual_seed(K)
+    a, b = (torch.randn(*s, device=DEV, generator=gen).to(dtype) for s in ((G, M, K), (G, K, N)))
+    out, whole = launches(lambda o: K_.grouped_mm_3d3d(a, b, o), (G, M, N), dtype)
+    for g in range(G):
+        if g % 5 == 0 or not torch.equal(out[g], whole[g]):
+            check(out[g, :, -700:], a[g].cpu(), b[g, :, -700:].cpu())
+    bound = (K + 1) * 2.0 ** -23 * (a.float().abs() @ b.float().abs()) + (0 if dtype == torch.float32 else 2.0 ** -7) * whole.float().abs()
+    assert ((out.float() - whole.float()).abs() <= bound).all()       # both within half of that of the exact sum
