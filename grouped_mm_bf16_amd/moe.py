@@ -9,7 +9,7 @@ Here no count ever reaches the host: the kernels read ``offs`` from device memor
 by ``tokens * top_k``, which the host knows.
 
 Forward only (inference); the functions take and return plain tensors.  Each one is also registered as a
-torch custom op (``grouped_mm_bf16_amd::moe_route``, ``gathered``, ``swiglu``, ``activation``, ``combine``) and
+torch custom op (``grouped_mm_bf16_amd::moe_route``, ``gathered``, ``gate_up``, ``swiglu``, ``activation``, ``combine``) and
 dispatches to it while a model around it is being traced or compiled.
 """
 from __future__ import annotations

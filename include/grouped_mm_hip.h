@@ -59,7 +59,7 @@ const char* gmm_status_string(int status);
  * once.  gmm_2d2d uses it in two more ways: groups that are long beside the number of tiles are cut into parts in the same
  * manner, and tiles of groups of uneven length are drawn from counters in it by whichever workgroup is free.
  * With and without a workspace (or with one of another size) the last bits of a result may differ where tiles are cut: gmm_2d3d,
- * gmm_3d3d and gmm_3d2d with a partly filled last round, gmm_2d2d with a first operand contiguous along its rows or with
+ * gmm_3d3d and gmm_3d2d with a partly filled last or only round, gmm_2d2d with a first operand contiguous along its rows or with
  * fp32 or unaligned operands; aligned 16-bit gmm_2d2d with a first operand contiguous along K is never cut.  Eager and
  * captured launches that both have one of gmm_workspace_bytes() give the same bits.
  * Layout: 4096 bytes of counters, then slots of 262144 bytes (one fp32 tile each); the more
