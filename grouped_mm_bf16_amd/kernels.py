@@ -43,6 +43,10 @@ def current_stream(device: torch.device) -> int:
     return torch._C._cuda_getCurrentRawStream(device.index)
 
 
+# The same for torch.cuda.current_device(), which first makes sure that there is a device: here a tensor lies on it.
+current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 # One workspace per (device, stream): launches on one stream run one after the other, so they can share it;
 # launches on different streams may overlap and must not.  Allocated on first use and kept (the library leaves
 # the arrival counters at its head zero after every launch).  For eager launches only: a captured launch runs on
@@ -114,7 +118,7 @@ def _launch_now(variant: int, a: torch.Tensor, b: torch.Tensor, offs: Optional[t
     _require_gpu(a, b, offs, out)
     device = a.device
     # the device guard costs microseconds; only switch when the tensors live on another device
-    if device.index != torch.cuda.current_device():
+    if device.index != current_device():
         with torch.cuda.device(device):
             _launch_here(lib, device, variant, a, b, offs, out)
     else:
@@ -191,7 +195,7 @@ def launch_zeroed(variant: int, a: torch.Tensor, b: torch.Tensor, offs: torch.Te
 
 
 def _zero_unowned(out: torch.Tensor, offs: torch.Tensor, by_columns: bool) -> None:
-    with torch.cuda.device(out.device) if out.device.index != torch.cuda.current_device() else contextlib.nullcontext():
+    with torch.cuda.device(out.device) if out.device.index != current_device() else contextlib.nullcontext():
         rc = _lib.load().gmm_zero_unowned(out.data_ptr(), offs.data_ptr(), offs.numel(), int(by_columns), out.size(0), out.size(1),
                                           out.stride(0), out.stride(1), _dtype_code(out.dtype), current_stream(out.device))
     _lib.check(rc, "zeros past the last offset")

@@ -34,13 +34,17 @@ class Routing(NamedTuple):
     token_rows: torch.Tensor    # int32 [S]  row of each slot (inverse permutation)
 
 
+_HERE = contextlib.nullcontext()
+
+
 def _guard(t: torch.Tensor):
-    return torch.cuda.device(t.device) if t.device.index != torch.cuda.current_device() else contextlib.nullcontext()
+    return torch.cuda.device(t.device) if t.device.index != kernels.current_device() else _HERE
 
 
-def _route_packed_now(router_logits: torch.Tensor, top_k: int, renormalize: bool) -> torch.Tensor:
-    """The five routing results in one int32 buffer [E + 4 S] (offs, slot_expert, slot_weight bits, row_token,
-    token_rows): one allocation for results and workspace (each allocation costs microseconds of host time)."""
+def _route_now(router_logits: torch.Tensor, top_k: int, renormalize: bool) -> torch.Tensor:
+    """The five routing results in one int32 buffer (offs [E], slot_expert, slot_weight bits, row_token, token_rows, [S] each)
+    with the workspace behind them: one allocation, cut once (each tensor costs a microsecond of host time, a layer of a few
+    tokens 39)."""
     _require_gpu(router_logits)
     if router_logits.dim() != 2:
         raise RuntimeError("router_logits has to be 2D [tokens, experts]")
@@ -57,14 +61,18 @@ def _route_packed_now(router_logits: torch.Tensor, top_k: int, renormalize: bool
     if ws_bytes < 0:
         raise RuntimeError("moe_route: sizes out of range")
     buf = torch.empty(E + 4 * S + ws_bytes // 4, device=dev, dtype=torch.int32)
-    base, ws = buf.data_ptr(), buf[E + 4 * S:]
+    base = buf.data_ptr()
     with _guard(router_logits):
         rc = lib.gmm_moe_route(router_logits.data_ptr(), router_logits.stride(0) if T else E,
                                _dtype_code(router_logits.dtype), T, E, top_k, int(bool(renormalize)),
                                base, base + 4 * E, base + 4 * (E + S), base + 4 * (E + 2 * S), base + 4 * (E + 3 * S),
-                               ws.data_ptr(), ws_bytes, kernels.current_stream(dev))
+                               base + 4 * (E + 4 * S), ws_bytes, kernels.current_stream(dev))
     _lib.check(rc, "moe_route")
-    return buf[:E + 4 * S]
+    return buf
+
+
+def _route_packed_now(router_logits: torch.Tensor, top_k: int, renormalize: bool) -> torch.Tensor:
+    return _route_now(router_logits, top_k, renormalize)[:router_logits.size(1) + 4 * router_logits.size(0) * top_k]
 
 
 _route_op = torch.library.custom_op("grouped_mm_bf16_amd::moe_route", mutates_args=())(_route_packed_now)
@@ -83,10 +91,10 @@ def moe_route(router_logits: torch.Tensor, top_k: int, renormalize: bool = True)
     weights are the softmax over the chosen logits (``renormalize``) or the chosen entries of the softmax
     over all experts.
     """
-    impl = _route_op if torch.compiler.is_compiling() else _route_packed_now
+    impl = _route_op if torch.compiler.is_compiling() else _route_now
     buf = impl(router_logits, top_k, bool(renormalize))
     E, S = router_logits.size(1), router_logits.size(0) * top_k
-    parts = torch.split(buf, [E, S, S, S, S])
+    parts = torch.split(buf, [E, S, S, S, S, buf.size(0) - E - 4 * S])
     return Routing(parts[0], parts[1], parts[2].view(torch.float32), parts[3], parts[4])
 
 
