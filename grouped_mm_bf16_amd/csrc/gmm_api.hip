@@ -205,12 +205,16 @@ int run(Problem& pr, hipStream_t stream) {
       automatic = automatic && fo < 0;
     }
     // small products run on 128 x 128 tiles of the register-staged kernel, unless something of the assembly tile is forced
-    const bool staged = automatic && cfg == GMM_CFG_ASM_256x256 && gmm_staged_preferred(p, cus);
+    automatic = automatic && cfg == GMM_CFG_ASM_256x256;
     if (pr.eager_only) {
+      // Does the launch have a use for a workspace?  Judged with a full one, also where none came along (a stream that has run
+      // nothing before the capture): some products go to the register-staged kernel because they can be cut there.
       const GmmParams q = with_full_workspace(p, cus);
-      if ((staged ? gmm_staged_uses_workspace(q, pr.in_dtype, cus) : gmm_mfma_uses_workspace(q, lay, cfg, cus)) && capture_id(stream))
-        return GMM_ERR_WORKSPACE;
+      const bool uses = automatic && gmm_staged_preferred(q, cus) ? gmm_staged_uses_workspace(q, pr.in_dtype, cus)
+                                                                  : gmm_mfma_uses_workspace(q, lay, cfg, cus);
+      if (uses && capture_id(stream)) return GMM_ERR_WORKSPACE;
     }
+    const bool staged = automatic && gmm_staged_preferred(p, cus);
     rc = staged ? gmm_launch_staged(p, pr.in_dtype, pr.out_dtype, cus, stream)
                 : gmm_launch_mfma(p, lay, pr.in_dtype, pr.out_dtype, cfg, cus, stream);
     t_last_path = GMM_PATH_MFMA;

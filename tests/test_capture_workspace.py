@@ -138,3 +138,57 @@ def test_capture_that_torch_does_not_know_of():
         # the same products, summed uncut
         torch.testing.assert_close(out.float(), eager.float(), rtol=1.6e-2, atol=1e-2 * 8)
     assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
+def _cut_cases():
+    """Launches whose tiles are cut along K: aligned and few (the assembly tile's without a workspace), unaligned and few, the
+    last round behind whole ones, gathered rows, and a layer whose up projection is one of them."""
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    r = lambda *s, dtype=torch.bfloat16: torch.randn(*s, device=DEV, generator=gen).to(dtype)
+    a1, b1 = r(2, 96, 2048), r(2, 2048, 1024)
+    a2, b2, o2 = r(8, 2048), r(8, 2048, 1536), _offs([1] * 8)
+    a3, b3 = r(2, 90, 2047), r(2, 2047, 1001)
+    a4, b4 = r(26, 130, 801, dtype=torch.float32), r(26, 801, 2500, dtype=torch.float32)
+    idx = torch.randint(0, 8, (8,), device=DEV, dtype=torch.int32, generator=gen)
+    x, logits, w_up, w_down = r(6, 2048), r(6, 8), r(8, 2048, 1024), r(8, 512, 2048)
+    return {
+        "aligned": lambda: _into((2, 96, 1024), lambda out: K_.grouped_mm_3d3d(a1, b1, out)),
+        "decode": lambda: _into((8, 1536), lambda out: K_.grouped_mm_2d3d(a2, b2, o2, out)),
+        "unaligned": lambda: _into((2, 90, 1001), lambda out: K_.grouped_mm_3d3d(a3, b3, out)),
+        "last round": lambda: _into((26, 130, 2500), lambda out: K_.grouped_mm_3d3d(a4, b4, out), torch.float32),
+        "gathered": lambda: moe.grouped_mm_gathered(a2, idx, b2, o2),
+        "layer": lambda: moe.moe_forward(x, logits, w_up, w_down, 2),
+    }
+
+
+def _into(shape, launch, dtype=torch.bfloat16):
+    out = torch.empty(shape, device=DEV, dtype=dtype)
+    launch(out)
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["aligned", "decode", "unaligned", "last round", "gathered", "layer"])
+def test_cut_tiles_on_a_capture_stream_without_a_workspace(name):
+    """torch.cuda.graph captures on a stream that no eager launch has used: the launch is recorded with the same kernel and
+    the same cuts, so that every replay gives the eager result's bits."""
+    call = _cut_cases()[name]
+    bits = lambda t: t.view(torch.int32 if t.dtype == torch.float32 else torch.int16)
+    eager = call()
+    kernel = K_.last_kernel()
+    assert kernel == "any" or name == "layer"
+    with K_.tail_split(False):
+        assert name == "layer" or not torch.equal(bits(call()), bits(eager)), "nothing was cut"
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    K_._workspaces.pop((torch.cuda.current_device(), stream.cuda_stream), None)      # torch hands out streams again
+    with torch.cuda.graph(graph, stream=stream):
+        out = call()
+        assert K_.last_kernel() == kernel
+    assert (torch.cuda.current_device(), stream.cuda_stream) not in K_._workspaces
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(bits(out), bits(eager))
+        assert torch.equal(bits(call()), bits(eager))
