@@ -614,6 +614,8 @@ def gen_epilogue(v, e, L):
         e("v_mov_b32 %s, %d" % (vr(vtmp), esz * el))
         e("v_cndmask_b32 %s, %s, %s, vcc" % (vr(eoff + el), vr(V_OOB), vr(vtmp)))
     e.label("L_nopart_setup_%s" % L)
+    if v.rounded:
+        e("s_mov_b32 %s, 0x3e800000" % sr(S_T))       # 0.25
     nstore = 0
     for p0 in range(0, v.tm, ipp):
         k = 0
@@ -650,17 +652,37 @@ def gen_epilogue(v, e, L):
                     for r in range(4):
                         e("v_exp_f32 %s, %s" % (vr(b + 8 + r), vr(b + 8 + r)))
                     e("s_nop 0")
-                    for r in range(4):
-                        e("v_add_f32 %s, 1.0, %s" % (vr(b + 8 + r), vr(b + 8 + r)))
-                    for r in range(4):
-                        e("v_rcp_f32 %s, %s" % (vr(b + 8 + r), vr(b + 8 + r)))
-                    # rounded: the gate's activation first, the order of the activation kernel (a gate far below zero
-                    # makes the result zero however large its partner is)
-                    first, second = (b + 8, b + 4) if v.rounded else (b + 4, b + 8)
-                    for r in range(4):
-                        e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(b + r), vr(first + r)))
-                    for r in range(4):
-                        e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(b + r), vr(second + r)))
+                    if v.rounded:
+                        # g / d, d = 1 + 2^(-g log2 e), rounded as the activation kernel's division: one correction of the
+                        # quotient by its residual.  Both a quarter as large: the reciprocal of a d from 2^126 on would be
+                        # subnormal, which v_rcp_f32 takes for zero.  An infinite d is left to v_div_fixup_f32.  Then times
+                        # the partner, in that order: a gate far below zero makes the result zero, however large its partner.
+                        x = t + 48 + 12 * (k % 2)
+                        for r in range(4):
+                            e("v_fma_f32 %s, %s, %s, %s" % (vr(b + 8 + r), vr(b + 8 + r), sr(S_T), sr(S_T)))
+                        for r in range(4):
+                            e("v_rcp_f32 %s, %s" % (vr(x + r), vr(b + 8 + r)))
+                        for r in range(4):
+                            e("v_mul_f32 %s, %s, %s" % (vr(b + r), sr(S_T), vr(b + r)))
+                        for r in range(4):
+                            e("v_mul_f32 %s, %s, %s" % (vr(x + 4 + r), vr(b + r), vr(x + r)))
+                        for r in range(4):
+                            e("v_fma_f32 %s, -%s, %s, %s" % (vr(x + 8 + r), vr(b + 8 + r), vr(x + 4 + r), vr(b + r)))
+                        for r in range(4):
+                            e("v_fma_f32 %s, %s, %s, %s" % (vr(x + 4 + r), vr(x + 8 + r), vr(x + r), vr(x + 4 + r)))
+                        for r in range(4):
+                            e("v_div_fixup_f32 %s, %s, %s, %s" % (vr(x + 4 + r), vr(x + 4 + r), vr(b + 8 + r), vr(b + r)))
+                        for r in range(4):
+                            e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(x + 4 + r), vr(b + 4 + r)))
+                    else:
+                        for r in range(4):
+                            e("v_add_f32 %s, 1.0, %s" % (vr(b + 8 + r), vr(b + 8 + r)))
+                        for r in range(4):
+                            e("v_rcp_f32 %s, %s" % (vr(b + 8 + r), vr(b + 8 + r)))
+                        for r in range(4):
+                            e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(b + r), vr(b + 4 + r)))
+                        for r in range(4):
+                            e("v_mul_f32 %s, %s, %s" % (vr(b + r), vr(b + r), vr(b + 8 + r)))
                     e("v_cvt_pk_%s_f32 %s, %s, %s" % (v.dt, vr(b + 8), vr(b), vr(b + 1)))
                     e("v_cvt_pk_%s_f32 %s, %s, %s" % (v.dt, vr(b + 9), vr(b + 2), vr(b + 3)))
                     e("ds_write_b64 %s, %s offset:%d" % (vr(V_EPI), vr(b + 8, 2), rowoff + 16 * j * 2))

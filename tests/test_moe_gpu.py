@@ -278,6 +278,34 @@ def test_swiglu_with_gate_and_partner_columns_apart(dtype, K, N, b_col):
     ulp_close(got[:M][ok], two[ok], dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_swiglu_epilogue_rounds_as_the_activation_kernel(dtype):
+    """Every 16-bit gate with partners over the type's range: the bits of product and activation in two kernels.  Gates of -88
+    have a logistic value below the smallest normal fp32 number, but not a result below it."""
+    gates = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
+    top = 15 if dtype == torch.float16 else 126
+    partners = torch.tensor([(1 + (7 * c % 64) / 64) * 2.0 ** (top * (c - 32) // 32) * (-1) ** c for c in range(64)]).to(dtype)
+    a, w = torch.zeros(65536, 64, dtype=dtype), torch.zeros(1, 64, 128, dtype=dtype)
+    a[:, 0], a[:, 1], w[0, 0, :64], w[0, 1, 64:] = gates, 1, 1, partners       # row: one gate, column: one partner
+    a, w, offs = a.to(DEV), w.to(DEV), offs_of([65536]).to(DEV)
+    rows = torch.arange(65536, dtype=torch.int32, device=DEV)
+    out = torch.empty(65536, 64, device=DEV, dtype=dtype)
+    rc = _lib.load().gmm_2d3d_swiglu_apart(a.data_ptr(), rows.data_ptr(), w.data_ptr(), out.data_ptr(), offs.data_ptr(), 1, 65536, 65536, 128, 64,
+                                           *a.stride(), *w.stride(), *out.stride(), K_._dtype_code(dtype), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and K_.last_kernel() == "assembly"
+    h = moe.grouped_mm_gathered(a, rows, w, offs)
+    two = moe.moe_activation(h, "swiglu")
+    assert torch.equal(out.isnan(), two.isnan())
+    same = (out.view(torch.int16) == two.view(torch.int16)) | two.isnan()
+    assert same.all(), (int((~same).sum()), h[:, 0][~same.all(1)][:8].tolist())
+    h64 = h.double().cpu()                                                     # and what both of them should be
+    want = h64[:, :64] / (1 + (-h64[:, :64]).exp()) * h64[:, 64:]
+    ok = want.isfinite() & (want.abs() <= torch.finfo(dtype).max) & (h64[:, :64] > -88)
+    least = torch.finfo(dtype).tiny                                            # below it: units of the subnormal numbers
+    err = (out.double().cpu() - want).abs()[ok]
+    assert (err <= 2.0 ** (-10 if dtype == torch.float16 else -7) * want[ok].abs().clamp(min=least)).all()
+
+
 def test_layers_whose_up_projection_stays_two_kernels():
     """Few rows of large matrices, an inner size that is no multiple of 64, forced kernels: the same layer results."""
     for T, H, I, E, k in [(40, 2048, 2048, 2, 1), (40, 64, 72, 4, 2)]:
