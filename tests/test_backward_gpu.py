@@ -271,7 +271,7 @@ def test_1023_groups_backward_bf16_mfma():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("extent,other", [(40, 33), (3, 1), (257, 130)])
+@pytest.mark.parametrize("extent,other", [(40, 33), (3, 1), (257, 130), (5003, 5)])
 @pytest.mark.parametrize("rows", [True, False])
 def test_what_no_group_owns_is_zeroed(rows, extent, other, dtype):
     """Every place the owned part can end, offsets that go back or past the extent among them, into
@@ -300,6 +300,16 @@ def test_what_no_group_owns_is_zeroed(rows, extent, other, dtype):
     assert (out == 0).all()
 
 
+def poison_new_memory(monkeypatch):
+    """From here on what torch.empty hands out on the GPU holds NaN."""
+    real = torch.empty
+
+    def poisoned(*args, **kwargs):
+        t = real(*args, **kwargs)
+        return t.fill_(float("nan")) if t.is_cuda and t.is_floating_point() else t
+    monkeypatch.setattr(torch, "empty", poisoned)
+
+
 @pytest.mark.parametrize("variant", ["2d3d", "2d2d", "3d2d"])
 @pytest.mark.parametrize("clear_first", [True, False])
 def test_gradients_past_the_last_offset(variant, clear_first, monkeypatch):
@@ -311,10 +321,9 @@ def test_gradients_past_the_last_offset(variant, clear_first, monkeypatch):
     shapes = {"2d3d": ((tot, 40), (4, 40, 24)), "2d2d": ((32, tot), (tot, 24)), "3d2d": ((4, 32, 40), (40, tot))}[variant]
     a, b = (rnd(gen, *s).to(torch.bfloat16) for s in shapes)
     ad, bd = a.to(DEV).requires_grad_(), b.to(DEV).requires_grad_()
-    junk = torch.full((1 << 22,), float("nan"), device=DEV)     # what torch.empty hands out next holds NaN
-    del junk
     out = grouped_mm(ad, bd, offs=ends.to(DEV))
     go = rnd(gen, *out.shape).to(torch.bfloat16)
+    poison_new_memory(monkeypatch)
     out.backward(go.to(DEV))
     ar, br = a.float().requires_grad_(), b.float().requires_grad_()
     loop_reference(variant, ar, br, ends).backward(go.float())
@@ -325,3 +334,26 @@ def test_gradients_past_the_last_offset(variant, clear_first, monkeypatch):
         assert (ad.grad[end:] == 0).all() if variant == "2d3d" else (ad.grad[:, end:] == 0).all() and (bd.grad[end:] == 0).all()
     else:
         assert (bd.grad[:, end:] == 0).all()
+
+
+@pytest.mark.parametrize("variant,dtype,other", [("2d3d", torch.bfloat16, 520), ("2d2d", torch.bfloat16, 520), ("3d2d", torch.bfloat16, 520),
+                                                 ("2d3d", torch.float32, 263), ("2d2d", torch.float32, 263), ("3d2d", torch.float16, 521)])
+def test_large_gradients_past_the_last_offset(variant, dtype, other, monkeypatch):
+    """Gradients from 32 MiB on are not cleared first: the bits of those that are."""
+    gen = torch.Generator(device=DEV).manual_seed(other)
+    extent, ends = 33003, [7000, 7000, 20001]
+    shapes = {"2d3d": ((extent, other), (3, other, 8)), "2d2d": ((other, extent), (extent, 8)), "3d2d": ((3, 8, other), (other, extent))}[variant]
+    a, b = (torch.randn(*s, device=DEV, generator=gen).to(dtype).requires_grad_() for s in shapes)
+    out = grouped_mm(a, b, offs=torch.tensor(ends, dtype=torch.int32, device=DEV))
+    go = torch.randn(out.shape, device=DEV, generator=gen).to(dtype)
+    assert max(t.numel() * t.element_size() for t in (a, b)) >= K_._CLEAR_FIRST_BELOW
+    with monkeypatch.context() as m:
+        poison_new_memory(m)
+        got = torch.autograd.grad(out, (a, b), go, retain_graph=True)
+    monkeypatch.setattr(K_, "_CLEAR_FIRST_BELOW", 1 << 40)
+    want = torch.autograd.grad(out, (a, b), go)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    for g, w in zip(got, want):
+        assert w.isfinite().all() and torch.equal(g.view(bits), w.view(bits))
+    jagged = want[1] if variant == "3d2d" else want[0]
+    assert (jagged[ends[-1]:] == 0).all() if variant == "2d3d" else (jagged[:, ends[-1]:] == 0).all()
