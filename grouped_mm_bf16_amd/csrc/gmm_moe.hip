@@ -260,32 +260,48 @@ __global__ void __launch_bounds__(64) moe_scatter_kernel(const int32_t* __restri
 
 // ---------------------------------------------------------------- routing of up to kPlaceSlots slots: one kernel
 // Workgroup b places slots [b * 1024, b * 1024 + 1024), each of its 16 waves 64 of them.  It counts the experts of all slots
-// itself, those before its own apart from the others (LDS atomics, four copies against conflicts), so there is no table of
-// counts to write, wait for and scan: histogram, scan and scatter were three launches.  The placing is that of
-// moe_scatter_kernel.  With the choice, us: 32768 slots of 128 experts 26 -> 12, 16384 of 8 18 -> 11.  Counting grows with the
-// slots, in every workgroup: at 131072 29 against 44, at 196608 and more the three kernels are as fast.
+// itself, those before its own apart from those behind them, so there is no table of counts to write, wait for and scan:
+// histogram, scan and scatter were three launches.  The placing is that of moe_scatter_kernel.
+// Slots of one expert would count one after the other on one LDS word (131072 tokens that all choose expert 0 of 8 took 132 us):
+// each count is several words, for lanes next to each other.  us with the choice, three kernels / this one: 4096 tokens, 8 of
+// 128 experts 26 / 13; 16384, 2 of 8 21 / 12; 65536, 2 of 8 39 / 32; 131072, 1 of 8 47 / 38, of 64 52 / 41, all on one of them 52
+// / 40.  Counting grows with the slots, in every workgroup: past kPlaceSlots the three kernels.
 constexpr int kPlaceWaves = 16;
 constexpr int kPlaceBlock = 64 * kPlaceWaves;
-constexpr int kPlaceCopies = 4;
 constexpr int kPlaceSlots = 131072;
+constexpr int kPlaceWords = (kPlaceWaves + 2 * 8) * (kMaxExperts + 1);   // LDS: kPlaceWaves * E cursors and the counts
 
-// Rows of E counts: copies of the slots before the workgroup's own, copies of those behind them, the waves' cursors.
-constexpr int kPlaceRows = 2 * kPlaceCopies + kPlaceWaves;
+// Words of a count, as a power of two: 32 up to 32 experts, 8 from 128 on.  More of them cost more to clear and to add up than
+// they save where slots spread over many experts.
+__device__ __forceinline__ int place_copy_bits(int E) {
+  int bits = 5;
+  while (bits > 3 && (E << bits) > 1024) --bits;
+  return bits;
+}
 
-// expert: of the thread's slot s0 + tid, -1 if there is none.  count: as above, the counts of the workgroup's own slots still
-// zero.
-__device__ __forceinline__ void moe_place(int32_t* count, int32_t* part, int expert, int s0, int E, int k, bool write_offs, int32_t* offs,
-                                          int32_t* row_token, int32_t* token_rows) {
+// expert: of the thread's slot s0 + tid, -1 if there is none.  cursor: a row of E words for each wave, zero in all of them.
+// others: E counts of the slots before the workgroup's own, then those of the slots behind them, complete at the next barrier;
+// null: there are no other slots.
+__device__ __forceinline__ void moe_place(int32_t* cursor, const int32_t* others, int32_t* part, int expert, int s0, int E, int k,
+                                          bool write_offs, int32_t* offs, int32_t* row_token, int32_t* token_rows) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int32_t* const cursor = count + 2 * kPlaceCopies * E;
-  if (expert >= 0) atomicAdd(&cursor[wave * E + expert], 1);
+  const bool live = expert >= 0;
+  const int bits = E > 1 ? 32 - __clz(E - 1) : 0;
+  uint64_t same = __ballot(live);   // the wave's slots of the same expert
+  for (int bit = 0; bit < bits; ++bit) {
+    const bool on = (expert >> bit) & 1;
+    const uint64_t with_bit = __ballot(on && live);
+    same &= on ? with_bit : ~with_bit;
+  }
+  const int rank = __popcll(same & ((uint64_t(1) << lane) - 1));
+  if (live && rank == 0) cursor[wave * E + expert] = __popcll(same);
   __syncthreads();
   // thread e owns expert e: prefix over the experts, then over the waves
   int before = 0, total = 0;
   if (tid < E) {
-    for (int c = 0; c < kPlaceCopies; ++c) {
-      before += count[c * E + tid];
-      total += count[(kPlaceCopies + c) * E + tid];
+    if (others) {
+      before = others[tid];
+      total = others[E + tid];
     }
     total += before;
     for (int w = 0; w < kPlaceWaves; ++w) total += cursor[w * E + tid];
@@ -293,8 +309,8 @@ __device__ __forceinline__ void moe_place(int32_t* count, int32_t* part, int exp
   int incl = total;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const int up = __shfl_up(incl, o);
-    if (lane >= o) incl += up;
+    const int v = __shfl_up(incl, o);
+    if (lane >= o) incl += v;
   }
   if (lane == 63) part[wave] = incl;
   __syncthreads();
@@ -310,16 +326,8 @@ __device__ __forceinline__ void moe_place(int32_t* count, int32_t* part, int exp
     }
   }
   __syncthreads();
-  const bool live = expert >= 0;
-  const int bits = E > 1 ? 32 - __clz(E - 1) : 0;
-  uint64_t same = __ballot(live);
-  for (int bit = 0; bit < bits; ++bit) {
-    const bool on = (expert >> bit) & 1;
-    const uint64_t with_bit = __ballot(on && live);
-    same &= on ? with_bit : ~with_bit;
-  }
   if (live) {
-    const int row = cursor[wave * E + expert] + __popcll(same & ((uint64_t(1) << lane) - 1));
+    const int row = cursor[wave * E + expert] + rank;
     row_token[row] = (s0 + tid) / k;
     token_rows[s0 + tid] = row;
   }
@@ -328,25 +336,39 @@ __device__ __forceinline__ void moe_place(int32_t* count, int32_t* part, int exp
 __global__ void __launch_bounds__(kPlaceBlock) moe_place_kernel(const int32_t* __restrict__ slot_expert, int slots, int E, int k,
                                                                 int32_t* __restrict__ offs, int32_t* __restrict__ row_token,
                                                                 int32_t* __restrict__ token_rows) {
-  __shared__ int32_t count[kPlaceRows * kMaxExperts];
+  __shared__ __align__(16) int32_t words[kPlaceWords];
+  __shared__ int32_t sums[2 * kMaxExperts];
   __shared__ int32_t part[kPlaceWaves];
-  const int tid = threadIdx.x, copy = (tid >> 6) & (kPlaceCopies - 1), own = blockIdx.x;
+  const int tid = threadIdx.x, own = blockIdx.x, blocks = gridDim.x;
   const int expert = own * kPlaceBlock + tid < slots ? slot_expert[own * kPlaceBlock + tid] : -1;
-  for (int i = tid; i < kPlaceRows * E; i += kPlaceBlock) count[i] = 0;
+  const int copy_bits = place_copy_bits(E), copy = tid & ((1 << copy_bits) - 1);
+  int32_t* const count = words + kPlaceWaves * E;
+  for (int i = tid; i < (kPlaceWaves + (blocks > 1 ? 2 << copy_bits : 0)) * E / 4; i += kPlaceBlock)
+    reinterpret_cast<int4*>(words)[i] = make_int4(0, 0, 0, 0);
   __syncthreads();
-  const int blocks = gridDim.x;
-  for (int b0 = 0; b0 < blocks; b0 += 8) {
-    int e[8];
+  if (blocks > 1) {
+    for (int b0 = 0; b0 < blocks; b0 += 8) {
+      int e[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int s = (b0 + i) * kPlaceBlock + tid;
-      e[i] = b0 + i != own && s < slots ? slot_expert[s] : -1;
+      for (int i = 0; i < 8; ++i) {
+        const int s = (b0 + i) * kPlaceBlock + tid;
+        e[i] = b0 + i != own && s < slots ? slot_expert[s] : -1;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (e[i] >= 0) atomicAdd(&count[(((b0 + i < own ? 0 : E) + e[i]) << copy_bits) + copy], 1);
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (e[i] >= 0) atomicAdd(&count[(b0 + i < own ? copy : kPlaceCopies + copy) * E + e[i]], 1);
+    __syncthreads();
+    // a count's words: four to a lane, the lanes next to each other
+    const int lanes = 1 << (copy_bits - 2);
+    for (int i = tid; i < 2 * E * lanes; i += kPlaceBlock) {
+      const int4 v = reinterpret_cast<const int4*>(count)[i];
+      int sum = v.x + v.y + v.z + v.w;
+      for (int o = lanes >> 1; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+      if ((i & (lanes - 1)) == 0) sums[i >> (copy_bits - 2)] = sum;
+    }
   }
-  moe_place(count, part, expert, own * kPlaceBlock, E, k, own == 0, offs, row_token, token_rows);
+  moe_place(words, blocks > 1 ? sums : nullptr, part, expert, own * kPlaceBlock, E, k, own == 0, offs, row_token, token_rows);
 }
 
 // The whole routing of a decoding step, one launch: 16 tokens at a time, one to a wave, the next one's logits on their way while
@@ -363,13 +385,13 @@ __global__ void __launch_bounds__(kPlaceBlock) moe_route_kernel(const T* __restr
                                                                 int32_t* __restrict__ offs, int32_t* __restrict__ slot_expert,
                                                                 float* __restrict__ slot_weight, int32_t* __restrict__ row_token,
                                                                 int32_t* __restrict__ token_rows) {
-  __shared__ int32_t count[kPlaceRows * kMaxExperts];
+  __shared__ int32_t cursor[kPlaceWaves * kMaxExperts];
   __shared__ int32_t part[kPlaceWaves];
   __shared__ int32_t chosen[kPlaceBlock];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   MoeTopk<T, kPer> next;
   if (wave < tokens) next.load(logits + int64_t(wave) * ld, E, lane);
-  for (int i = tid; i < kPlaceRows * E; i += kPlaceBlock) count[i] = 0;
+  for (int i = tid; i < kPlaceWaves * E; i += kPlaceBlock) cursor[i] = 0;
   for (int t = wave; t < tokens; t += kPlaceWaves) {
     const MoeTopk<T, kPer> token = next;
     if (t + kPlaceWaves < tokens) next.load(logits + int64_t(t + kPlaceWaves) * ld, E, lane);
@@ -383,7 +405,7 @@ __global__ void __launch_bounds__(kPlaceBlock) moe_route_kernel(const T* __restr
     }
   }
   __syncthreads();
-  moe_place(count, part, tid < tokens * k ? chosen[tid] : -1, 0, E, k, true, offs, row_token, token_rows);
+  moe_place(cursor, nullptr, part, tid < tokens * k ? chosen[tid] : -1, 0, E, k, true, offs, row_token, token_rows);
 }
 
 // ---------------------------------------------------------------- activation

@@ -69,6 +69,17 @@ def test_routing_at_the_edges_of_its_kernels(T, E, k):
         check_routing(moe.moe_route(logits.to(DEV), k, renormalize=renorm), moe_oracle.route(logits, k, renorm))
 
 
+@pytest.mark.parametrize("T,E,k", [(3000, 1, 1), (32768, 8, 1), (9000, 8, 2), (5000, 64, 3), (4500, 409, 2), (4500, 410, 2), (4097, 1023, 1), (131072, 3, 1)])
+def test_routing_when_tokens_crowd_few_experts(T, E, k):
+    """Equal logits (padding: every token takes the first experts) and one expert ahead of all others, in blocks with ordinary tokens
+    between them: the counts of many slots on one expert, before, in and behind a workgroup's own."""
+    gen = torch.Generator().manual_seed(T + E)
+    logits = torch.randn(T, E, generator=gen)
+    logits[: T // 3] = 0.0
+    logits[T // 2:, E - 1] = 9.0
+    check_routing(moe.moe_route(logits.to(DEV), k), moe_oracle.route(logits, k, True))
+
+
 def test_routing_fp16_skewed_padded_and_empty():
     gen = torch.Generator().manual_seed(3)
     # skew: most tokens pick expert 0, several experts stay empty
