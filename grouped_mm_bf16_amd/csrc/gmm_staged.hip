@@ -26,6 +26,8 @@
 //     with a check per chunk, without branches, in a loop of their own.
 //   * What bounds it: 16-bit, 4 x 4 blocks per wave: LDS reads and writes take 1.5 times the cycles of the MFMAs; fp32:
 //     the MFMA pipe (64 to 75 % busy), the rest is the last, partly filled round.
+#include <cmath>
+
 #include "gmm_device.h"
 #include "gmm_launch.h"
 
@@ -348,6 +350,17 @@ __device__ __forceinline__ bool join_parts(const GmmParams& p, const GmmTile& ti
   return true;
 }
 
+// Parts of each of the `tail` tiles of a last, partly filled round behind `whole` tiles on `wgs` workgroups: as many as there are
+// places for, and behind whole rounds only if that makes four of each.  Places: the workgroups; behind whole rounds of 64 x 64
+// tiles, four of which share a CU's matrix cores, half of them (a tile that is alone on its CU already runs three times as fast as
+// in a full round).
+__host__ __device__ inline int tail_parts(int tail, int whole, int wgs, int edge, const GmmParams& p) {
+  if (tail == 0) return 1;
+  const int places = edge == 64 && whole ? wgs / 2 : wgs, room = places < p.k_parts ? places : p.k_parts;
+  const int parts = room / tail < p.k_split ? room / tail : p.k_split;
+  return parts < (whole ? 4 : 2) ? 1 : parts;
+}
+
 // SPLIT = 1: a jagged contraction whose groups may be cut along K.  SPLIT = 2: any other product, the tiles of the last round
 // cut along K.
 template <typename T, typename OutT, bool A_TR, bool B_TR, int EDGE, int SPLIT>
@@ -377,13 +390,8 @@ __global__ void __launch_bounds__(NT, tile_wgs(EDGE)) gmm_staged_kernel(const Gm
     return __builtin_amdgcn_readfirstlane(in_registers ? groups.build(p, BM, BN, chunk) : gmm_build_tile_table<NT>(p, BM, BN, cum, chunk));
   };
   int total = build();
-  // the tiles of the last, partly filled round: each in as many parts as there are places for, and behind whole rounds only if
-  // that makes four of each.  Places: the workgroups; behind whole rounds of 64 x 64 tiles, four of which share a CU's matrix
-  // cores, half of them (a tile that is alone on its CU already runs three times as fast as in a full round).
   const int tail = SPLIT == 2 ? total % int(gridDim.x) : 0, whole = total - tail;
-  const int places = EDGE == 64 && whole ? int(gridDim.x) / 2 : int(gridDim.x);
-  int split = SPLIT == 2 && tail ? gmm_max(gmm_min(p.k_split, gmm_min(places, p.k_parts) / tail), 1) : 1;
-  if (SPLIT == 2 && whole && split < 4) split = 1;
+  const int split = SPLIT == 2 ? tail_parts(tail, whole, gridDim.x, EDGE, p) : 1;
   if (SPLIT == 2) total = whole + tail * split;
   if (SPLIT == 1 && chunk && total > p.k_parts) {   // offsets that overlap: more parts than K elements have room for
     chunk = 0;
@@ -618,12 +626,37 @@ bool split_tiles(GmmParams& p, int64_t most_wgs) {
   return true;
 }
 
-// Cut the tiles of the last round along K where it holds only a few?  The device knows how many; launches of one to four
-// rounds with at least 24 K tiles can have a use for it.  us, whole / cut: fp32 1024 x 1024 x 8192 columns in 8 groups (2.1
-// rounds) 165 / 157, 8192 x 1024 x 4096 in 8 groups 617 / 577; bf16 8191 x 2047 x 2047 in 8 groups 157 / 148, 5 products of 7 x
-// 13204 x 2148 (520 tiles, 512 workgroups) 99 / 71.  400 random launches: 1.4 at best, 0.96 at worst, uncut ones among them.
+// Does a number of tiles that the launch may well have leave a last round that is cut?  p.k_split and p.k_parts are set.
+bool may_be_cut(const GmmParams& p, int edge, int wgs) {
+  const int tm = (p.M + edge - 1) / edge, tn = (p.N + edge - 1) / edge;
+  int lo = p.G * tm, hi = lo, step = tn;      // step times so many tiles
+  if (p.jag != GMM_JAG_NONE) {
+    const bool rows = p.jag == GMM_JAG_M;
+    const int extent = rows ? p.M : p.N, groups = p.G < extent ? p.G : extent;
+    const float middle = float(extent) / edge + 0.5f * groups, away = 2.0f * sqrtf(groups / 12.0f);
+    step = rows ? tn : tm;
+    lo = int(ceilf(middle - away));
+    hi = int(floorf(middle + away));
+    if (lo < (rows ? tm : tn)) lo = rows ? tm : tn;
+  }
+  for (int n = lo; n <= hi; ++n) {
+    const int tiles = n * step, tail = tiles % wgs;
+    if (tail_parts(tail, tiles - tail, wgs, edge, p) > 1) return true;
+  }
+  return false;
+}
+
+// Cut the tiles of the last round along K where it holds only a few?  Only the device knows how many there are, and the kernel
+// that can cut them is 0.6 % slower where it does not (up to 4.5 %), a captured launch also clears a workspace for it (2 us).  So
+// launches of one to four rounds with at least 24 K tiles that may well be cut: equal products make a known number of tiles;
+// groups end anywhere in a tile, each makes half a tile more on average, all together with a deviation of the square root of
+// G / 12, and a number up to two deviations away has to be one that is cut.  us, whole / cut: fp32 1024 x 1024 x 8192 columns in 8
+// uneven groups (2.1 rounds) 166 / 159; bf16 8191 x 2047 x 2047 in 8 groups 142 / 135, 5 products of 7 x 13204 x 2148 (520 tiles,
+// 512 workgroups) 97 / 69.  544 random launches of such sizes: 56 are cut, 1.13
+// times as fast (1.0 to 1.41), the other 488 as fast as without a workspace (0.999; 0.994 when all of them ran the kernel that can cut).
 template <int EDGE>
 bool split_tail(GmmParams& p, int64_t most_wgs, int esz) {
+  p.k_split = 0;
   if (p.jag == GMM_JAG_K || p.ws_parts <= 0 || int64_t(p.K) * esz < 24 * ROW_BYTES) return false;
   const int64_t tiles = expected_tiles(p, EDGE);
   int64_t room = int64_t(p.ws_parts) * GMM_WS_SLOT / (EDGE * EDGE * 4);
@@ -631,7 +664,9 @@ bool split_tail(GmmParams& p, int64_t most_wgs, int esz) {
   if (tiles <= most_wgs || tiles > 4 * most_wgs) return false;
   p.k_split = p.K / (GMM_K_SPLIT_MIN / 2) < GMM_K_CLUSTER ? p.K / (GMM_K_SPLIT_MIN / 2) : GMM_K_CLUSTER;
   p.k_parts = int32_t(room);
-  return true;
+  if (may_be_cut(p, EDGE, int(most_wgs))) return true;
+  p.k_split = 0;
+  return false;
 }
 
 template <typename T, typename OutT, int EDGE>

@@ -93,16 +93,22 @@ def test_replays_leave_the_streams_workspace_alone(name):
 
 
 @pytest.mark.gpu
-def test_launch_without_a_use_for_a_workspace_is_captured_as_it_is():
-    a = torch.randn(64, 64, device=DEV, dtype=torch.bfloat16)
-    b = torch.randn(2, 64, 64, device=DEV, dtype=torch.bfloat16)
-    offs, out = _offs([10, 54]), torch.empty(64, 64, device=DEV, dtype=torch.bfloat16)
-    K_.grouped_mm_2d3d(a, b, offs, out)
+@pytest.mark.parametrize("sizes,G,M,K,N,dtype", [
+    ([10, 54], 2, 64, 64, 64, torch.bfloat16),
+    # a last round of 168 tiles of 1024, of 129 of 512, and, whichever way the rows are split, of 160 to 176 of 512: too many to cut
+    (None, 27, 130, 801, 2500, torch.float32), (None, 1, 81, 1601, 641 * 128 - 1, torch.bfloat16),
+    ([2700, 2600], 2, 5300, 1601, 2047, torch.bfloat16)])
+def test_launch_without_a_use_for_a_workspace_is_captured_as_it_is(sizes, G, M, K, N, dtype):
+    a = torch.randn((G, M, K) if sizes is None else (M, K), device=DEV).to(dtype)
+    b, out = torch.randn(G, K, N, device=DEV).to(dtype), torch.empty((G, M, N) if sizes is None else (M, N), device=DEV, dtype=dtype)
+    offs = None if sizes is None else _offs(sizes)
+    launch = lambda: K_.grouped_mm_3d3d(a, b, out) if offs is None else K_.grouped_mm_2d3d(a, b, offs, out)
+    launch()
     torch.cuda.synchronize()
     before = torch.cuda.memory_reserved()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        K_.grouped_mm_2d3d(a, b, offs, out)
+        launch()
     assert torch.cuda.memory_reserved() - before < 1 << 20
 
 
