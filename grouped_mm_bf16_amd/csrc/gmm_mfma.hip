@@ -469,6 +469,21 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   GmmKQueue q;
   if constexpr (QUEUE) q.build<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, reinterpret_cast<uint32_t*>(lds));
   else total_tiles = gmm_build_tile_table2<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, total_tall);
+  bool renumber = p.xcd_remap != 0;
+  if constexpr (!A_TR && B_TR && !QUEUE) {
+    if (p.xcd_remap == GMM_REMAP_SHARED) {
+      int shared = 0;   // tiles of groups of several rows of them
+      for (int g = tid; g < p.G; g += WAVES * 64) {
+        const int tiles = cum_tall[g + 1] - cum_tall[g] + cum_short[g + 1] - cum_short[g];
+        shared += tiles > gmm_cdiv(p.N, GMM_TILE_N) ? tiles : 0;
+      }
+      if (tid == 0) split_flag = 0;
+      __syncthreads();
+      if (shared) atomicAdd(&split_flag, shared);
+      __syncthreads();
+      renumber = __builtin_amdgcn_readfirstlane(split_flag) > total_tiles / 8;
+    }
+  }
   // The tiles of the last, partly filled round may be cut along K into `nparts` parts each (gmm_tail_split).
   // Tiles before split_base are dealt round-robin (workgroup w takes w, w + grid, ...); the parts are taken
   // from a ticket counter in the workspace by whichever workgroup is free: part q is K part q / tail of tile
@@ -497,7 +512,7 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
       }
     } else if (tid < BATCH && mine < split_base) {
       const int t = int(mine);
-      const int tt = p.xcd_remap ? gmm_xcd_remap(t, split_base, gridDim.x) : t;
+      const int tt = renumber ? gmm_xcd_remap(t, split_base, gridDim.x) : t;
       gmm_store_rec(&tiles[tid], gmm_locate_tile2(p, cum_tall, cum_short, total_tall, tt, GMM_TILE_N), -1);
     }
     __syncthreads();
@@ -636,16 +651,19 @@ int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
   return gmm_use_k_queue(p, GMM_TILE_N, p.num_wg) ? launch_asm<OUT_F32, F16, 1>(p, lay, stream) : launch_asm<OUT_F32, F16, 0>(p, lay, stream);
 }
 
-// Launches whose tiles are not renumbered for the XCDs.  Where every group is one row of tiles (decoding; judged by the rows of a
-// group on average) there is nothing worth an L2, the second operand is read once.  If such a row is more than an XCD's share of
-// a round, the chip then reads 128 KB that lie side by side in memory in launch order, and eight times 16 KB renumbered: 8 groups
-// of 4096 x 28672, 64 rows in all, 303 -> 290 us (6.5 TB/s; plain reads of such pieces 6.3 and 6.0), 16 of 2048 x 14336 157 ->
-// 151.  Short reads pay for pages that eight XCDs share: 24 products of 8 x 8192 x 1024 69 us renumbered, 72 in launch order, 24
-// of 8 x 28672 x 256 83 and 85; narrow groups: a decoding step with 128 groups of 2048 x 1536 200.4 and 201.8.
-bool stays_in_order(const GmmParams& p, int num_cus) {
+// Launches whose tiles are not renumbered for the XCDs.  Where every group is one row of tiles (decoding) there is nothing worth an
+// L2, the second operand is read once.  If such a row is more than an XCD's share of a round, the chip then reads 128 KB of a
+// row-major matrix that lie side by side in memory in launch order, and eight times 16 KB renumbered.  us, renumbered / in launch
+// order: 8 groups of 4096 x 28672, 64 rows in all 305 / 291 (6.5 TB/s; plain reads of such pieces 6.0 and 6.3), 16 of 2048 x 14336
+// 166 / 159.  A column-major matrix lies in memory tile by tile: 354 / 364 and 206 / 214.  Tiles of a group of several rows share it:
+// all 256 rows in one of those 8 groups 55 / 76, 249 of them (a fifth of the tiles) 297 / 312; 500 of 810 rows in one of 32 groups of
+// 2048 x 16384 (a ninth) 374 / 353.  So the kernel looks at the groups and renumbers if they hold more than an eighth.
+// Short reads pay for pages that eight XCDs share: 24 products of 8 x 8192 x 1024 69 / 72, 24 of 8 x 28672 x 256 83 / 85; narrow
+// groups: a decoding step with 128 groups of 2048 x 1536 200.4 / 201.8.
+bool may_stay_in_order(const GmmParams& p, GmmLayout lay, int num_cus) {
   const bool few = p.jag == GMM_JAG_M ? int64_t(p.M) <= 32 * int64_t(p.G) : p.jag == GMM_JAG_NONE && p.M <= 64;
   const int64_t groups = p.jag == GMM_JAG_M ? gmm_min(p.G, p.M) : p.G;
-  return few && p.N >= 48 * 256 && p.K >= 1024 && 4 * groups * gmm_cdiv(p.N, 256) >= 3 * int64_t(num_cus);
+  return few && lay.a_kc && !lay.b_kc && p.N >= 48 * 256 && p.K >= 1024 && 4 * groups * gmm_cdiv(p.N, 256) >= 3 * int64_t(num_cus);
 }
 
 // Grid, tile heights and use of the workspace of a launch.
@@ -681,7 +699,8 @@ bool gmm_mfma_uses_workspace(GmmParams p, GmmLayout lay, int config, int num_cus
 
 int gmm_launch_mfma(GmmParams p, GmmLayout lay, int in_dtype, int out_dtype, int config, int num_cus, hipStream_t stream) {
   plan(p, lay, config, num_cus);
-  if (config == GMM_CFG_ASM_256x256 && stays_in_order(p, num_cus)) p.xcd_remap = 0;
+  if (config == GMM_CFG_ASM_256x256 && p.xcd_remap && may_stay_in_order(p, lay, num_cus))
+    p.xcd_remap = p.jag == GMM_JAG_M ? GMM_REMAP_SHARED : 0;
   const bool out16 = out_dtype == in_dtype;   // else fp32
   if (!out16 && out_dtype != GMM_DT_F32) return -1;
   if (config == GMM_CFG_ASM_256x256) {

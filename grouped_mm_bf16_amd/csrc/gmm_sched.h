@@ -27,6 +27,7 @@ enum GmmJag : int32_t { GMM_JAG_NONE = 0, GMM_JAG_M = 1, GMM_JAG_N = 2, GMM_JAG_
 
 constexpr int GMM_MAX_GROUPS = 1024;  // offs.numel() < 1024 is enforced by the host layer
 constexpr int GMM_BAND = 8;           // tile rows per band in the within-group tile order
+constexpr int GMM_REMAP_SHARED = 2;   // GmmParams::xcd_remap: the kernel decides, from the tiles that have others to share with
 
 // Everything a kernel needs to know about one call.  Strides are in elements.
 struct GmmParams {
@@ -41,7 +42,7 @@ struct GmmParams {
   int64_t a_sg, a_sm, a_sk;
   int64_t b_sg, b_sk, b_sn;
   int64_t c_sg, c_sm, c_sn;
-  int32_t xcd_remap;  // 1: renumber tiles so that each XCD works on a compact block
+  int32_t xcd_remap;  // 1: renumber tiles so that each XCD works on a compact block; GMM_REMAP_SHARED: if it shares enough
   int32_t num_wg;     // persistent grid size
   int32_t tall;       // tile list with several heights: rows of a "tall" tile (256 or 128) ...
   int32_t shrt;       // ... and of the shortest tile for group remainders (64), or 0: tall tiles only

@@ -175,26 +175,30 @@ def test_small_groups_on_every_tile_height(K, N, b_col, tall, shrt):
     assert K_.last_kernel() == ("any" if (tall, K) == (-1, 72) else "assembly")
 
 
+@pytest.mark.parametrize("b_col", [False, True])
 @pytest.mark.parametrize("sizes,N,K", [([8] * 8, 12288, 1024), ([30, 0, 1, 33, 64, 0, 3, 125], 12288, 1024), ([64] * 2, 28672, 1032),
-                                       ([8] * 8, 12280, 1024), ([8] * 8, 12288, 1016)])
-def test_launch_order_of_wide_decoding_products(sizes, N, K):
-    """Both sides of the line between launches in order and renumbered ones: the same bits."""
+                                       ([8] * 8, 12280, 1024), ([8] * 8, 12288, 1016), ([0, 249] + [1] * 6, 12288, 1024),
+                                       ([129] + [2] * 14, 12288, 1024), ([129] + [2] * 13, 12288, 1024)])
+def test_launch_order_of_wide_decoding_products(sizes, N, K, b_col):
+    """Both sides of the lines between launches in order and renumbered ones (two of 16 and of 15 rows of tiles in one group
+    among them): as asked for, and always in order.  Every element of both against fp32 products, and bit for bit."""
     gen = torch.Generator(device=DEV).manual_seed(N + K)
     a = torch.randn(sum(sizes), K, device=DEV, generator=gen).bfloat16()
     b = torch.randn(len(sizes), K, N, device=DEV, generator=gen).bfloat16()
+    bv = b.transpose(1, 2).contiguous().transpose(1, 2) if b_col else b
     outs = []
     for remap in (1, 0):
         prev = K_._lib.load().gmm_set_xcd_remap(remap)
         try:
             outs.append(torch.full((sum(sizes), N), float("nan"), device=DEV, dtype=torch.bfloat16))
             with K_.tail_split(False):
-                K_.grouped_mm_2d3d(a, b, offs_of(sizes).to(DEV), outs[-1])
+                K_.grouped_mm_2d3d(a, bv, offs_of(sizes).to(DEV), outs[-1])
         finally:
             K_._lib.load().gmm_set_xcd_remap(prev)
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
-    g = len(sizes) - 1
-    lo = sum(sizes[:g])
-    oracle.assert_close(outs[0][lo:, :512].cpu(), (a[lo:].float() @ b[g, :, :512].float()).bfloat16().cpu(), K)
+    for g, lo in enumerate([0] + offs_of(sizes).tolist()[:-1]):
+        if sizes[g]:
+            oracle.assert_close(outs[0][lo:lo + sizes[g]].cpu(), (a[lo:lo + sizes[g]].float() @ b[g].float()).bfloat16().cpu(), K)
 
 
 def test_output_larger_than_4_gib():
