@@ -444,11 +444,15 @@ __device__ __forceinline__ GmmTileDesc gmm_describe_tile(const GmmParams& p, con
   return dsc;
 }
 
-// QUEUE = 1: jagged contraction, the longest groups' tiles first, drawn on demand (GmmKQueue).  A kernel of its own: with
-// both ways in one, every other launch took 1.6 us longer.
-template <int A_TR, int B_TR, int OUT_F32, int F16, int ACT = 0, int QUEUE = 0>
+// ORDER = ORDER_QUEUE: jagged contraction, the longest groups' tiles first, drawn on demand (GmmKQueue).  ORDER_SHARED: renumbered
+// for the XCDs only if groups share enough tiles (may_stay_in_order).  Kernels of their own: with the queue in one with the others,
+// every other launch took 1.6 us longer, with the look at the groups 0.3 (111235 rows in 197 groups, 144 to 104, 34.7 us).
+constexpr int ORDER_PLAIN = 0, ORDER_QUEUE = 1, ORDER_SHARED = 2;
+
+template <int A_TR, int B_TR, int OUT_F32, int F16, int ACT = 0, int ORDER = ORDER_PLAIN>
 __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   constexpr int WAVES = 4;
+  constexpr bool QUEUE = ORDER == ORDER_QUEUE;
   constexpr bool SHORT_TILES = !A_TR;
   constexpr int LDS_256 = gmm_tile_lds_bytes<A_TR, B_TR, 4>();
   constexpr int LDS_128 = SHORT_TILES ? gmm_tile_lds_bytes<0, B_TR, 2>() : 0;
@@ -470,19 +474,17 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   if constexpr (QUEUE) q.build<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, reinterpret_cast<uint32_t*>(lds));
   else total_tiles = gmm_build_tile_table2<WAVES * 64>(p, GMM_TILE_N, cum_tall, cum_short, total_tall);
   bool renumber = p.xcd_remap != 0;
-  if constexpr (!A_TR && B_TR && !QUEUE) {
-    if (p.xcd_remap == GMM_REMAP_SHARED) {
-      int shared = 0;   // tiles of groups of several rows of them
-      for (int g = tid; g < p.G; g += WAVES * 64) {
-        const int tiles = cum_tall[g + 1] - cum_tall[g] + cum_short[g + 1] - cum_short[g];
-        shared += tiles > gmm_cdiv(p.N, GMM_TILE_N) ? tiles : 0;
-      }
-      if (tid == 0) split_flag = 0;
-      __syncthreads();
-      if (shared) atomicAdd(&split_flag, shared);
-      __syncthreads();
-      renumber = __builtin_amdgcn_readfirstlane(split_flag) > total_tiles / 8;
+  if constexpr (ORDER == ORDER_SHARED) {
+    int shared = 0;   // tiles of groups of several rows of them
+    for (int g = tid; g < p.G; g += WAVES * 64) {
+      const int tiles = cum_tall[g + 1] - cum_tall[g] + cum_short[g + 1] - cum_short[g];
+      shared += tiles > gmm_cdiv(p.N, GMM_TILE_N) ? tiles : 0;
     }
+    if (tid == 0) split_flag = 0;
+    __syncthreads();
+    if (shared) atomicAdd(&split_flag, shared);
+    __syncthreads();
+    renumber = __builtin_amdgcn_readfirstlane(split_flag) > total_tiles / 8;
   }
   // The tiles of the last, partly filled round may be cut along K into `nparts` parts each (gmm_tail_split).
   // Tiles before split_base are dealt round-robin (workgroup w takes w, w + grid, ...); the parts are taken
@@ -601,33 +603,38 @@ __global__ void __launch_bounds__(256, 1) gmm_asm_kernel(const GmmParams p) {
   }
 }
 
-template <int OUT_F32, int F16, int QUEUE>
+template <int B_TR, int OUT_F32, int F16, int ORDER>
+int launch_swiglu(const GmmParams& p, hipStream_t stream) {
+  if constexpr (OUT_F32 || ORDER == ORDER_QUEUE) {
+    return -1;
+  } else {
+    const dim3 grid(p.num_wg), block(256);
+    if (p.act == 3)
+      hipLaunchKernelGGL((gmm_asm_kernel<0, B_TR, 0, F16, 3, ORDER>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((gmm_asm_kernel<0, B_TR, 0, F16, 1, ORDER>), grid, block, 0, stream, p);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+  }
+}
+
+template <int OUT_F32, int F16, int ORDER>
 int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
   const dim3 grid(p.num_wg), block(256);
-  if (p.act) {
-    if constexpr (OUT_F32 || QUEUE) {
-      return -1;
-    } else {
-      if (!lay.a_kc) return -1;
-      if (p.act == 3 && lay.b_kc)
-        hipLaunchKernelGGL((gmm_asm_kernel<0, 0, 0, F16, 3>), grid, block, 0, stream, p);
-      else if (p.act == 3)
-        hipLaunchKernelGGL((gmm_asm_kernel<0, 1, 0, F16, 3>), grid, block, 0, stream, p);
-      else if (lay.b_kc)
-        hipLaunchKernelGGL((gmm_asm_kernel<0, 0, 0, F16, 1>), grid, block, 0, stream, p);
-      else
-        hipLaunchKernelGGL((gmm_asm_kernel<0, 1, 0, F16, 1>), grid, block, 0, stream, p);
-      return hipGetLastError() == hipSuccess ? 0 : 1;
-    }
+  if constexpr (ORDER == ORDER_SHARED) {      // K-contiguous first operand, row-major second one
+    if (p.act) return launch_swiglu<1, OUT_F32, F16, ORDER>(p, stream);
+    hipLaunchKernelGGL((gmm_asm_kernel<0, 1, OUT_F32, F16, 0, ORDER>), grid, block, 0, stream, p);
+  } else {
+    if (p.act && !lay.a_kc) return -1;
+    if (p.act) return lay.b_kc ? launch_swiglu<0, OUT_F32, F16, ORDER>(p, stream) : launch_swiglu<1, OUT_F32, F16, ORDER>(p, stream);
+    if (lay.a_kc && lay.b_kc)
+      hipLaunchKernelGGL((gmm_asm_kernel<0, 0, OUT_F32, F16, 0, ORDER>), grid, block, 0, stream, p);
+    else if (lay.a_kc && !lay.b_kc)
+      hipLaunchKernelGGL((gmm_asm_kernel<0, 1, OUT_F32, F16, 0, ORDER>), grid, block, 0, stream, p);
+    else if (!lay.a_kc && lay.b_kc)
+      hipLaunchKernelGGL((gmm_asm_kernel<1, 0, OUT_F32, F16, 0, ORDER>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((gmm_asm_kernel<1, 1, OUT_F32, F16, 0, ORDER>), grid, block, 0, stream, p);
   }
-  if (lay.a_kc && lay.b_kc)
-    hipLaunchKernelGGL((gmm_asm_kernel<0, 0, OUT_F32, F16, 0, QUEUE>), grid, block, 0, stream, p);
-  else if (lay.a_kc && !lay.b_kc)
-    hipLaunchKernelGGL((gmm_asm_kernel<0, 1, OUT_F32, F16, 0, QUEUE>), grid, block, 0, stream, p);
-  else if (!lay.a_kc && lay.b_kc)
-    hipLaunchKernelGGL((gmm_asm_kernel<1, 0, OUT_F32, F16, 0, QUEUE>), grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL((gmm_asm_kernel<1, 1, OUT_F32, F16, 0, QUEUE>), grid, block, 0, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -648,7 +655,8 @@ int launch_layout(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
 
 template <int OUT_F32, int F16>
 int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
-  return gmm_use_k_queue(p, GMM_TILE_N, p.num_wg) ? launch_asm<OUT_F32, F16, 1>(p, lay, stream) : launch_asm<OUT_F32, F16, 0>(p, lay, stream);
+  if (gmm_use_k_queue(p, GMM_TILE_N, p.num_wg)) return launch_asm<OUT_F32, F16, ORDER_QUEUE>(p, lay, stream);
+  return p.xcd_remap == GMM_REMAP_SHARED ? launch_asm<OUT_F32, F16, ORDER_SHARED>(p, lay, stream) : launch_asm<OUT_F32, F16, ORDER_PLAIN>(p, lay, stream);
 }
 
 // Launches whose tiles are not renumbered for the XCDs.  Where every group is one row of tiles (decoding) there is nothing worth an

@@ -374,12 +374,16 @@ __global__ void __launch_bounds__(kPlaceBlock) moe_place_kernel(const int32_t* _
 }
 
 // The whole routing of a decoding step, one launch: 16 tokens at a time, one to a wave, the next one's logits on their way while
-// one chooses.  Worth it while no wave makes more than kRouteChoices choices beyond its first token's: a choice takes 0.28 us,
-// the second launch 3 us.  1 token, 8 of 128 experts 8.9 -> 5.0 us, 32 tokens, 2 of 8 6.9 -> 4.8; 64 tokens, 8 of 128 13.6 (24
-// choices more) against 7.7 in two launches.
-constexpr int kRouteChoices = 8;
-bool route_in_one(int64_t tokens, int64_t top_k) {
-  return tokens * top_k <= kPlaceBlock && ((tokens + kPlaceWaves - 1) / kPlaceWaves - 1) * top_k <= kRouteChoices;
+// one chooses.  It saves 1.1 us between two launches, but a compute unit's four SIMDs share the choices that otherwise spread over
+// the chip: a token takes one of them 0.03 us times (7 + choices * (keys of a lane + 1)), in rounds of 16 tokens.  Four tokens
+// have a SIMD each; more while a SIMD's share is up to 124 of those units.  us, one launch / two: 16 tokens, 8 of 128 experts 6.1 /
+// 6.9, 32 8.7 / 7.0; 48, 1 of 8 5.3 / 5.3, 144 9.7 / 5.5; 32, 2 of 8 5.0 / 5.4, 48 5.8 / 5.4; 32, 4 of 64 5.9 / 5.9, 48 7.0 / 5.9; 1, 8
+// of 512 8.8 / 9.8, 16 12.8 / 10.3.
+int lane_keys(int64_t E) { return E <= 64 ? 1 : E <= 128 ? 2 : E <= 256 ? 4 : E <= 512 ? 8 : E <= 768 ? 12 : 16; }
+bool route_in_one(int64_t tokens, int64_t E, int64_t top_k) {
+  if (tokens <= 4) return true;
+  const int64_t per_simd = tokens <= kPlaceWaves ? (tokens + 3) / 4 : (tokens + kPlaceWaves - 1) / kPlaceWaves * 4;
+  return tokens * top_k <= kPlaceBlock && per_simd * (7 + top_k * (lane_keys(E) + 1)) <= 124;
 }
 
 template <typename T, int kPer>
@@ -497,7 +501,7 @@ int route_checked(const void* logits, int64_t ld, int dtype, int64_t tokens, int
   if (size_t(pl.nb) * size_t(E) * sizeof(int32_t) > table_bytes) return GMM_ERR_WORKSPACE;
   if (pl.nb > 0 && !table) return GMM_ERR_BAD_ARGUMENT;
   if (tokens > 0) {
-    const bool one = route_in_one(tokens, top_k);
+    const bool one = route_in_one(tokens, E, top_k);
     const auto launch = [&](const auto* rows, auto per) {
       using T = std::remove_const_t<std::remove_pointer_t<decltype(rows)>>;
       constexpr int kPer = decltype(per)::value;
@@ -509,12 +513,14 @@ int route_checked(const void* logits, int64_t ld, int dtype, int64_t tokens, int
                            int(E), int(top_k), renorm, slot_expert, slot_weight);
     };
     const auto topk = [&](const auto* rows) {
-      if (E <= 64) launch(rows, std::integral_constant<int, 1>{});
-      else if (E <= 128) launch(rows, std::integral_constant<int, 2>{});
-      else if (E <= 256) launch(rows, std::integral_constant<int, 4>{});
-      else if (E <= 512) launch(rows, std::integral_constant<int, 8>{});
-      else if (E <= 768) launch(rows, std::integral_constant<int, 12>{});
-      else launch(rows, std::integral_constant<int, 16>{});
+      switch (lane_keys(E)) {
+        case 1: launch(rows, std::integral_constant<int, 1>{}); break;
+        case 2: launch(rows, std::integral_constant<int, 2>{}); break;
+        case 4: launch(rows, std::integral_constant<int, 4>{}); break;
+        case 8: launch(rows, std::integral_constant<int, 8>{}); break;
+        case 12: launch(rows, std::integral_constant<int, 12>{}); break;
+        default: launch(rows, std::integral_constant<int, 16>{}); break;
+      }
     };
     if (dtype == GMM_DT_BF16) topk(static_cast<const Bf16*>(logits));
     else if (dtype == GMM_DT_F16) topk(static_cast<const F16*>(logits));
