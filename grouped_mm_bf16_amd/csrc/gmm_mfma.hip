@@ -446,7 +446,8 @@ __device__ __forceinline__ GmmTileDesc gmm_describe_tile(const GmmParams& p, con
 
 // ORDER = ORDER_QUEUE: jagged contraction, the longest groups' tiles first, drawn on demand (GmmKQueue).  ORDER_SHARED: renumbered
 // for the XCDs only if groups share enough tiles (may_stay_in_order).  Kernels of their own: with the queue in one with the others,
-// every other launch took 1.6 us longer, with the look at the groups 0.3 (111235 rows in 197 groups, 144 to 104, 34.7 us).
+// every other launch took 1.6 us longer, with the look at the groups the SwiGLU kernels spilled 30 scalars more (546 tokens, 2 of 9
+// experts of 1624 to 2 x 13952 324 -> 327 us).
 constexpr int ORDER_PLAIN = 0, ORDER_QUEUE = 1, ORDER_SHARED = 2;
 
 template <int A_TR, int B_TR, int OUT_F32, int F16, int ACT = 0, int ORDER = ORDER_PLAIN>
