@@ -242,8 +242,7 @@ __device__ __forceinline__ void gmm_tile_compute(const GmmTileDesc& t, unsigned 
     if (t.sharers > 0) {
       const int per_tile = (256 + t.sharers - 1) / t.sharers, per_wave = (per_tile + 3) >> 2;
       const int idx = wave * per_wave + lane, line = t.share * per_tile + idx;
-      if (lane < per_wave && idx < per_tile && line < 256)
-{
+      if (lane < per_wave && idx < per_tile && line < 256) {
         int col = B_TR ? (line & 3) * 64 : line;
         if (ACT == 3) col = gmm_apart_column(col, t.b.apart);
         off_b = B_TR ? (line >> 2) * t.b.ld * 2 + col * 2 : col * t.b.ld * 2;

@@ -47,7 +47,7 @@ def test_routing_matches_the_oracle(T, E, k, dtype):
 
 @pytest.mark.parametrize("T,E,k", [(1, 1, 1), (4096, 3, 1), (4097, 3, 1), (128, 1023, 32), (129, 1023, 32), (585, 65, 7),
                                    (16, 128, 4), (1025, 64, 2)])
-def test_slots_at_the_edges_of_the_one_workgroup_sort(T, E, k):
+def test_slots_at_the_edges_of_a_workgroup(T, E, k):
     """A workgroup of 16 waves places 1024 slots, 64 to a wave."""
     gen = torch.Generator().manual_seed(T + E + k)
     logits = torch.randn(T, E, generator=gen)
@@ -60,7 +60,7 @@ def test_slots_at_the_edges_of_the_one_workgroup_sort(T, E, k):
                                    (131073, 5, 1), (4, 512, 8), (4, 513, 8), (700, 512, 4), (700, 513, 32), (90, 768, 32), (91, 769, 3), (48, 8, 1), (49, 8, 1),
                                    (32, 8, 2), (33, 8, 2), (17, 128, 8), (8, 256, 8), (9, 256, 8), (5, 512, 8), (4, 1023, 32), (5, 1023, 32)])
 def test_routing_at_the_edges_of_its_kernels(T, E, k):
-    """One launch while no wave chooses more than eight times beyond its first token, then 1024 slots to a workgroup, from
+    """One launch for a few tokens, the more the fewer experts and choices, then 1024 slots to a workgroup, from
     131073 slots on a table of counts; 64, 128, 256, 512 and 768 experts to a lane's registers.  Ties and masked experts among them."""
     gen = torch.Generator().manual_seed(T + E + k)
     logits = torch.randn(T, E, generator=gen).round(decimals=1)
@@ -551,6 +551,12 @@ def test_custom_ops_pass_opcheck_and_match_the_direct_calls():
     h = moe.grouped_mm_gathered(xd, r.row_token, wu, r.offs)
     assert torch.equal(ops.gathered(xd, r.row_token, wu, r.offs).view(torch.int16), h.view(torch.int16))
     torch.library.opcheck(ops.gathered.default, (xd, r.row_token, wu, r.offs), test_utils=checks)
+    up = moe.moe_activation(h, "swiglu")
+    for weights in (wu, wu[:, :, : I + 16]):      # one kernel, and two where the columns are no multiple of 128
+        got = ops.gate_up(xd, r.row_token, weights, r.offs)
+        want = up if weights is wu else moe.moe_activation(moe.grouped_mm_gathered(xd, r.row_token, weights, r.offs), "swiglu")
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+        torch.library.opcheck(ops.gate_up.default, (xd, r.row_token, weights, r.offs), test_utils=checks)
     wil = moe.interleave_gate_up(wu)
     fused = moe.grouped_mm_swiglu(xd, r.row_token, wil, r.offs)
     assert torch.equal(ops.swiglu(xd, r.row_token, wil, r.offs).view(torch.int16), fused.view(torch.int16))
