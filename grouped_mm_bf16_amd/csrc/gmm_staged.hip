@@ -351,12 +351,13 @@ __device__ __forceinline__ bool join_parts(const GmmParams& p, const GmmTile& ti
 }
 
 // Parts of each of the `tail` tiles of a last, partly filled round behind `whole` tiles on `wgs` workgroups: as many as there are
-// places for, and behind whole rounds only if that makes four of each.  Places: the workgroups; behind whole rounds of 64 x 64
-// tiles, four of which share a CU's matrix cores, half of them (a tile that is alone on its CU already runs three times as fast as
-// in a full round).
+// places for, and behind whole rounds only if that makes four of each.  Places: the workgroups; behind whole rounds half of them
+// where that is enough for four parts of each (one to a compute unit with 128 x 128 tiles: 64 tiles of 2048 x 1667, 31 groups of 2247
+// columns 82.1 us uncut, 64.6 in 4 parts, 82.1 in 8; 48 of 2255 100 / 76 / 85), and for 64 x 64 tiles, four of which share a CU's matrix
+// cores, always (a tile that is alone on its CU already runs three times as fast as in a full round).
 __host__ __device__ inline int tail_parts(int tail, int whole, int wgs, int edge, const GmmParams& p) {
   if (tail == 0) return 1;
-  const int places = edge == 64 && whole ? wgs / 2 : wgs, room = places < p.k_parts ? places : p.k_parts;
+  const int places = whole && (edge == 64 || 8 * tail <= wgs) ? wgs / 2 : wgs, room = places < p.k_parts ? places : p.k_parts;
   const int parts = room / tail < p.k_split ? room / tail : p.k_split;
   return parts < (whole ? 4 : 2) ? 1 : parts;
 }
