@@ -634,11 +634,12 @@ bool may_be_cut(const GmmParams& p, int edge, int wgs) {
   if (p.jag != GMM_JAG_NONE) {
     const bool rows = p.jag == GMM_JAG_M;
     const int extent = rows ? p.M : p.N, groups = p.G < extent ? p.G : extent;
-    const float middle = float(extent) / edge + 0.5f * groups, away = 2.0f * sqrtf(groups / 12.0f);
+    const float full = float(extent) / edge, away = 2.0f * sqrtf(groups / 12.0f);
     step = rows ? tn : tm;
-    lo = int(ceilf(middle - away));
-    hi = int(floorf(middle + away));
+    lo = int(ceilf(full + groups / 3.0f - away));
+    hi = int(floorf(full + groups / 2.0f + away));
     if (lo < (rows ? tm : tn)) lo = rows ? tm : tn;
+    if (hi < groups) hi = groups;
   }
   for (int n = lo; n <= hi; ++n) {
     const int tiles = n * step, tail = tiles % wgs;
@@ -651,10 +652,12 @@ bool may_be_cut(const GmmParams& p, int edge, int wgs) {
 // that can cut them is 0.6 % slower where it does not (up to 4.5 %), a captured launch also clears a workspace for it (2 us).  So
 // launches of one to four rounds with at least 24 K tiles that may well be cut: equal products make a known number of tiles;
 // groups end anywhere in a tile, each makes half a tile more on average, all together with a deviation of the square root of
-// G / 12, and a number up to two deviations away has to be one that is cut.  us, whole / cut: fp32 1024 x 1024 x 8192 columns in 8
-// uneven groups (2.1 rounds) 166 / 159; bf16 8191 x 2047 x 2047 in 8 groups 142 / 135, 5 products of 7 x 13204 x 2148 (520 tiles,
-// 512 workgroups) 97 / 69.  544 random launches of such sizes: 56 are cut, 1.13
-// times as fast (1.0 to 1.41), the other 488 as fast as without a workspace (0.999; 0.994 when all of them ran the kernel that can cut).
+// G / 12, up to a third of the groups may be empty, and groups that are short make a tile each.  Any number in between, two
+// deviations added, has to be one that is cut.  us, whole / cut: fp32 1024 x 1024 x 8192 columns in 8 uneven groups (2.1 rounds) 166 /
+// 159; bf16 8191 x 2047 x 2047 in 8 groups 142 / 135, 5 products of 7 x 13204 x 2148 (520 tiles, 512 workgroups) 97 / 69; 3827 rows
+// in 31 groups, 6 of them empty, of 3189 x 1841 198 / 151.  170 random 16-bit launches whose last
+// round is cut 1.24 times as fast (0.99 to 1.6); with K below 2048 and most of the time spent on memory it can lose (28 products of
+// 2048 x 1835 to 7305 columns in all, 80 to 128 tiles in the last round 0.88 to 1.0).  fp32, 24 launches 1.06 (1.01 to 1.18).
 template <int EDGE>
 bool split_tail(GmmParams& p, int64_t most_wgs, int esz) {
   p.k_split = 0;

@@ -136,3 +136,17 @@ def test_last_round_behind_whole_ones(dtype, G, M, N, K, cut):
             check(out[g, :, -700:], a[g].cpu(), b[g, :, -700:].cpu())
     bound = (K + 1) * 2.0 ** -23 * (a.float().abs() @ b.float().abs()) + (0 if dtype == torch.float32 else 2.0 ** -7) * whole.float().abs()
     assert ((out.float() - whole.float()).abs() <= bound).all()       # both within half of that of the exact sum
+
+
+# 38 rows of 15 tiles, six groups empty; 33 rows of 48 tiles, every group shorter than one
+@pytest.mark.parametrize("dtype,sizes,N", [(torch.float16, [256, 0, 41] * 6 + [256] * 7 + [42] * 5 + [43], 1841), (torch.bfloat16, [2, 3] * 13 + [0] + [2] * 7, 6037)])
+def test_last_round_with_empty_and_with_short_groups(dtype, sizes, N):
+    K, gen = 1601, torch.Generator(device=DEV).manual_seed(N)
+    ends = torch.tensor(sizes).cumsum(0).tolist()
+    offs = torch.tensor(ends, dtype=torch.int32, device=DEV)
+    a, b = (torch.randn(*s, device=DEV, generator=gen).to(dtype) for s in ((ends[-1], K), (len(sizes), K, N)))
+    out, whole = launches(lambda o: K_.grouped_mm_2d3d(a, b, offs, o), (ends[-1], N), dtype)
+    assert out.isfinite().all() and not torch.equal(out.view(torch.int16), whole.view(torch.int16)), "nothing was cut"
+    for g, (s, e) in enumerate(zip(sizes, ends)):
+        if s:
+            check(out[e - s:e, -400:], a[e - s:e].cpu(), b[g, :, -400:].cpu())
