@@ -67,6 +67,8 @@ struct GmmParams {
   int32_t k_chunk, k_parts;
   // Register-staged kernel, any other product: the most parts that a tile is cut into along K.
   int32_t k_split;
+  // With that: the longest part of a launch of few tiles that gets a compute unit to itself.
+  int32_t k_alone;
 };
 
 constexpr int GMM_WS_HEADER = 4096;          // 1024 int32: arrival counters, one per tile of the split round, ...

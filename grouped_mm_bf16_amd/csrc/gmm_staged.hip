@@ -351,13 +351,17 @@ __device__ __forceinline__ bool join_parts(const GmmParams& p, const GmmTile& ti
 }
 
 // Parts of each of the `tail` tiles of a last, partly filled round behind `whole` tiles on `wgs` workgroups: as many as there are
-// places for, and behind whole rounds only if that makes four of each.  Places: the workgroups; behind whole rounds half of them
-// where that is enough for four parts of each (one to a compute unit with 128 x 128 tiles: 64 tiles of 2048 x 1667, 31 groups of 2247
-// columns 82.1 us uncut, 64.6 in 4 parts, 82.1 in 8; 48 of 2255 100 / 76 / 85), and for 64 x 64 tiles, four of which share a CU's matrix
-// cores, always (a tile that is alone on its CU already runs three times as fast as in a full round).
+// places for, and behind whole rounds only if that makes four of each.  Places: the workgroups.  Of 128 x 128 tiles half of them, one
+// to a compute unit, where that is enough for four parts of each: a second part on a unit slows the first, and each is stored and
+// read again.  us uncut / one part to a unit / two: a last round of 64 tiles of 2047 x 1667 (31 groups, 2247 columns) 82.1 / 64.6 /
+// 82.1, 48 of 2255 100 / 76 / 85; 1024 x 1024 x 2304 on 64 tiles 26.8 on the assembly tile / 25.7 / 38.2.  Where they alone make the
+// launch, parts past k_alone elements are better on two, full tiles later (1024 x 1024 x 5000, 64 tiles with A contiguous along M 34 /
+// 47) than those with few rows or columns (8 products of 64 x 1024 x 2560 22.0 / 24.1, x 4000 28.3 / 28.1, x 6144 35.6 / 32.7).  Behind whole rounds of 64 x 64 tiles, four of which share a CU's matrix cores, always half (a tile
+// that is alone on its CU already runs three times as fast as in a full round).
 __host__ __device__ inline int tail_parts(int tail, int whole, int wgs, int edge, const GmmParams& p) {
   if (tail == 0) return 1;
-  const int places = whole && (edge == 64 || 8 * tail <= wgs) ? wgs / 2 : wgs, room = places < p.k_parts ? places : p.k_parts;
+  const bool one_each = edge == 64 ? whole > 0 : 8 * tail <= wgs && (whole || int64_t(p.K) * tail <= int64_t(p.k_alone) * (wgs / 2));
+  const int places = one_each ? wgs / 2 : wgs, room = places < p.k_parts ? places : p.k_parts;
   const int parts = room / tail < p.k_split ? room / tail : p.k_split;
   return parts < (whole ? 4 : 2) ? 1 : parts;
 }
@@ -605,9 +609,9 @@ bool full_rows(const GmmParams& p) { return p.jag == GMM_JAG_M ? int64_t(p.M) >=
 // takes as long as one tile: each is cut into as many parts as there are workgroups for (the device knows the number of tiles),
 // of at least GMM_K_SPLIT_MIN elements, joined like those of a jagged contraction.  Joining costs 8 to 12 us.  us, whole / cut:
 // 16 rows, 8 groups of 4001 x 2047 112 / 47; 3 x 4 tiles of 331 x 517 x 4099, four products 86 / 40; fp32 500 x 500 x 8000, two
-// 173 / 92.  Over 350 random launches of up to half the workgroups 2.3 (16-bit) and 2.1 (fp32) times as fast; the line leaves
-// out what lost there or at sizes that fit the tiles exactly: K up to 1024 (two products of 512 x 1024 x 1024 17 / 22), more
-// than 64 full tiles with a first operand contiguous along M up to 2048 (0.97), more than 80 fp32 tiles up to 3072 (0.9 to 1.4).
+// 173 / 92.  Random launches of up to 256 tiles 2.7 (16-bit) and 2.8 (fp32) times as fast, 0.99 at worst.  The line leaves out what
+// lost: K up to 1024 (two products of 512 x 1024 x 1024 17 / 22), more than 64 full tiles up to 1536 (two of 1000 x 1001 x 1101 27 /
+// 33) or, with a first operand contiguous along M, up to 2048, more than 80 fp32 tiles up to 3072 (0.9 to 1.4).
 constexpr int GMM_K_SPLIT_MIN = 256;
 template <int EDGE>
 bool split_tiles(GmmParams& p, int64_t most_wgs) {
@@ -619,11 +623,12 @@ bool split_tiles(GmmParams& p, int64_t most_wgs) {
   if (tiles > 256 || 2 * tiles > most_wgs || 2 * tiles > room) return false;
   int least = 1024;
   if (EDGE == 64 && tiles > 80) least = 3072;
-  if (EDGE == 128 && tiles > 128) least = 1536;
+  if (EDGE == 128 && (tiles > 128 || (tiles > 64 && p.jag == GMM_JAG_NONE && full_rows(p)))) least = 1536;
   if (EDGE == 128 && tiles > 64 && p.a_sk != 1 && full_rows(p)) least = 2048;
   if (p.K <= least) return false;
   p.k_split = int32_t(p.K / GMM_K_SPLIT_MIN < GMM_K_PARTS_MAX ? p.K / GMM_K_SPLIT_MIN : GMM_K_PARTS_MAX);
   p.k_parts = int32_t(room);
+  p.k_alone = full_rows(p) && (p.jag == GMM_JAG_N ? int64_t(p.N) >= 96 * int64_t(p.G) : p.N >= 96) ? 1280 : 640;
   return true;
 }
 
@@ -714,10 +719,11 @@ bool small_tiles(const GmmParams& p, int in_dtype, int num_cus) {
 //   A contiguous along M: the assembly tile always has 256 rows.  1256 x 824 x 456 in 11 groups 32 / 21; 1392 x 1312 x
 //   352 in 40 groups 47 / 37; 2160 tiles of 1880 x 144 x 1120 35 / 37.  It wins once there are rounds to fill.
 //   Few tiles, K past 1024: cut along K (split_tiles).  The assembly tile cuts its own tiles from K = 4096 on, into longer
-//   parts.  us, assembly tile / here: one row each of 8 groups of 2048 x 1536 30 / 20; 8 products of 64 x 1024 x 4096 49 / 29;
-//   512 rows, 8 groups of 4096 x 1024 57 / 31; A contiguous along M, two products of 1024 x 1024 x 8192 89 / 58.  Full tiles want
-//   more K or fewer of them (two products of 1024 x 1024 x 2048 26 / 32).  Random launches, ragged sizes / sizes of whole tiles:
-//   few rows, five parts and more to a tile 1.6 / 1.6, full rows 1.5 / 1.4, A contiguous along M 2.2 / 1.7.
+//   parts.  us, assembly tile / here: one row each of 8 groups of 2048 x 1536 30 / 20; 8 products of 64 x 1024 x 4000 53 / 29;
+//   512 rows, 8 groups of 4000 x 1024 55 / 30; A contiguous along M, 1024 x 1024 x 8192 81 / 52.  Full tiles want more K or fewer of
+//   them: 1024 x 1024 x 2056 26 / 27, x 2816 31 / 27; 512 x 1024 x 1288 19 / 21, x 1800 23 / 22; 1472 x 1264 x 2304 29 / 33, x 3456 40 /
+//   38 (groups make fewer tiles than the most).  150 random launches of up to 256 tiles 1.55 times as fast (0.95 to 3.6, those that
+//   stay on the assembly tile among them).
 //   Jagged contraction: cut along K (above) it fills the chip whatever the groups' lengths.  A contiguous along M, up to 384
 //   tiles: 64 groups of 32 x 64 with 2048 elements each 46 / 13; 24 groups of 328 x 360, 95496 elements 201 / 98; two groups
 //   of 328 x 712, 40424 elements 652 / 62; past 384 the larger tile catches up (496 tiles of 184 x 464 in 62 even groups
@@ -744,8 +750,9 @@ bool gmm_staged_cut_preferred(const GmmParams& p, int num_cus) {
   if (!gmm_staged_eligible(p) || !split_tiles<128>(cut, tile_wgs(128) * int64_t(num_cus))) return false;
   const int64_t tiles = most_tiles(p, 128), parts = tile_wgs(128) * int64_t(num_cus) / tiles;
   if (p.a_sk != 1) return p.K >= 2560 && (parts >= 4 || p.K <= 6144);
-  if (parts >= 16) return true;
-  if (full_rows(p)) return p.K > 2048 && (parts >= 8 || (parts >= 4 && p.K <= 4096));
+  const bool equal = p.jag == GMM_JAG_NONE && p.N >= 96;    // full tiles; of groups most_tiles() is more than there are
+  if (parts >= 16) return !(equal && p.M > 128) || p.K >= (parts >= 20 ? 1280 : 1664);
+  if (full_rows(p)) return p.K > (equal && p.M > 192 && parts < 8 ? 3072 : 2048) && (parts >= 8 || (parts >= 4 && p.K <= 4096));
   return parts >= 5 && p.K <= 6144;
 }
 

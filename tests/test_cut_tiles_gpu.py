@@ -73,7 +73,9 @@ def test_unaligned_products(sizes, M, N, K, dtype, a_col, b_col):
     ("3d3d", 3, 104, 1408, 2048, False, False), ("3d3d", 8, 104, 1152, 4096, False, True), ("3d3d", 8, 104, 1152, 4104, False, False),
     ("2d3d", 10, 120, 1280, 1032, False, True), ("2d3d", 10, 120, 1408, 1032, False, False), ("2d3d", 10, 120, 1280, 6152, False, False),
     ("2d3d", 2, 32, 1024, 14336, False, True), ("3d2d", 4, 40, 1024, 2560, True, True), ("3d2d", 4, 40, 1024, 2552, True, False),
-    ("3d3d", 3, 520, 1664, 6144, True, True), ("3d3d", 3, 520, 1664, 6152, True, False)])
+    ("3d3d", 3, 520, 1664, 6144, True, True), ("3d3d", 3, 520, 1664, 6152, True, False), ("3d3d", 2, 136, 512, 1272, False, False),
+    ("3d3d", 2, 136, 512, 1280, False, True), ("3d3d", 1, 1032, 1024, 3072, False, False), ("3d3d", 1, 1032, 1024, 3080, False, True),
+    ("3d3d", 1, 1024, 1024, 2056, False, True), ("3d3d", 1, 1024, 1024, 5128, False, True)])
 def test_aligned_products_at_the_lines_of_the_rule(variant, G, M, N, K, a_col, cut):
     gen = torch.Generator().manual_seed(G + K)
     r = lambda *s: torch.randn(*s, generator=gen).bfloat16()
