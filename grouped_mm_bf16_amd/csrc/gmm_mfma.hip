@@ -663,16 +663,19 @@ int launch_asm(const GmmParams& p, GmmLayout lay, hipStream_t stream) {
 // Launches whose tiles are not renumbered for the XCDs.  Where every group is one row of tiles (decoding) there is nothing worth an
 // L2, the second operand is read once.  If such a row is more than an XCD's share of a round, the chip then reads 128 KB of a
 // row-major matrix that lie side by side in memory in launch order, and eight times 16 KB renumbered.  us, renumbered / in launch
-// order: 8 groups of 4096 x 28672, 64 rows in all 305 / 291 (6.5 TB/s; plain reads of such pieces 6.0 and 6.3), 16 of 2048 x 14336
-// 166 / 159.  A column-major matrix lies in memory tile by tile: 354 / 364 and 206 / 214.  Tiles of a group of several rows share it:
+// order: 8 groups of 4096 x 28672, 64 rows in all 304 / 291 (6.5 TB/s), 16 of 2048 x 14336 154 / 150, of 3072 x 14336 226 / 217, 8 of
+// 4096 x 20992 227 / 217.  Its rows have to lie whole KB apart, on cache lines: where the workgroups' pieces of 512 bytes share lines
+// or pages otherwise than in powers of two, they wait for each other.  8 groups of 4096 x 14592 143 / 146, x 14344 152 / 172, 16 of 2048
+// x 16256 168 / 204, x 20144 203 / 233.  Short columns gain nothing: 16 of 1160 x 16384 96 / 101, x 14336 94 / 96, of 1536 x 16384 125 /
+// 126.  A column-major matrix lies in memory tile by tile: 354 / 364 and 206 / 214.  Tiles of a group of several rows share it:
 // all 256 rows in one of those 8 groups 55 / 76, 249 of them (a fifth of the tiles) 297 / 312; 500 of 810 rows in one of 32 groups of
 // 2048 x 16384 (a ninth) 374 / 353.  So the kernel looks at the groups and renumbers if they hold more than an eighth.
-// Short reads pay for pages that eight XCDs share: 24 products of 8 x 8192 x 1024 69 / 72, 24 of 8 x 28672 x 256 83 / 85; narrow
-// groups: a decoding step with 128 groups of 2048 x 1536 200.4 / 201.8.
+// Narrow groups: a decoding step with 128 groups of 2048 x 1536 200.4 / 201.8.
 bool may_stay_in_order(const GmmParams& p, GmmLayout lay, int num_cus) {
   const bool few = p.jag == GMM_JAG_M ? int64_t(p.M) <= 32 * int64_t(p.G) : p.jag == GMM_JAG_NONE && p.M <= 64;
   const int64_t groups = p.jag == GMM_JAG_M ? gmm_min(p.G, p.M) : p.G;
-  return few && lay.a_kc && !lay.b_kc && p.N >= 48 * 256 && p.K >= 1024 && 4 * groups * gmm_cdiv(p.N, 256) >= 3 * int64_t(num_cus);
+  const bool lines = ((p.b_sk | p.b_sg) & 511) == 0 && (reinterpret_cast<uintptr_t>(p.b) & 127) == 0;
+  return few && lay.a_kc && !lay.b_kc && lines && p.N >= 48 * 256 && p.K >= 2048 && 4 * groups * gmm_cdiv(p.N, 256) >= 3 * int64_t(num_cus);
 }
 
 // Grid, tile heights and use of the workspace of a launch.

@@ -178,7 +178,9 @@ def test_small_groups_on_every_tile_height(K, N, b_col, tall, shrt):
 @pytest.mark.parametrize("b_col", [False, True])
 @pytest.mark.parametrize("sizes,N,K", [([8] * 8, 12288, 1024), ([30, 0, 1, 33, 64, 0, 3, 125], 12288, 1024), ([64] * 2, 28672, 1032),
                                        ([8] * 8, 12280, 1024), ([8] * 8, 12288, 1016), ([0, 249] + [1] * 6, 12288, 1024),
-                                       ([129] + [2] * 14, 12288, 1024), ([129] + [2] * 13, 12288, 1024)])
+                                       ([129] + [2] * 14, 12288, 1024), ([129] + [2] * 13, 12288, 1024), ([8] * 8, 12288, 2048),
+                                       ([8] * 8, 12288, 2040), ([8] * 8, 12544, 2048), ([30, 0, 1, 33, 64, 0, 3, 125], 12800, 2056),
+                                       ([0, 249] + [1] * 6, 12288, 2048), ([129] + [2] * 14, 12288, 2048), ([129] + [2] * 13, 12288, 2048)])
 def test_launch_order_of_wide_decoding_products(sizes, N, K, b_col):
     """Both sides of the lines between launches in order and renumbered ones (two of 16 and of 15 rows of tiles in one group
     among them): as asked for, and always in order.  Every element of both against fp32 products, and bit for bit."""
