@@ -374,16 +374,17 @@ __global__ void __launch_bounds__(kPlaceBlock) moe_place_kernel(const int32_t* _
 }
 
 // The whole routing of a decoding step, one launch: 16 tokens at a time, one to a wave, the next one's logits on their way while
-// one chooses.  It saves 1.1 us between two launches, but a compute unit's four SIMDs share the choices that otherwise spread over
-// the chip: a token takes one of them 0.03 us times (7 + choices * (keys of a lane + 1)), in rounds of 16 tokens.  Four tokens
-// have a SIMD each; more while a SIMD's share is up to 124 of those units.  us, one launch / two: 16 tokens, 8 of 128 experts 6.1 /
-// 6.9, 32 8.7 / 7.0; 48, 1 of 8 5.3 / 5.3, 144 9.7 / 5.5; 32, 2 of 8 5.0 / 5.4, 48 5.8 / 5.4; 32, 4 of 64 5.9 / 5.9, 48 7.0 / 5.9; 1, 8
-// of 512 8.8 / 9.8, 16 12.8 / 10.3.
+// one chooses.  It saves 1.1 us between two launches and 2 us of host time, but a compute unit's four SIMDs share the choices that
+// otherwise spread over the chip: a token takes one of them 0.02 to 0.03 us times (7 + choices * (keys of a lane + 1)), in rounds of
+// 16 tokens.  Four tokens have a SIMD each; more while a SIMD's share is up to 184 of those units, where the time lost on the GPU is
+// half of what the host saves.  us on the GPU, one launch / two: 16 tokens, 8 of 128 experts 6.1 / 6.9, 32 8.7 / 7.0; 48, 1 of 8 5.3 / 5.3,
+// 144 9.7 / 5.5; 32, 2 of 8 5.0 / 5.4, 48 5.8 / 5.4; 32, 4 of 64 5.9 / 5.9, 48 7.0 / 5.9; 1, 8 of 512 8.8 / 9.8, 16 12.8 / 10.3.  Launched
+// one after the other: 41, 2 of 6 5.3 / 7.2, 18, 8 of 13 5.8 / 7.4.
 int lane_keys(int64_t E) { return E <= 64 ? 1 : E <= 128 ? 2 : E <= 256 ? 4 : E <= 512 ? 8 : E <= 768 ? 12 : 16; }
 bool route_in_one(int64_t tokens, int64_t E, int64_t top_k) {
   if (tokens <= 4) return true;
   const int64_t per_simd = tokens <= kPlaceWaves ? (tokens + 3) / 4 : (tokens + kPlaceWaves - 1) / kPlaceWaves * 4;
-  return tokens * top_k <= kPlaceBlock && per_simd * (7 + top_k * (lane_keys(E) + 1)) <= 124;
+  return tokens * top_k <= kPlaceBlock && per_simd * (7 + top_k * (lane_keys(E) + 1)) <= 184;
 }
 
 template <typename T, int kPer>

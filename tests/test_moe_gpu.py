@@ -58,7 +58,8 @@ def test_slots_at_the_edges_of_a_workgroup(T, E, k):
 @pytest.mark.parametrize("T,E,k", [(16, 64, 8), (17, 65, 8), (32, 128, 8), (33, 129, 8), (144, 5, 1), (145, 5, 1), (32, 1023, 32), (16, 256, 32),
                                    (80, 257, 2), (81, 1023, 2), (1023, 9, 1), (341, 9, 3), (1024, 7, 1), (1025, 7, 1), (131072, 5, 1),
                                    (131073, 5, 1), (4, 512, 8), (4, 513, 8), (700, 512, 4), (700, 513, 32), (90, 768, 32), (91, 769, 3), (48, 8, 1), (49, 8, 1),
-                                   (32, 8, 2), (33, 8, 2), (17, 128, 8), (8, 256, 8), (9, 256, 8), (5, 512, 8), (4, 1023, 32), (5, 1023, 32)])
+                                   (32, 8, 2), (33, 8, 2), (17, 128, 8), (8, 256, 8), (9, 256, 8), (5, 512, 8), (4, 1023, 32), (5, 1023, 32), (80, 8, 1),
+                                   (81, 8, 1), (64, 8, 2), (65, 8, 2), (32, 64, 8), (33, 64, 8), (12, 256, 8), (13, 256, 8), (8, 512, 8)])
 def test_routing_at_the_edges_of_its_kernels(T, E, k):
     """One launch for a few tokens, the more the fewer experts and choices, then 1024 slots to a workgroup, from
     131073 slots on a table of counts; 64, 128, 256, 512 and 768 experts to a lane's registers.  Ties and masked experts among them."""
