@@ -712,7 +712,7 @@ bool gmm_mfma_uses_workspace(GmmParams p, GmmLayout lay, int config, int num_cus
 int gmm_launch_mfma(GmmParams p, GmmLayout lay, int in_dtype, int out_dtype, int config, int num_cus, hipStream_t stream) {
   plan(p, lay, config, num_cus);
   if (config == GMM_CFG_ASM_256x256 && p.xcd_remap && may_stay_in_order(p, lay, num_cus))
-    p.xcd_remap = p.jag == GMM_JAG_M ? GMM_REMAP_SHARED : 0;
+    p.xcd_remap = p.jag == GMM_JAG_M && p.M > 128 ? GMM_REMAP_SHARED : 0;   // up to 128 rows make one row of tiles, whoever has them
   const bool out16 = out_dtype == in_dtype;   // else fp32
   if (!out16 && out_dtype != GMM_DT_F32) return -1;
   if (config == GMM_CFG_ASM_256x256) {
