@@ -662,7 +662,7 @@ bool may_be_cut(const GmmParams& p, int edge, int wgs) {
 // 159; bf16 8191 x 2047 x 2047 in 8 groups 142 / 135, 5 products of 7 x 13204 x 2148 (520 tiles, 512 workgroups) 97 / 69; 3827 rows
 // in 31 groups, 6 of them empty, of 3189 x 1841 198 / 151.  170 random 16-bit launches whose last
 // round is cut 1.24 times as fast (0.99 to 1.6); with K below 2048 and most of the time spent on memory it can lose (28 products of
-// 2048 x 1835 to 7305 columns in all, 80 to 128 tiles in the last round 0.88 to 1.0).  fp32, 24 launches 1.06 (1.01 to 1.18).
+// 2048 x 1835 to 7305 columns in all, 80 to 128 tiles in the last round 0.79 to 1.0).  fp32, 24 launches 1.06 (1.01 to 1.18).
 template <int EDGE>
 bool split_tail(GmmParams& p, int64_t most_wgs, int esz) {
   p.k_split = 0;

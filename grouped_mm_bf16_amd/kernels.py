@@ -176,7 +176,7 @@ def _launch(variant: int, a: torch.Tensor, b: torch.Tensor, offs: Optional[torch
 
 
 # Bytes from which a gradient is not cleared first: torch's fill of 32 MiB takes as long as the kernel that looks at the offsets
-# (6 us; 134 MB 18.5), and a smaller one costs less host time than that launch.
+# (5 us; 134 MB 18.5), and a smaller one costs less host time than that launch.
 _CLEAR_FIRST_BELOW = 32 << 20
 
 

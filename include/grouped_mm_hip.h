@@ -131,7 +131,9 @@ int gmm_2d3d_swiglu(const void* a, const int32_t* row_index, const void* b, void
  * product rounded to the output's type before the activation, as gmm_2d3d_gather and gmm_moe_activation leave it:
  *   out[r, c] = silu(h[r, c]) * h[r, N / 2 + c].
  * With b contiguous along K also (N / 2 + 256) * b_stride_n * 2 < 2^31.  GMM_ERR_UNSUPPORTED as well where the two calls are
- * faster: up to 64 rows a group on average with K >= 2048 and K * N >= 2^23. */
+ * faster: up to 64 rows a group on average with K >= 2048 and K * N >= 2^23, and products of few tiles with K > 1024 that
+ * gmm_2d3d_gather cuts along K.  The latter assumes that gmm_2d3d_gather is then given a workspace of gmm_workspace_bytes();
+ * without one it does not cut them. */
 int gmm_2d3d_swiglu_apart(const void* a, const int32_t* row_index, const void* b, void* out,
                           const int32_t* offs, int32_t G, int64_t a_rows,
                           int64_t M_total, int64_t N, int64_t K,
@@ -196,8 +198,8 @@ int gmm_zero_unowned(void* out, const int32_t* offs, int32_t G, int32_t by_colum
  *   token_rows  int32[tokens * top_k]   the row of each slot (inverse of the sort)
  * experts <= 1023, top_k <= min(experts, 32), tokens * top_k < 2^31.  `workspace` is device memory of at
  * least gmm_moe_route_workspace_bytes(...) bytes (per-workgroup expert histograms; contents need not be
- * initialised); too small a workspace returns GMM_ERR_WORKSPACE.  One launch on `stream` for a few
- * tokens, two for up to 131072 slots, four for more (the workspace is theirs); no host sync. */
+ * initialised); too small a workspace returns GMM_ERR_WORKSPACE, whatever the number of slots.  One launch on `stream` for a
+ * few tokens, two for up to 131072 slots, four for more (only these four use the workspace); no host sync. */
 int64_t gmm_moe_route_workspace_bytes(int64_t tokens, int64_t experts, int64_t top_k);
 int gmm_moe_route(const void* logits, int64_t logits_stride, int32_t logits_dtype,
                   int64_t tokens, int64_t experts, int64_t top_k, int32_t renormalize,
@@ -211,8 +213,8 @@ int gmm_moe_route(const void* logits, int64_t logits_stride, int32_t logits_dtyp
  * holds on every GPU it runs on until the process ends; the call allocates nothing.  Problems whose
  * gmm_moe_route_workspace_bytes(...) exceeds 262144 bytes are refused with GMM_ERR_WORKSPACE (any problem
  * with experts <= 256 fits; with 1023 experts up to 65536 slots).  All calls on one GPU with more than 131072
- * slots share that array: such calls that may overlap on one GPU (different streams, different threads) race and must be serialised by
- * the caller.  The first call on a device looks the array's device address up (hipGetSymbolAddress, no
+ * slots share that array: such calls that may overlap on one GPU (different streams, different threads) race and must
+ * be serialised by the caller.  The first call on a device looks the array's device address up (hipGetSymbolAddress, no
  * allocation): make that first call outside a stream capture -- one eager call per device at start-up is
  * enough -- and every later call, captured or not, only launches.  Outputs and everything else as
  * gmm_moe_route. */
